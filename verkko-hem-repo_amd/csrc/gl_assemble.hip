@@ -102,136 +102,6 @@ __device__ inline double hess_entry(const double *__restrict__ G, const double *
          2.0 * M.b5 * (dmn * Avu_lk + vml * unk + dmn * Auv_lk - uml * vnk + W * dkl);
 }
 
-// rho_c = alpha x_c + 2 sum_n beta_n r_n(E_c), the bulk residual density, for
-// the components (mu, k) of u (ru) and of v (rv) at once, from the 18 values
-// x of one point.  The Gram entries it needs (|u|^2, |v|^2, u:v and row mu of
-// u u^T, v v^T, u v^T, v u^T) are summed in the order of gram_entry; x sits in
-// registers, and its entries at run-time indices are read again from memory
-// (LDS) so that no register array is indexed at run time.
-template <typename TA>
-__device__ inline void rho_pair(const TA *x, int mu, int k, const Material &M, double &ru, double &rv)
-{
-  double u[9], v[9];
-#pragma unroll
-  for (int a = 0; a < 9; ++a) { u[a] = (double)x[a]; v[a] = (double)x[9 + a]; }
-  double U2 = 0.0, V2 = 0.0, UV = 0.0;
-#pragma unroll
-  for (int a = 0; a < 9; ++a) U2 += u[a] * u[a];
-#pragma unroll
-  for (int a = 0; a < 9; ++a) V2 += v[a] * v[a];
-#pragma unroll
-  for (int a = 0; a < 9; ++a) UV += u[a] * v[a];
-  const double D = U2 - V2, N = U2 + V2;
-  double um[3], vm[3];  // row mu of u and of v
-#pragma unroll
-  for (int j = 0; j < 3; ++j) { um[j] = (double)x[3 * mu + j]; vm[j] = (double)x[9 + 3 * mu + j]; }
-  double Pu = 0, Pv = 0, Qu = 0, Qv = 0, Su = 0, Sv = 0, Wu = 0, Wv = 0;
-#pragma unroll
-  for (int nu = 0; nu < 3; ++nu) {
-    double uu = 0.0, vv = 0.0, uvmn = 0.0, uvnm = 0.0;  // uut, vvt, uvt at (mu, nu); uvt at (nu, mu)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      uu += um[j] * u[3 * nu + j];
-      vv += vm[j] * v[3 * nu + j];
-      uvmn += um[j] * v[3 * nu + j];
-      uvnm += u[3 * nu + j] * vm[j];
-    }
-    const double P = uu - vv, S = uu + vv, Q = uvmn + uvnm, W = uvnm - uvmn;
-    const double un = (double)x[3 * nu + k], vn = (double)x[9 + 3 * nu + k];
-    Pu += P * un; Pv += P * vn; Qu += Q * un; Qv += Q * vn;
-    Su += S * un; Sv += S * vn; Wu += W * un; Wv += W * vn;
-  }
-  const double ua = (double)x[3 * mu + k], va = (double)x[9 + 3 * mu + k];
-  ru = M.al * ua + 2.0 * (M.b1 * (D * ua + 2.0 * UV * va) + M.b2 * (N * ua) + M.b3 * (Pu + Qv) + M.b4 * (Su - Wv) +
-                          M.b5 * (Su + Wv));
-  rv = M.al * va + 2.0 * (M.b1 * (-D * va + 2.0 * UV * ua) + M.b2 * (N * va) + M.b3 * (Qu - Pv) + M.b4 * (Sv + Wu) +
-                          M.b5 * (Sv - Wu));
-}
-
-// H(s) x for the components (mu, k) of u (zu) and of v (zv) without forming
-// H: the derivative of rho at the state s in the direction x (18 values
-// each, in LDS), term by term the linearisation of rho_pair:
-//   d|u|^2 = 2 u:a, d|v|^2 = 2 v:b, d(u:v) = u:b + a:v,
-//   d(u u^T) = a u^T + u a^T, d(v v^T) = b v^T + v b^T, d(u v^T) = a v^T + u b^T,
-//   d(P u) = dP u + P a, ...  with (a, b) the u and v parts of x.
-// In two stages, so that a point's 9 items share the sums through LDS
-// instead of each forming all of them.  The row-pair sums are symmetric in
-// (mu, nu) but for W and dW, which change sign:
-//   uu, vv symmetric; uvmn(nu, mu) = uvnm(mu, nu), so Q is symmetric and W
-//   antisymmetric; likewise duu, dvv, dQ and dW.
-// The six pairs mu <= nu, numbered (0,0) (0,1) (0,2) (1,1) (1,2) (2,2), hold
-// 8 values each, P S Q W dP dS dQ dW; the pairs (mu, mu) also give the 9-term
-// sums: D = sum_mu P, N = sum_mu S, u:v = sum_mu Q / 2, dD = sum_mu dP,
-// dN = sum_mu dS, d(u:v) = sum_mu dQ / 2.
-// Stage 1: the 8 sums of pair p at the state s in the direction x, to r.
-template <typename TA>
-__device__ inline void hx_row_sums(const TA *s, const TA *x, int p, TA *r)
-{
-  const int mu = p < 3 ? 0 : (p < 5 ? 1 : 2), nu = p < 3 ? p : (p < 5 ? p - 2 : 2);
-  TA uu = 0, vv = 0, uvmn = 0, uvnm = 0, duu = 0, dvv = 0, duvmn = 0, duvnm = 0;
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const TA um = s[3 * mu + j], vm = s[9 + 3 * mu + j], am = x[3 * mu + j], bm = x[9 + 3 * mu + j];
-    const TA un = s[3 * nu + j], vn = s[9 + 3 * nu + j], an = x[3 * nu + j], bn = x[9 + 3 * nu + j];
-    uu += um * un;
-    vv += vm * vn;
-    uvmn += um * vn;
-    uvnm += un * vm;
-    duu += am * un + um * an;
-    dvv += bm * vn + vm * bn;
-    duvmn += am * vn + um * bn;
-    duvnm += an * vm + un * bm;
-  }
-  r[0] = uu - vv;
-  r[1] = uu + vv;
-  r[2] = uvmn + uvnm;
-  r[3] = uvnm - uvmn;
-  r[4] = duu - dvv;
-  r[5] = duu + dvv;
-  r[6] = duvmn + duvnm;
-  r[7] = duvnm - duvmn;
-}
-
-// Stage 2: H(s) x for the components (mu, k) of u (zu) and of v (zv) from the
-// point's 48 pair sums R (stage 1) and its s and x.
-template <typename TA>
-__device__ inline void hx_from_sums(const TA *R, const TA *s, const TA *x, int mu, int k, const Material &M, TA &zu,
-                                    TA &zv)
-{
-  // the 9-term sums from the pairs (0,0), (1,1), (2,2)
-  TA D = 0, N = 0, Q2 = 0, dD = 0, dN = 0, dQ2 = 0;
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    const TA *r = R + 8 * (m == 0 ? 0 : (m == 1 ? 3 : 5));
-    D += r[0];
-    N += r[1];
-    Q2 += r[2];
-    dD += r[4];
-    dN += r[5];
-    dQ2 += r[6];
-  }
-  const TA UV = (TA)0.5 * Q2, dUV = (TA)0.5 * dQ2;
-  TA dPu = 0, dPv = 0, dQu = 0, dQv = 0, dSu = 0, dSv = 0, dWu = 0, dWv = 0;
-#pragma unroll
-  for (int nu = 0; nu < 3; ++nu) {
-    const int lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
-    const TA *r = R + 8 * (lo == 0 ? hi : (lo == 1 ? hi + 2 : 5));
-    const TA sg = mu > nu ? (TA)-1 : (TA)1;  // W and dW of the pair (mu, nu)
-    const TA P = r[0], S = r[1], Q = r[2], W = sg * r[3], dP = r[4], dS = r[5], dQ = r[6], dW = sg * r[7];
-    const TA un = s[3 * nu + k], vn = s[9 + 3 * nu + k], an = x[3 * nu + k], bn = x[9 + 3 * nu + k];
-    dPu += dP * un + P * an; dPv += dP * vn + P * bn;
-    dQu += dQ * un + Q * an; dQv += dQ * vn + Q * bn;
-    dSu += dS * un + S * an; dSv += dS * vn + S * bn;
-    dWu += dW * un + W * an; dWv += dW * vn + W * bn;
-  }
-  const TA u0 = s[3 * mu + k], v0 = s[9 + 3 * mu + k], a0 = x[3 * mu + k], b0 = x[9 + 3 * mu + k];
-  const TA al = (TA)M.al, b1 = (TA)M.b1, b2 = (TA)M.b2, b3 = (TA)M.b3, b4 = (TA)M.b4, b5 = (TA)M.b5;
-  zu = al * a0 + (TA)2 * (b1 * (dD * u0 + D * a0 + (TA)2 * (dUV * v0 + UV * b0)) + b2 * (dN * u0 + N * a0) +
-                          b3 * (dPu + dQv) + b4 * (dSu - dWv) + b5 * (dSu + dWv));
-  zv = al * b0 + (TA)2 * (b1 * ((TA)2 * (dUV * u0 + UV * a0) - (dD * v0 + D * b0)) + b2 * (dN * v0 + N * b0) +
-                          b3 * (dQu - dPv) + b4 * (dSv + dWu) + b5 * (dSv - dWu));
-}
-
 __device__ inline bool face_zeroed(int bid, int c) { return (c % 9) % 3 == bid - 2; }
 
 __device__ inline double face_area(int lf, const double *h)
@@ -491,7 +361,7 @@ __global__ __launch_bounds__(NT) void k_mf_setup(RefTables T, MeshDev Mh, Materi
     double xv = 0;
     for (int a = 0; a < NS; ++a) xv += T.N[q * NS + a] * sU[a * 18 + c];
     sX[i] = xv;
-    Uq[(size_t)e * NQ * 18 + i] = (TH)xv;  // the iterate at the points, the product's state
+    Uq[(size_t)e * NQ * 18 + c * NQ + q] = (TH)xv;  // the iterate at the points, the product's state
   }
   __syncthreads();
   for (int i = tid; i < NQ * GRAM; i += NT) {
@@ -586,335 +456,680 @@ __global__ __launch_bounds__(NT) void k_mf_setup(RefTables T, MeshDev Mh, Materi
 }
 
 // The product in sum-factorised form: N_b(q) = L_bx(x_qx) L_by(x_qy) L_bz(x_qz),
-// so x and its gradients at the quadrature points take three 1D passes (x, y,
-// z) and the test against N_a and its gradients three more (z, y, x),
-// 2 x 18 x 27 x 27 multiply-adds per Q2 cell instead of 8 x 18 x 27 x 27.
-// One thread per 1D line of points and component (a pencil) in each pass: it
-// reads its N1 inputs once and applies the 1D bases from registers, so the
-// passes move about 2.5x fewer LDS words than one thread per (point,
-// component) with the bases in LDS.  At the points, H(q) X(q) is not read
-// from a stored Hessian (171 values per point) but formed as the derivative
-// of rho at the stored iterate U(q) (18 values per point) in the direction
-// X(q) (hx_row_sums, hx_from_sums): the operator's state shrinks from
-// 1.21 GB to 0.13 GB on the 32^3 Q2 cube, and the kernel is bound by its
-// arithmetic and LDS passes instead of the Hessian stream.  At the points a
-// thread owns the components c and c + 9 of one point (the same orbital
-// entry in u and in v), after six threads per point have formed the point's
-// row-pair sums.
+// so x and its gradients at the quadrature points take 1D passes in the three
+// directions, and the test against N_a and its gradients three more.  At the
+// points, H(q) X(q) is formed as the derivative of rho at the stored iterate
+// U(q) (18 values per point) in the direction X(q).
 // TH: the stored iterate (FP64, or FP32 for the FP32 inner solve); TX: x.
 // TA, the arithmetic, LDS and cell-slot type, is FP32 when both are FP32 (the
-// FP32 inner solve, with FP32 accumulation) and FP64 otherwise.  cells[]
-// lists the cells in the launch order, -1 for padding (the XCD-aware order of
-// mf_cell_order).
+// FP32 inner solve, with FP32 accumulation) and FP64 otherwise.
 // RES: the residual R(x) of the cell loop (residual.cc:164-232, the Robin
 // faces :235-278) through the same passes: x is the iterate (no column
 // masking), and rho(X(q)), the bulk residual density, takes the place of
 // H(q) X(q); Uq is not read, and flag is the batch's instance_active.
-template <int DEG, typename TH>
-constexpr int mf_threads() { return DEG == 1 ? 128 : 256; }
+
+// One 1D line of the tensor-product element FE_Q(DEG) x Gauss(DEG + 1), in
+// Q2 in local polynomial coefficients: with tau = xi - 1/2 a quadratic is
+// m + tau d + 2 tau^2 w (m = v1, d = v2 - v0, w = v0 - 2 v1 + v2).  The Gauss
+// points are symmetric about the middle, so values and derivatives of a line
+// at its points take 8 operations instead of 18 multiply-adds with the
+// tables, and their transposes (the test passes) 12; the middle point's value
+// is m and its derivative d.  (Q1 keeps the two node weights: the shorter
+// v0 + xi d rounds worse in FP32.)  The
+// transposes carry the 1D weights relative to the middle point's; the factor
+// that is left per cell is W0 (the middle weight) cubed.
+template <int DEG, typename T>
+struct Line;
+
+template <typename T>
+struct Line<2, T> {
+  static constexpr int N = 3;
+  static constexpr double W0 = 8.0 / 18.0;
+  static constexpr double h = 0.38729833462074168852;  // sqrt(3/5) / 2, the outer points' tau
+  static constexpr double r = 0.625;                    // the outer points' weight over the middle one's
+  // coefficients of the line (in place of its values)
+  static __device__ inline void coef(T &a, T &b, T &c)
+  {
+    const T m = b, d = c - a, w = (a + c) - (T)2 * b;
+    a = m;
+    b = d;
+    c = w;
+  }
+  static __device__ inline void uncoef(T &a, T &b, T &c)  // transpose of coef
+  {
+    const T m = a, d = b, w = c;
+    a = w - d;
+    b = m - (T)2 * w;
+    c = w + d;
+  }
+  // point q (uniform) of the z lines: value and derivative from coefficients
+  T v1, v2, d2, wq, wv1, wv2, wd2;
+  __device__ inline void point(int q)
+  {
+    v1 = (T)(q == 0 ? -h : q == 1 ? 0.0 : h);
+    v2 = (T)(q == 1 ? 0.0 : 2 * h * h);
+    d2 = (T)(q == 0 ? -4 * h : q == 1 ? 0.0 : 4 * h);
+    wq = (T)(q == 1 ? 1.0 : r);
+    wv1 = (T)(q == 0 ? -r * h : q == 1 ? 0.0 : r * h);
+    wv2 = (T)(q == 1 ? 0.0 : r * 2 * h * h);
+    wd2 = (T)(q == 0 ? -r * 4 * h : q == 1 ? 0.0 : r * 4 * h);
+  }
+  __device__ inline T val(const T *k) const { return k[0] + v1 * k[1] + v2 * k[2]; }
+  __device__ inline T der(const T *k) const { return k[1] + d2 * k[2]; }
+  // transpose of both: k += val^T p + der^T g, with the weight of the point
+  __device__ inline void back(T p, T g, T *k) const
+  {
+    k[0] += wq * p;
+    k[1] += wv1 * p;
+    k[1] += wq * g;
+    k[2] += wv2 * p;
+    k[2] += wd2 * g;
+  }
+  __device__ inline void back(T p, T *k) const
+  {
+    k[0] += wq * p;
+    k[1] += wv1 * p;
+    k[2] += wv2 * p;
+  }
+  // values (and derivatives) of a line at its points
+  static __device__ inline void values(const T *v, T *p)
+  {
+    const T d = v[2] - v[0], w = (v[0] + v[2]) - (T)2 * v[1], e = v[1] + (T)(2 * h * h) * w;
+    p[0] = e - (T)h * d;
+    p[1] = v[1];
+    p[2] = e + (T)h * d;
+  }
+  static __device__ inline void both(const T *v, T *p, T *g)
+  {
+    const T d = v[2] - v[0], w = (v[0] + v[2]) - (T)2 * v[1], e = v[1] + (T)(2 * h * h) * w;
+    p[0] = e - (T)h * d;
+    p[1] = v[1];
+    p[2] = e + (T)h * d;
+    g[0] = d - (T)(4 * h) * w;
+    g[1] = d;
+    g[2] = d + (T)(4 * h) * w;
+  }
+  // their transposes, with the points' weights
+  static __device__ inline void test_v(const T *p, T *v)
+  {
+    const T a = p[0] + p[2], b = (T)(r * h) * (p[2] - p[0]), w = (T)(r * 2 * h * h) * a, m = p[1] + (T)r * a;
+    v[0] = w - b;
+    v[1] = m - (T)2 * w;
+    v[2] = w + b;
+  }
+  static __device__ inline void test_d(const T *g, T *v)
+  {
+    const T d = g[1] + (T)r * (g[0] + g[2]), w = (T)(r * 4 * h) * (g[2] - g[0]);
+    v[0] = w - d;
+    v[1] = (T)-2 * w;
+    v[2] = w + d;
+  }
+  static __device__ inline void test_vd(const T *p, const T *g, T *v)
+  {
+    const T a = p[0] + p[2], m = p[1] + (T)r * a;
+    const T d = (T)(r * h) * (p[2] - p[0]) + (g[1] + (T)r * (g[0] + g[2]));
+    const T w = (T)(r * 2 * h * h) * a + (T)(r * 4 * h) * (g[2] - g[0]);
+    v[0] = w - d;
+    v[1] = m - (T)2 * w;
+    v[2] = w + d;
+  }
+  // 1D mass matrix of a unit edge times 30 (the Robin faces)
+  static constexpr double M0 = 1.0 / 30.0;
+  static __device__ inline void mass(const T *v, T *y)
+  {
+    y[0] = (T)4 * v[0] + (T)2 * v[1] - v[2];
+    y[1] = (T)2 * v[0] + (T)16 * v[1] + (T)2 * v[2];
+    y[2] = (T)-1 * v[0] + (T)2 * v[1] + (T)4 * v[2];
+  }
+};
+
+template <typename T>
+struct Line<1, T> {
+  static constexpr int N = 2;
+  static constexpr double W0 = 0.5;
+  static constexpr double t0 = 0.21132486540518711775, t1 = 0.78867513459481288225;  // (1 -+ 1/sqrt(3)) / 2
+  T a, b;  // of the z lines' point q: the weights of the two nodes
+  __device__ inline void point(int q)
+  {
+    a = (T)(q == 0 ? t1 : t0);
+    b = (T)(q == 0 ? t0 : t1);
+  }
+  __device__ inline T val(const T *k) const { return a * k[0] + b * k[1]; }
+  __device__ inline T der(const T *k) const { return k[1] - k[0]; }
+  __device__ inline void back(T p, T g, T *k) const
+  {
+    k[0] += a * p - g;
+    k[1] += b * p + g;
+  }
+  __device__ inline void back(T p, T *k) const
+  {
+    k[0] += a * p;
+    k[1] += b * p;
+  }
+  static __device__ inline void values(const T *v, T *p)
+  {
+    p[0] = (T)t1 * v[0] + (T)t0 * v[1];
+    p[1] = (T)t0 * v[0] + (T)t1 * v[1];
+  }
+  static __device__ inline void both(const T *v, T *p, T *g)
+  {
+    values(v, p);
+    g[0] = g[1] = v[1] - v[0];
+  }
+  static __device__ inline void test_v(const T *p, T *v)
+  {
+    v[0] = (T)t1 * p[0] + (T)t0 * p[1];
+    v[1] = (T)t0 * p[0] + (T)t1 * p[1];
+  }
+  static __device__ inline void test_d(const T *g, T *v)
+  {
+    v[1] = g[0] + g[1];
+    v[0] = -v[1];
+  }
+  static __device__ inline void test_vd(const T *p, const T *g, T *v)
+  {
+    const T d = g[0] + g[1];
+    v[0] = ((T)t1 * p[0] + (T)t0 * p[1]) - d;
+    v[1] = ((T)t0 * p[0] + (T)t1 * p[1]) + d;
+  }
+  static constexpr double M0 = 1.0 / 6.0;
+  static __device__ inline void mass(const T *v, T *y)
+  {
+    y[0] = (T)2 * v[0] + v[1];
+    y[1] = v[0] + (T)2 * v[1];
+  }
+};
+
+// The bulk term at one point.  rho and its derivative are a symmetric 6 x 6
+// matrix on the spin index of (u, v), rows mu, times the 6 x 3 matrix (u; v):
+//   rho(A) = N(A) (u; v),   H(A) X = N(A) (a; b) + dN(A; X) (u; v),
+//   N = [[E, C], [C^T, F]],
+//   E = 2 (b3+b4+b5) u u^T + 2 (b4+b5-b3) v v^T + (al + 2 b1 p + 2 b2 s) 1,
+//   F = 2 (b4+b5-b3) u u^T + 2 (b3+b4+b5) v v^T + (al - 2 b1 p + 2 b2 s) 1,
+//   C = 2 (b3+b4-b5) u v^T + 2 (b3-b4+b5) v u^T + 4 b1 (u:v) 1,
+// p = |u|^2 - |v|^2, s = |u|^2 + |v|^2: the terms of the reference's density
+// collected by the Gram matrices u u^T, v v^T, u v^T, in which N is linear
+// (dN is N of their derivatives, without al).  One thread forms the 18
+// entries of a point from registers in about 500 operations (rho: 230),
+// against 936 term by term.
+template <typename T>
+struct BulkMat {
+  T E[6], F[6], C[9];  // symmetric entries 00 01 02 11 12 22
+  __device__ inline void set(const T *uu, const T *vv, const T *uv, T al, T tb1, T tb2, T c1, T c2, T d1, T d2)
+  {
+    const T tu = uu[0] + uu[3] + uu[5], tv = vv[0] + vv[3] + vv[5], q = (T)2 * (uv[0] + uv[4] + uv[8]);
+    const T p = tu - tv, s = tu + tv, i2 = al + tb2 * s;
+    const T ei = i2 + tb1 * p, fi = i2 - tb1 * p, ci = tb1 * q;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const bool dg = i == 0 || i == 3 || i == 5;
+      E[i] = c1 * uu[i] + c2 * vv[i];
+      F[i] = c2 * uu[i] + c1 * vv[i];
+      if (dg) {
+        E[i] += ei;
+        F[i] += fi;
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int n = 0; n < 3; ++n) {
+        C[3 * m + n] = d1 * uv[3 * m + n] + d2 * uv[3 * n + m];
+        if (m == n) C[3 * m + n] += ci;
+      }
+  }
+  // (zu, zv) += N (a; b) for the orbital column k
+  __device__ inline void add(const T *a, const T *b, int k, T *zu, T *zv) const
+  {
+    constexpr int id[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int n = 0; n < 3; ++n) {
+        zu[m] += E[id[3 * m + n]] * a[3 * n + k];
+        zu[m] += C[3 * m + n] * b[3 * n + k];
+        zv[m] += C[3 * n + m] * a[3 * n + k];
+        zv[m] += F[id[3 * m + n]] * b[3 * n + k];
+      }
+  }
+};
+
+// u u^T, v v^T (symmetric entries) and u v^T of the 18 values s
+template <typename T>
+__device__ inline void gram(const T *s, T *uu, T *vv, T *uv)
+{
+  int i = 0;
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      T a = s[3 * m] * s[9 + 3 * n];
+      a += s[3 * m + 1] * s[9 + 3 * n + 1];
+      a += s[3 * m + 2] * s[9 + 3 * n + 2];
+      uv[3 * m + n] = a;
+      if (n < m) continue;
+      T b = s[3 * m] * s[3 * n], c = s[9 + 3 * m] * s[9 + 3 * n];
+#pragma unroll
+      for (int k = 1; k < 3; ++k) {
+        b += s[3 * m + k] * s[3 * n + k];
+        c += s[9 + 3 * m + k] * s[9 + 3 * n + k];
+      }
+      uu[i] = b;
+      vv[i] = c;
+      ++i;
+    }
+}
+
+// their derivatives at s in the direction x
+template <typename T>
+__device__ inline void dgram(const T *s, const T *x, T *uu, T *vv, T *uv)
+{
+  int i = 0;
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      T a = 0, b = 0, c = 0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        a += x[3 * m + k] * s[9 + 3 * n + k];
+        a += s[3 * m + k] * x[9 + 3 * n + k];
+        if (n < m) continue;
+        b += x[3 * m + k] * s[3 * n + k];
+        c += x[9 + 3 * m + k] * s[9 + 3 * n + k];
+        if (n == m) continue;
+        b += s[3 * m + k] * x[3 * n + k];
+        c += s[9 + 3 * m + k] * x[9 + 3 * n + k];
+      }
+      uv[3 * m + n] = a;
+      if (n < m) continue;
+      uu[i] = n == m ? (T)2 * b : b;
+      vv[i] = n == m ? (T)2 * c : c;
+      ++i;
+    }
+}
+
 template <typename TH, typename TX>
 using mf_arith = typename std::conditional<std::is_same<TH, float>::value && std::is_same<TX, float>::value, float,
                                            double>::type;
+// Cells per workgroup: 7 on two waves (126 of 128 lanes hold a column, 189 Q2
+// points fill three rounds of a wave), or for meshes of few cells, where the
+// length of one thread's work counts, 1 on one wave with a thread per column
+// and plane of points.
+constexpr int MF_CELLS = 7;
+template <int NCELL>
+constexpr int mf_threads() { return NCELL == 1 ? 64 : 128; }
 
-// waves per SIMD the register allocation aims at (FP64: also the LDS limit of
-// 4 workgroups per CU)
-template <int DEG, typename TH, typename TX>
-constexpr int mf_waves() { return std::is_same<mf_arith<TH, TX>, float>::value ? (DEG == 1 ? 5 : 6) : 4; }
+// waves per SIMD the register allocation aims at
+template <int DEG, typename TA, int NCELL>
+constexpr int mf_waves() { return NCELL == 1 ? 1 : std::is_same<TA, float>::value ? (DEG == 1 ? 4 : 3) : 2; }
 
-template <int DEG, typename TH, typename TX, bool RES = false>
-__global__ __launch_bounds__((mf_threads<DEG, TH>()), (mf_waves<DEG, TH, TX>())) void k_mf_apply(RefTables T, MeshDev Mh, Material M0,
-                                                                      const TH *__restrict__ Uq,
-                                                                      const TX *__restrict__ x,
-                                                                      const int *__restrict__ cells,
-                                                                      const int *__restrict__ flag,
-                                                                      mf_arith<TH, TX> *__restrict__ ycell)
+// The product of NCELL cells per workgroup.  Two stages in registers with
+// one exchange through LDS between them:
+//   columns  a thread owns one component of one cell: its NS node values stay
+//            in registers, and a plane of Gauss points at a time it forms X
+//            and the three gradients (Line), the divergence with the two
+//            other orbital components of its spin row (lane shuffles), the
+//            fluxes K1 G_k + K23 [k == own] div, and tests them at once
+//            (accumulators in registers).  Only X goes to LDS.
+//   points   a thread owns one point: the 18 values of X from LDS, the iterate
+//            from memory ([cell][component][point], so that the lanes read
+//            consecutive points), H(q) X(q) in registers, back over X in LDS.
+// and the columns then test it and write their NS values.  Before, a thread
+// per pencil passed every 1D pass through LDS, with nine barriers per cell.
+// XCD x works through the cells [x n8, (x+1) n8) in order, so neighbours
+// share their nodes' x in that XCD's L2.
+template <int DEG, typename TH, typename TX, bool RES, int NCELL>
+__global__ __launch_bounds__(mf_threads<NCELL>(), (mf_waves<DEG, mf_arith<TH, TX>, NCELL>())) void k_mf_apply(
+    MeshDev Mh, Material M0, const TH *__restrict__ Uq, const TX *__restrict__ x, int n_cells, int n8,
+    const int *__restrict__ flag, mf_arith<TH, TX> *__restrict__ ycell)
 {
   static_assert(!RES || (std::is_same<TH, double>::value && std::is_same<TX, double>::value), "FP64 residual");
+  constexpr bool SPLIT = NCELL == 1;  // a thread per column and plane of points
+  constexpr int MF_THREADS = mf_threads<NCELL>();
+  static_assert(SPLIT || NCELL * 18 <= 126, "a column per lane of two waves");
   using TA = mf_arith<TH, TX>;
-  constexpr int N1 = DEG + 1, NS = N1 * N1 * N1, NQ = NS, V = NS * 18, NTA = mf_threads<DEG, TH>();
-  constexpr int NP = N1 * N1 * 18;  // pencils per pass
-  constexpr int NH = NQ * 9;        // (point, component pair) items of H X
-  static_assert(NH <= NTA, "one H X item per thread");
-  // Regions of one value per (point or node, component), in the order
-  //   x -> A0 A1 -> B0 B1 B2 -> X G0 G1 G2 -> Z K0 K1 K2 -> C0 C1 C2 -> D0 D1,
-  // and the iterate U(q) of the product.
-  // A pencil reads exactly the points it writes, so the FP32 kernel lets each
-  // pass overwrite its inputs in place in one set of four regions, and keeps
-  // the point stage's pair sums and Z in four more (17.7 KB for Q2 with U(q):
-  // register-limited at 6 waves per SIMD).  The FP64 kernel alternates
-  // between two sets and keeps x (39 KB, 4 workgroups per CU), which saves a
-  // barrier and the Robin faces' second gather of x.
-  constexpr bool IP = std::is_same<TA, float>::value;
-  constexpr int NXR = (V + NTA - 1) / NTA;  // x values per thread
-  // room for the unconditional x and U(q) stores, U(q) after x
-  constexpr int SU_OFF = (IP ? 3 * V : 8 * V) + NXR * NTA;
-  constexpr int RS_OFF = SU_OFF + (RES ? 0 : NXR * NTA);
-  __shared__ TA S[RS_OFF + (IP && !RES ? 4 * V : 0)];
-  TA *const P0 = S, *const P1 = IP ? S : S + 4 * V, *const SX = IP ? S : S + 8 * V, *const SU = S + SU_OFF;
+  using L = Line<DEG, TA>;
+  constexpr int N = DEG + 1, N2 = N * N, NS = N2 * N, V = NS * 18;
+  // per cell: fluxes' factors A_k (own gradient) and B_k (divergence), 1/h_k,
+  // the bulk coefficients, Robin factor; A, B and the bulk ones with the
+  // cell's volume and W0^3
+  enum { CA = 0, CB = 3, CI = 6, CM = 9, CR = 16, NCONST = 17 };
+  __shared__ __attribute__((aligned(16))) TA sX[NCELL * V];
+  __shared__ TA sC[NCELL][NCONST];
+  __shared__ int sE[NCELL];
+  __shared__ int sNode[NCELL * NS];
+  __shared__ uint32_t sMask[NCELL * NS];
+  __shared__ TA sD[SPLIT ? 2 * V : 1];
   const int tid = threadIdx.x;
-  const int e = cells[blockIdx.x];
-  if (e < 0) return;                           // padding of the XCD-aware order
-  if (flag && !flag[Mh.cell_inst[e]]) return;  // instance not iterating: its rows are not read
-  const Material M = Mh.mats ? Mh.mats[Mh.cell_mat[e]] : M0;
-  const int *cn = Mh.cell_nodes + (size_t)e * NS;
-  double h[3];
-  TA ih[3];
-  for (int k = 0; k < 3; ++k) { h[k] = Mh.cell_h[3 * e + k]; ih[k] = (TA)(1.0 / h[k]); }
-  const double vol = h[0] * h[1] * h[2];
-  const uint32_t cface = Mh.cell_face[e];
-  TA L[N1][N1], dL[N1][N1];  // L[q][b] = L_b(x_q): uniform, scalar loads into scalar registers
-  const TA *tL, *tdL;
-  if constexpr (std::is_same<TA, float>::value) { tL = T.L1f; tdL = T.dL1f; }
-  else { tL = T.L1; tdL = T.dL1; }
+  const int in0 = NCELL * (blockIdx.x >> 3), e0 = (blockIdx.x & 7) * n8 + in0;  // this XCD's range
+  const int n_in = min(min(NCELL, n8 - in0), n_cells - e0);                     // may be <= 0
+  // the cells' nodes (and their masks) at once; a cell's instance flag beside
+  constexpr int NL = (NCELL * NS + MF_THREADS - 1) / MF_THREADS;
+  int nd[NL];
 #pragma unroll
-  for (int q = 0; q < N1; ++q)
+  for (int r = 0; r < NL; ++r) {
+    const int t = tid + r * MF_THREADS;
+    nd[r] = 0;
+    if (t < n_in * NS) nd[r] = Mh.cell_nodes[(size_t)e0 * NS + t];
+  }
+  if (tid < NCELL) {
+    int e = tid < n_in ? e0 + tid : -1;
+    if (e >= 0 && flag && !flag[Mh.cell_inst[e]]) e = -1;  // instance not iterating: its rows are not read
+    sE[tid] = e;
+  }
+  uint32_t mk[NL], mor = 0;
 #pragma unroll
-    for (int b = 0; b < N1; ++b) {
-      L[q][b] = tL[q * N1 + b];
-      dL[q][b] = tdL[q * N1 + b];
+  for (int r = 0; r < NL; ++r) {
+    const int t = tid + r * MF_THREADS;
+    if (t < NCELL * NS) sNode[t] = nd[r];
+    if constexpr (!RES) mk[r] = Mh.node_mask[nd[r]];
+  }
+  __syncthreads();
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < NCELL; ++j) any = any || sE[j] >= 0;
+  if (!any) return;  // uniform: padding, or instances that are not iterating
+  // the column of this thread: component c of cell j; three neighbouring
+  // lanes hold the orbital components of one spin row (63 = 21 triples per
+  // wave; lane 63 repeats its neighbour and writes nothing)
+  constexpr int NCOL = SPLIT ? 18 * N : 18 * NCELL;
+  const int lane = tid & 63, col0 = 63 * (tid >> 6) + (lane < 63 ? lane : 62);
+  const int col = min(col0, NCOL - 1);
+  const int pl = SPLIT ? col / 18 : 0;  // SPLIT: the plane of points, and of nodes in the end
+  const int j = SPLIT ? 0 : col / 18, c = col % 18, kc = c % 3;
+  const int e = sE[j];
+  const bool on = lane < 63 && col == col0 && e >= 0;
+  TA v[NS];
+#pragma unroll
+  for (int a = 0; a < NS; ++a) v[a] = (TA)x[(size_t)sNode[j * NS + a] * 18 + c];
+  // the cells' constants, while x is on its way
+  constexpr int TC = SPLIT ? NCOL : 64;  // threads without a column, or the second wave's first
+  if (tid >= TC && tid < TC + NCELL) {
+    const int ec = max(sE[tid - TC], 0);
+    const Material M = Mh.mats ? Mh.mats[Mh.cell_mat[ec]] : M0;
+    double h[3], ih[3];
+    for (int k = 0; k < 3; ++k) { h[k] = Mh.cell_h[3 * ec + k]; ih[k] = 1.0 / h[k]; }
+    const double vol = h[0] * h[1] * h[2], s = vol * (L::W0 * L::W0 * L::W0);
+    TA *C = sC[tid - TC];
+    for (int k = 0; k < 3; ++k) {
+      C[CA + k] = (TA)(s * M.K1 * ih[k] * ih[k]);
+      C[CB + k] = (TA)(s * M.K23 * ih[k]);
+      C[CI + k] = (TA)ih[k];
     }
-  // A wave's vector loads may return out of order, so a wait for one is a
-  // wait for all outstanding.  x at the cell's nodes is therefore gathered
-  // and stored to LDS first, and U(q) is requested after that wait: it stays
-  // in flight through the interpolation passes, which wait only on LDS.
-  // Both without branches (indices clamped into range, unused values stored
-  // to padding).
-  // x, Dirichlet components 0 (the masked columns; the residual's iterate as it is):
-  auto xval = [&](int i) -> TA {
-    const int node = cn[i / 18], c = i % 18;
-    const TA xv = (TA)x[(size_t)node * 18 + c];
-    if constexpr (RES) return xv;
-    return ((Mh.node_mask[node] >> c) & 1u) ? (TA)0 : xv;
+    C[CM + 0] = (TA)(s * M.al);
+    C[CM + 1] = (TA)(2.0 * s * M.b1);
+    C[CM + 2] = (TA)(2.0 * s * M.b2);
+    C[CM + 3] = (TA)(2.0 * s * (M.b3 + M.b4 + M.b5));
+    C[CM + 4] = (TA)(2.0 * s * (M.b4 + M.b5 - M.b3));
+    C[CM + 5] = (TA)(2.0 * s * (M.b3 + M.b4 - M.b5));
+    C[CM + 6] = (TA)(2.0 * s * (M.b3 - M.b4 + M.b5));
+    C[CR] = (TA)(M.robin * vol);
+  }
+  if constexpr (RES) {
+    __syncthreads();
+  } else {
+    // Dirichlet components 0 (the masked columns): few cells have any
+#pragma unroll
+    for (int r = 0; r < NL; ++r) {
+      const int t = tid + r * MF_THREADS;
+      if (t < NCELL * NS) {
+        sMask[t] = mk[r];
+        mor |= mk[r];
+      }
+    }
+    if (__syncthreads_or((int)(mor & 0x3ffffu))) {
+#pragma unroll
+      for (int a = 0; a < NS; ++a)
+        if ((sMask[j * NS + a] >> c) & 1u) v[a] = (TA)0;
+    }
+  }
+  // SPLIT: the point's iterate already now (registers are free there)
+  TA s[18];
+  const auto load_u = [&](int p, int ep) {
+    const int q = p % NS;
+    const TH *Up = Uq + (size_t)ep * V + q;
+#pragma unroll
+    for (int i = 0; i < 18; ++i) s[i] = (TA)Up[i * NS];
   };
+  if constexpr (SPLIT && !RES) load_u(min(tid, NS - 1), e);
+  const TA *Cj = sC[j];
+  // z lines to coefficients: kz[b] of line b = by N + bx
+  // acc: coefficients of the z lines of the result (SPLIT: the tested values
+  // and z-derivatives of the own plane)
+  TA kz[N2][N], acc[N2][SPLIT ? 2 : N];
 #pragma unroll
-  for (int r = 0; r < NXR; ++r) {
-    const int i = tid + r * NTA;
-    const TA v = xval(i < V ? i : V - 1);
-    SX[i] = i < V ? v : (TA)0;  // beyond V: the padding, never read
-  }
-  // keep the U(q) loads below the x stores (and so below their wait)
-  __builtin_amdgcn_sched_barrier(0);
-  TH us[NXR];  // this thread's share of the cell's U(q), stored to LDS after the z pass
-  if constexpr (!RES) {
-    const TH *Uc = Uq + (size_t)e * V;
+  for (int b = 0; b < N2; ++b) {
 #pragma unroll
-    for (int r = 0; r < NXR; ++r) {
-      const int i = tid + r * NTA;
-      us[r] = Uc[i < V ? i : V - 1];
+    for (int i = 0; i < N; ++i) {
+      kz[b][i] = v[i * N2 + b];
+      if (i < (SPLIT ? 2 : N)) acc[b][i] = (TA)0;
     }
+    if constexpr (DEG == 2) L::coef(kz[b][0], kz[b][1], kz[b][2]);
   }
-  const int hq = tid / 9 < NQ ? tid / 9 : NQ - 1, hc = tid % 9;  // H X item: point hq, components hc, hc + 9
-  __syncthreads();
-  auto at = [](int i0, int i1, int i2, int c) { return ((i2 * N1 + i1) * N1 + i0) * 18 + c; };
-  const int c = tid % 18, l = tid / 18, la = l % N1, lb = l / N1;  // pencil: line (la, lb), component c
-  const bool pen = tid < NP;
-  // x pass: line (by, bz) -> (qx, by, bz): x -> A0 A1
-  if (pen) {
-    TA v[N1];
+  TA *const Xc = sX + j * V + c;
+  {
+    const TA a0 = Cj[CA], a1 = Cj[CA + 1], a2 = Cj[CA + 2];
+    const TA b0 = kc == 0 ? Cj[CB] : (TA)0, b1 = kc == 1 ? Cj[CB + 1] : (TA)0, b2 = kc == 2 ? Cj[CB + 2] : (TA)0;
+    const TA m0 = kc == 0 ? Cj[CI] : (TA)0, m1 = kc == 1 ? Cj[CI + 1] : (TA)0, m2 = kc == 2 ? Cj[CI + 2] : (TA)0;
+    const int s1 = lane - kc + (kc + 1) % 3, s2 = lane - kc + (kc + 2) % 3;
+#pragma unroll 1
+    for (int qi = 0; qi < (SPLIT ? 1 : N); ++qi) {
+      const int qz = SPLIT ? pl : qi;
+      L ln;
+      ln.point(qz);
+      TA Y0[N][N], Yd[N][N], Y1[N][N];  // [qy][bx]
 #pragma unroll
-    for (int b = 0; b < N1; ++b) v[b] = SX[at(b, la, lb, c)];
+      for (int bx = 0; bx < N; ++bx) {
+        TA z0[N], z1[N], p[N], g[N];
 #pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      TA a0 = 0, a1 = 0;
+        for (int by = 0; by < N; ++by) {
+          z0[by] = ln.val(kz[by * N + bx]);
+          z1[by] = ln.der(kz[by * N + bx]);
+        }
+        L::both(z0, p, g);
 #pragma unroll
-      for (int b = 0; b < N1; ++b) {
-        a0 += L[q][b] * v[b];
-        a1 += dL[q][b] * v[b];
+        for (int q = 0; q < N; ++q) { Y0[q][bx] = p[q]; Yd[q][bx] = g[q]; }
+        L::values(z1, p);
+#pragma unroll
+        for (int q = 0; q < N; ++q) Y1[q][bx] = p[q];
       }
-      P1[at(q, la, lb, c)] = a0;
-      P1[V + at(q, la, lb, c)] = a1;
-    }
-  }
-  __syncthreads();
-  // y pass: line (qx, bz) -> (qx, qy, bz): A0 A1 -> B0 B1 B2
-  if (pen) {
-    TA v0[N1], v1[N1];
+      TA C0[N][N], C1[N][N], C2[N][N];  // [qy][ax]
 #pragma unroll
-    for (int b = 0; b < N1; ++b) {
-      v0[b] = P1[at(la, b, lb, c)];
-      v1[b] = P1[V + at(la, b, lb, c)];
-    }
+      for (int qy = 0; qy < N; ++qy) {
+        __builtin_amdgcn_sched_barrier(0);  // a row at a time: the rows' temporaries share registers
+        TA X[N], g0[N], g1[N], g2[N];
+        L::both(Y0[qy], X, g0);
+        L::values(Yd[qy], g1);
+        L::values(Y1[qy], g2);
 #pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      TA b0 = 0, b1 = 0, b2 = 0;
-#pragma unroll
-      for (int b = 0; b < N1; ++b) {
-        b0 += L[q][b] * v0[b];
-        b1 += L[q][b] * v1[b];
-        b2 += dL[q][b] * v0[b];
+        for (int qx = 0; qx < N; ++qx) {
+          if (on) Xc[((qz * N + qy) * N + qx) * 18] = X[qx];
+          const TA own = m0 * g0[qx] + m1 * g1[qx] + m2 * g2[qx];
+          const TA div = own + __shfl(own, s1) + __shfl(own, s2);
+          g0[qx] = a0 * g0[qx] + b0 * div;
+          g1[qx] = a1 * g1[qx] + b1 * div;
+          g2[qx] = a2 * g2[qx] + b2 * div;
+        }
+        L::test_d(g0, C0[qy]);
+        L::test_v(g1, C1[qy]);
+        L::test_v(g2, C2[qy]);
       }
-      P0[at(la, q, lb, c)] = b0;
-      P0[V + at(la, q, lb, c)] = b1;
-      P0[2 * V + at(la, q, lb, c)] = b2;
-    }
-  }
-  __syncthreads();
-  // z pass: line (qx, qy) -> (qx, qy, qz) = q: B0 B1 B2 -> X G0 G1 G2
-  if (pen) {
-    TA v0[N1], v1[N1], v2[N1];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int b = 0; b < N1; ++b) {
-      v0[b] = P0[at(la, lb, b, c)];
-      v1[b] = P0[V + at(la, lb, b, c)];
-      v2[b] = P0[2 * V + at(la, lb, b, c)];
-    }
+      for (int ax = 0; ax < N; ++ax) {
+        TA p[N], g[N], d0[N], d2[N];
 #pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      TA xv = 0, g0 = 0, g1 = 0, g2 = 0;
+        for (int q = 0; q < N; ++q) { p[q] = C0[q][ax]; g[q] = C1[q][ax]; }
+        L::test_vd(p, g, d0);
 #pragma unroll
-      for (int b = 0; b < N1; ++b) {
-        xv += L[q][b] * v0[b];
-        g0 += L[q][b] * v1[b];
-        g1 += L[q][b] * v2[b];
-        g2 += dL[q][b] * v0[b];
+        for (int q = 0; q < N; ++q) p[q] = C2[q][ax];
+        L::test_v(p, d2);
+#pragma unroll
+        for (int ay = 0; ay < N; ++ay) {
+          if constexpr (SPLIT) {
+            acc[ay * N + ax][0] = d0[ay];
+            acc[ay * N + ax][1] = d2[ay];
+          } else {
+            ln.back(d0[ay], d2[ay], acc[ay * N + ax]);
+          }
+        }
       }
-      const int o = at(la, lb, q, c);
-      P1[o] = xv;
-      P1[V + o] = g0 * ih[0];
-      P1[2 * V + o] = g1 * ih[1];
-      P1[3 * V + o] = g2 * ih[2];
     }
-  }
-  if constexpr (!RES) {
-#pragma unroll
-    for (int r = 0; r < NXR; ++r) SU[tid + r * NTA] = (TA)us[r];  // beyond V: padding, never read
   }
   __syncthreads();
-  // w vol H(q) X(q) and w vol gamma_k(q) / h_k for the components hc and hc + 9
-  // of point hq: read everything, then write Z and K.
-  // SPLIT (the product): H(q) X(q) from the point's shared pair sums
-  // (hx_row_sums, hx_from_sums), one more barrier.  Regions: the z pass left
-  // X G0 G1 G2 in P1; the pair sums (54 per point, 3V in all) go to RS, then
-  // Z to Zs = RS + 3V and K over G (Ks = P1 + V); the test passes write C to
-  // P0 and D to P1.  FP64: RS is P0, dead after the z pass; FP32: RS is a
-  // region of its own, and P0 = P1.  The residual (not SPLIT) writes Z and K
-  // over the regions of P0.
-  constexpr bool SPLIT = !RES;
-  TA *const RS = IP ? S + RS_OFF : P0;
-  TA *const Zs = SPLIT ? RS + 3 * V : P0, *const Ks = SPLIT ? P1 + V : P0 + V;
-  TA *const Cd = SPLIT ? P0 : P1, *const Dd = SPLIT ? P1 : P0;
-  TA zo[2], ko[2][3];
-  if (tid < NH) {
-    const TA wv = (TA)(T.w[hq] * vol), K1 = (TA)M.K1, K23 = (TA)M.K23;
-    const int mu = hc / 3, kc = hc % 3;
-    if constexpr (RES) {  // rho first: fewer registers live through it
-      double ru, rv;
-      rho_pair(&P1[hq * 18], mu, kc, M, ru, rv);
-      zo[0] = wv * ru;
-      zo[1] = wv * rv;
-    }
+  // the points: vol w H(q) X(q) (the points' relative weights come with the
+  // test passes), or rho(X(q)) for the residual
+#pragma unroll 1
+  for (int p = tid; p < NCELL * NS; p += MF_THREADS) {
+    const int jp = p / NS, ep = sE[jp];
+    if (ep < 0) continue;
+    const TA *Cp = sC[jp] + CM;
+    TA xp[18];
+    if constexpr (!SPLIT && !RES) load_u(p, ep);
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int i = hq * 18 + hc + 9 * r, base = hq * 18 + 9 * r + 3 * mu;
-      const TA dv = P1[V + base] + P1[2 * V + base + 1] + P1[3 * V + base + 2];
+    for (int i = 0; i < 18; ++i) xp[i] = sX[p * 18 + i];
+    BulkMat<TA> B;
+    TA uu[6], vv[6], uv[9];
+    gram(RES ? xp : s, uu, vv, uv);
+    B.set(uu, vv, uv, Cp[0], Cp[1], Cp[2], Cp[3], Cp[4], Cp[5], Cp[6]);
+    if constexpr (RES) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) ko[r][k] = wv * ih[k] * (K1 * P1[(1 + k) * V + i] + (k == kc ? K23 * dv : (TA)0));
+      for (int k = 0; k < 3; ++k) {
+        TA zu[3] = {0, 0, 0}, zv[3] = {0, 0, 0};
+        B.add(xp, xp + 9, k, zu, zv);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) { sX[p * 18 + 3 * m + k] = zu[m]; sX[p * 18 + 9 + 3 * m + k] = zv[m]; }
+      }
+    } else {
+      BulkMat<TA> D;
+      __builtin_amdgcn_sched_barrier(0);
+      dgram(s, xp, uu, vv, uv);
+      D.set(uu, vv, uv, (TA)0, Cp[1], Cp[2], Cp[3], Cp[4], Cp[5], Cp[6]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        __builtin_amdgcn_sched_barrier(0);
+        TA zu[3] = {0, 0, 0}, zv[3] = {0, 0, 0};
+        B.add(xp, xp + 9, k, zu, zv);
+        D.add(s, s + 9, k, zu, zv);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) { sX[p * 18 + 3 * m + k] = zu[m]; sX[p * 18 + 9 + 3 * m + k] = zv[m]; }
+      }
     }
   }
+  __syncthreads();
+  if (!SPLIT && !on) return;
+#pragma unroll 1
+  for (int qi = 0; qi < (SPLIT ? 1 : N); ++qi) {
+    const int qz = SPLIT ? pl : qi;
+    L ln;
+    ln.point(qz);
+    TA C0[N][N];
+#pragma unroll
+    for (int qy = 0; qy < N; ++qy) {
+      TA z[N];
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) z[qx] = Xc[((qz * N + qy) * N + qx) * 18];
+      L::test_v(z, C0[qy]);
+    }
+#pragma unroll
+    for (int ax = 0; ax < N; ++ax) {
+      TA p[N], d[N];
+#pragma unroll
+      for (int q = 0; q < N; ++q) p[q] = C0[q][ax];
+      L::test_v(p, d);
+#pragma unroll
+      for (int ay = 0; ay < N; ++ay) {
+        if constexpr (SPLIT) acc[ay * N + ax][0] += d[ay];
+        else ln.back(d[ay], acc[ay * N + ax]);
+      }
+    }
+  }
+  // the node values of the column (SPLIT: of its plane pl of nodes, summed
+  // over the planes of points through LDS)
+  TA out[N2][SPLIT ? 1 : N];
   if constexpr (SPLIT) {
-    // pair p of point tid / 6 (162 items for Q2), then the 9 items per point;
-    // 54 values per point (48 used) keep each pair's 8 values 16-byte aligned
-    // for 128-bit LDS accesses; of the strides 48-54 it ran fastest (an odd
-    // stride, 49, cost 10% of the kernel in bank conflicts)
-    if (tid < NQ * 6) {
-      const int sq = tid / 6, p = tid % 6;
-      hx_row_sums(SU + sq * 18, P1 + sq * 18, p, RS + sq * 54 + p * 8);
+    if (on) {
+#pragma unroll
+      for (int b = 0; b < N2; ++b) {
+        sD[(2 * pl * N2 + b) * 18 + c] = acc[b][0];
+        sD[((2 * pl + 1) * N2 + b) * 18 + c] = acc[b][1];
+      }
     }
     __syncthreads();
-    if (tid < NH) {
-      TA z[2];
-      hx_from_sums(RS + hq * 54, SU + hq * 18, P1 + hq * 18, hc / 3, hc % 3, M, z[0], z[1]);
-      const TA wv = (TA)(T.w[hq] * vol);
-      zo[0] = wv * z[0];
-      zo[1] = wv * z[1];
-    }
-  }
-  if constexpr (IP && !SPLIT) __syncthreads();
-  if (tid < NH) {
+    if (!on) return;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int i = hq * 18 + hc + 9 * r;
-      Zs[i] = zo[r];
+    for (int b = 0; b < N2; ++b) out[b][0] = (TA)0;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) Ks[k * V + i] = ko[r][k];
-    }
-  }
-  __syncthreads();
-  // test z pass: line (qx, qy) -> (qx, qy, az): Z K0 K1 K2 -> C0 C1 C2
-  if (pen) {
-    TA z[N1], k0[N1], k1[N1], k2[N1];
+    for (int q = 0; q < N; ++q) {
+      TA p[N] = {}, g[N] = {}, one[N], wv, wd;  // weight times value and derivative of L_pl at point q
+      p[q] = g[q] = (TA)1;
+      L::test_v(p, one);
+      wv = pl == 0 ? one[0] : pl == 1 ? one[1] : one[N - 1];
+      L::test_d(g, one);
+      wd = pl == 0 ? one[0] : pl == 1 ? one[1] : one[N - 1];
 #pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      const int o = at(la, lb, q, c);
-      z[q] = Zs[o];
-      k0[q] = Ks[o];
-      k1[q] = Ks[V + o];
-      k2[q] = Ks[2 * V + o];
-    }
-#pragma unroll
-    for (int a = 0; a < N1; ++a) {
-      TA c0 = 0, c1 = 0, c2 = 0;
-#pragma unroll
-      for (int q = 0; q < N1; ++q) {
-        c0 += L[q][a] * z[q] + dL[q][a] * k2[q];
-        c1 += L[q][a] * k0[q];
-        c2 += L[q][a] * k1[q];
+      for (int b = 0; b < N2; ++b) {
+        out[b][0] += wv * sD[(2 * q * N2 + b) * 18 + c];
+        out[b][0] += wd * sD[((2 * q + 1) * N2 + b) * 18 + c];
       }
-      const int o = at(la, lb, a, c);
-      Cd[o] = c0;
-      Cd[V + o] = c1;
-      Cd[2 * V + o] = c2;
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < N2; ++b) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) out[b][i] = acc[b][i];
+      if constexpr (DEG == 2) L::uncoef(out[b][0], out[b][1], out[b][2]);
     }
   }
-  __syncthreads();
-  // test y pass: line (qx, az) -> (qx, ay, az): C0 C1 C2 -> D0 D1
-  if (pen) {
-    TA v0[N1], v1[N1], v2[N1];
+  // Robin faces: robin * area * (1D masses along the face) on the components
+  // that the wall does not hold at zero
+  const TA rob = Cj[CR];
+  if (rob != (TA)0) {
+    const uint32_t cface = Mh.cell_face[e];
 #pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      const int o = at(la, q, lb, c);
-      v0[q] = Cd[o];
-      v1[q] = Cd[V + o];
-      v2[q] = Cd[2 * V + o];
-    }
+    for (int lf = 0; lf < 6; ++lf) {
+      const int bid = (int)((cface >> (3 * lf)) & 7u) - 1;
+      if (bid < 2 || bid > 4 || face_zeroed(bid, c)) continue;
+      // nodes of the face: f0 + i s0 + k s1 in the lexicographic order
+      const int s0 = lf < 2 ? N : 1, s1 = lf < 4 ? N2 : N;
+      const int f0 = (lf & 1) ? (N - 1) * (lf < 2 ? 1 : (lf < 4 ? N : N2)) : 0;
+      TA t[N][N];
 #pragma unroll
-    for (int a = 0; a < N1; ++a) {
-      TA d0 = 0, d1 = 0;
+      for (int i = 0; i < N; ++i) {
+        TA u[N];
 #pragma unroll
-      for (int q = 0; q < N1; ++q) {
-        d0 += L[q][a] * v0[q] + dL[q][a] * v2[q];
-        d1 += L[q][a] * v1[q];
-      }
-      Dd[at(la, a, lb, c)] = d0;
-      Dd[V + at(la, a, lb, c)] = d1;
-    }
-  }
-  __syncthreads();
-  // test x pass: line (ay, az) -> (ax, ay, az) = a, then the Robin faces
-  if (pen) {
-    TA v0[N1], v1[N1];
-#pragma unroll
-    for (int q = 0; q < N1; ++q) {
-      v0[q] = Dd[at(q, la, lb, c)];
-      v1[q] = Dd[V + at(q, la, lb, c)];
-    }
-#pragma unroll
-    for (int a = 0; a < N1; ++a) {
-      TA r = 0;
-#pragma unroll
-      for (int q = 0; q < N1; ++q) r += L[q][a] * v0[q] + dL[q][a] * v1[q];
-      const int na = (lb * N1 + la) * N1 + a, o = at(a, la, lb, c);
-      if (M.robin != 0.0)
-        for (int lf = 0; lf < 6; ++lf) {
-          const int bid = (int)((cface >> (3 * lf)) & 7u) - 1;
-          if (bid < 2 || bid > 4 || face_zeroed(bid, c)) continue;
-          const double *mf = T.Mf + (lf * NS + na) * NS;
-          TA sf = 0;
-          for (int b = 0; b < NS; ++b) sf += (TA)mf[b] * (IP ? xval(b * 18 + c) : SX[b * 18 + c]);
-          r += (TA)(M.robin * face_area(lf, h)) * sf;
+        for (int k = 0; k < N; ++k) {
+          const int a = j * NS + f0 + i * s0 + k * s1;
+          u[k] = (TA)x[(size_t)sNode[a] * 18 + c];
+          if constexpr (!RES)
+            if ((sMask[a] >> c) & 1u) u[k] = (TA)0;
         }
-      ycell[(size_t)e * V + o] = r;  // Dirichlet rows are replaced in the gather
+        L::mass(u, t[i]);
+      }
+      const TA f = rob * Cj[CI + lf / 2] * (TA)(L::M0 * L::M0);
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        TA u[N], y[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) u[i] = t[i][k];
+        L::mass(u, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const int a = f0 + i * s0 + k * s1;
+          if constexpr (!SPLIT) out[a % N2][a / N2] += f * y[i];
+          else if (a / N2 == pl) out[a % N2][0] += f * y[i];
+        }
+      }
     }
+  }
+  TA *const Y = ycell + (size_t)e * V + c;  // Dirichlet rows are replaced in the gather
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int b = 0; b < N2; ++b) Y[(pl * N2 + b) * 18] = out[b][0];
+  } else {
+#pragma unroll
+    for (int a = 0; a < NS; ++a) Y[a * 18] = out[a % N2][a / N2];
   }
 }
 
@@ -1136,37 +1351,56 @@ hipError_t launch_mf_setup(int deg, bool u32, const RefTables &T, const MeshDev 
   return hipGetLastError();
 }
 
-hipError_t launch_mf_apply(int deg, bool u32, bool x32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const void *Uq, const void *x, const int *cells, int n, const int *flag, void *ycell,
-                           hipStream_t s)
+namespace {
+// workgroups of nc cells: XCD x (workgroup index mod 8) takes the cells
+// [x n8, (x + 1) n8)
+inline int mf_range(int n_cells) { return (n_cells + 7) / 8; }
+inline int mf_grid(int n_cells, int nc) { return 8 * ((mf_range(n_cells) + nc - 1) / nc); }
+// Up to this many cells a thread takes one plane of one column (NCELL = 1):
+// its work is a third as long, but it reads and transforms the column once
+// per plane.  Measured, us per launch, NCELL 1 against 7: Q2 FP64 product
+// 7.5 / 12.1 at 8^3 cells, 9.8 / 13.4 at 10^3, 16.2 / 14.8 at 12^3; Q2 FP32
+// 9.6 / 12.0 at 12^3, 12.6 / 14.3 at 14^3; Q1 FP64 6.1 / 6.0 at 8^3 (residual
+// 5.1 / 5.7), 8.4 / 6.4 at 12^3.
+template <int DEG, typename TA>
+constexpr int mf_small_mesh() { return DEG == 1 ? 512 : std::is_same<TA, float>::value ? 3072 : 1536; }
+
+template <int DEG, typename TH, typename TX, bool RES>
+hipError_t mf_launch(const MeshDev &M, const Material &mat, const void *Uq, const void *x, int n_cells,
+                     const int *flag, void *ycell, hipStream_t s)
 {
-  if (n <= 0) return hipSuccess;
-  if (x32 && !u32) return hipErrorInvalidValue;  // an FP64 operator is applied to FP64 vectors only
-#define GLH_MFA(D, TH, TX)                                                                                  \
-  hipLaunchKernelGGL((k_mf_apply<D, TH, TX>), dim3(n), dim3((mf_threads<D, TH>())), 0, s, T, M, mat, (const TH *)Uq, \
-                     (const TX *)x, cells, flag, (mf_arith<TH, TX> *)ycell)
-  if (deg == 1) {
-    if (u32) { if (x32) GLH_MFA(1, float, float); else GLH_MFA(1, float, double); }
-    else GLH_MFA(1, double, double);
-  } else {
-    if (u32) { if (x32) GLH_MFA(2, float, float); else GLH_MFA(2, float, double); }
-    else GLH_MFA(2, double, double);
-  }
-#undef GLH_MFA
+  using TA = mf_arith<TH, TX>;
+  if (n_cells <= mf_small_mesh<DEG, TA>())
+    hipLaunchKernelGGL((k_mf_apply<DEG, TH, TX, RES, 1>), dim3(mf_grid(n_cells, 1)), dim3(mf_threads<1>()), 0, s, M,
+                       mat, (const TH *)Uq, (const TX *)x, n_cells, mf_range(n_cells), flag, (TA *)ycell);
+  else
+    hipLaunchKernelGGL((k_mf_apply<DEG, TH, TX, RES, MF_CELLS>), dim3(mf_grid(n_cells, MF_CELLS)),
+                       dim3(mf_threads<MF_CELLS>()), 0, s, M, mat, (const TH *)Uq, (const TX *)x, n_cells, mf_range(n_cells), flag, (TA *)ycell);
   return hipGetLastError();
 }
+}  // namespace
 
-hipError_t launch_res_apply(int deg, const RefTables &T, const MeshDev &M, const Material &mat, const double *U,
-                            const int *cells, int n, double *ycell, hipStream_t s)
+hipError_t launch_mf_apply(int deg, bool u32, bool x32, const MeshDev &M, const Material &mat, const void *Uq,
+                           const void *x, int n_cells, const int *flag, void *ycell, hipStream_t s)
 {
-  if (n <= 0) return hipSuccess;
-#define GLH_RES(D)                                                                                               \
-  hipLaunchKernelGGL((k_mf_apply<D, double, double, true>), dim3(n), dim3((mf_threads<D, double>())), 0, s, T, M, \
-                     mat, (const double *)nullptr, U, cells, M.inst_active, ycell)
-  if (deg == 1) GLH_RES(1);
-  else GLH_RES(2);
-#undef GLH_RES
-  return hipGetLastError();
+  if (n_cells <= 0) return hipSuccess;
+  if (x32 && !u32) return hipErrorInvalidValue;  // an FP64 operator is applied to FP64 vectors only
+  if (deg == 1) {
+    if (x32) return mf_launch<1, float, float, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+    if (u32) return mf_launch<1, float, double, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+    return mf_launch<1, double, double, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+  }
+  if (x32) return mf_launch<2, float, float, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+  if (u32) return mf_launch<2, float, double, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+  return mf_launch<2, double, double, false>(M, mat, Uq, x, n_cells, flag, ycell, s);
+}
+
+hipError_t launch_res_apply(int deg, const MeshDev &M, const Material &mat, const double *U, int n_cells,
+                            double *ycell, hipStream_t s)
+{
+  if (n_cells <= 0) return hipSuccess;
+  if (deg == 1) return mf_launch<1, double, double, true>(M, mat, nullptr, U, n_cells, M.inst_active, ycell, s);
+  return mf_launch<2, double, double, true>(M, mat, nullptr, U, n_cells, M.inst_active, ycell, s);
 }
 
 hipError_t launch_res_gather(int n_nodes, const int *ptr, const int *idx, const double *ycell, const uint32_t *mask,

@@ -19,9 +19,6 @@ struct RefTables {
   const double *Sp;   // [NPAIR*9]  sum_q w_q dN_a/dxi_k dN_b/dxi_l, index k*3+l
   const double *Mf;   // [6*NS*NS]  face mass on each unit face
   const int *pa, *pb; // [NPAIR]    pair list (a <= b)
-  const double *L1;   // [N1*N1]   1D Lagrange basis: L1[qx*N1 + bx] = L_bx(x_qx)
-  const double *dL1;  // [N1*N1]   its derivative
-  const float *L1f, *dL1f;  // the two rounded to FP32
 };
 
 struct Material {
@@ -116,10 +113,10 @@ hipError_t launch_transfer(int n_nodes, int deg, const int *cell, const float *t
 hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDev &M, const Material &mat,
                            const double *U, const int *cells, int n, void *J, hipStream_t s);
 // Matrix-free Jacobian: per cell the iterate at the quadrature points (Uq:
-// [n_cells][NQ][18]; the product forms H(q) X(q) from it) and the diagonal
+// [n_cells][18][NQ]; the product forms H(q) X(q) from it) and the diagonal
 // blocks (Jd: [n_nodes][324], one more per hanging node on a constrained
 // mesh), the setup colour-ordered like the assembly; the product writes
-// each listed cell's contribution to its slot of ycell ([n_cells][NS][18]),
+// each cell's contribution to its slot of ycell ([n_cells][NS][18]),
 // and launch_mf_gather sums them per node (node -> cell*NS + a lists, fixed
 // order) and writes the Dirichlet rows.
 // u32: the iterate stored in FP32 (for the FP32 inner solve); x32: x in FP32.
@@ -131,20 +128,19 @@ hipError_t launch_mf_setup(int deg, bool u32, const RefTables &T, const MeshDev 
                            hipStream_t s);
 // flag (per instance, or null): cells and rows of instances whose flag is 0
 // are skipped, as in the batched SpMV.
-hipError_t launch_mf_apply(int deg, bool u32, bool x32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const void *Uq, const void *x, const int *cells, int n, const int *flag, void *ycell,
-                           hipStream_t s);
+hipError_t launch_mf_apply(int deg, bool u32, bool x32, const MeshDev &M, const Material &mat, const void *Uq,
+                           const void *x, int n_cells, const int *flag, void *ycell, hipStream_t s);
 // sh (or null): a diagonal term added to every row (the continuation shift).
 template <typename TX>
 hipError_t launch_mf_gather(int n_nodes, const int *ptr, const int *idx, const void *ycell, const uint32_t *mask,
                             const double *Jd, const double *sh, const TX *x, const TX *b, const int *row_seg,
                             const int *flag, TX *y, hipStream_t s);
-// The residual through the product's sum-factorised passes: the listed cells'
+// The residual through the product's sum-factorised passes: the cells'
 // contributions to R at U in their ycell slots (cells of batch instances that
 // are not active skipped), then rhs = -R, all rows written: 0 on the
 // Dirichlet components and on the rows of instances that are not active.
-hipError_t launch_res_apply(int deg, const RefTables &T, const MeshDev &M, const Material &mat, const double *U,
-                            const int *cells, int n, double *ycell, hipStream_t s);
+hipError_t launch_res_apply(int deg, const MeshDev &M, const Material &mat, const double *U, int n_cells,
+                            double *ycell, hipStream_t s);
 hipError_t launch_res_gather(int n_nodes, const int *ptr, const int *idx, const double *ycell, const uint32_t *mask,
                              const int *row_seg, const int *active, double *rhs, hipStream_t s);
 // Per-cell free energy into Fcell[cell] for cells [0, n_cells).
