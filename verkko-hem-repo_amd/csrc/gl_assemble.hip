@@ -1196,22 +1196,49 @@ __global__ void k_mf_gather(int n_nodes, const int *__restrict__ ptr, const int 
 // system_rhs = -R from the residual's cell contributions: each node's sum in
 // the fixed cell order, negated; 0 on the Dirichlet components and on the
 // rows of a batch instance that is not active (whose cells were skipped).
-// Every row is written, so the output needs no fill.
-__global__ void k_res_gather(int n_nodes, const int *__restrict__ ptr, const int *__restrict__ idx,
-                             const double *__restrict__ ycell, const uint32_t *__restrict__ mask,
-                             const int *__restrict__ row_seg, const int *__restrict__ active,
-                             double *__restrict__ rhs)
+// Every row is written, so the output needs no fill.  One workgroup per
+// reduction chunk (ch: instance, first dof, end dof; even bounds, so a pair
+// of components stays in one chunk), which also leaves the chunk's sum of
+// squares in partial (unless null): the norm costs no pass of its own over
+// rhs (14 us of 107 per residual of the 32^3 Q2 cube, 28 of 182 on 256
+// slabs).  8 waves per workgroup: a chunk of 4096 takes 4 rounds of pairs,
+// one of 1024 one.
+constexpr int GT = 512;
+__global__ __launch_bounds__(GT) void k_res_gather(const long long *__restrict__ ch, const int *__restrict__ ptr,
+                                                   const int *__restrict__ idx, const double *__restrict__ ycell,
+                                                   const uint32_t *__restrict__ mask,
+                                                   const int *__restrict__ active, double *__restrict__ rhs,
+                                                   double *__restrict__ partial)
 {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)n_nodes * 9) return;
-  const int node = (int)(i / 9), c = 2 * (int)(i % 9);
-  const bool on = !active || active[row_seg[node]];
-  double s0 = 0.0, s1 = 0.0;
-  if (on) slot_pair_sum(ptr, idx, ycell, node, c, s0, s1);
-  const uint32_t mk = mask[node];
-  const size_t o = (size_t)node * 18 + c;
-  rhs[o] = (on && !((mk >> c) & 1u)) ? -s0 : 0.0;
-  rhs[o + 1] = (on && !((mk >> (c + 1)) & 1u)) ? -s1 : 0.0;
+  __shared__ double sh[GT / 64];
+  const long long sg = ch[3 * blockIdx.x], beg = ch[3 * blockIdx.x + 1], end = ch[3 * blockIdx.x + 2];
+  const bool on = !active || active[sg];
+  double acc = 0.0;
+  for (long long o = beg + 2 * threadIdx.x; o < end; o += 2 * GT) {
+    const int node = (int)(o / 18), c = (int)(o - 18LL * node);
+    double2 r = {0.0, 0.0};
+    if (on) {
+      double s0 = 0.0, s1 = 0.0;
+      slot_pair_sum(ptr, idx, ycell, node, c, s0, s1);
+      const uint32_t mk = mask[node];
+      r.x = ((mk >> c) & 1u) ? 0.0 : -s0;
+      r.y = ((mk >> (c + 1)) & 1u) ? 0.0 : -s1;
+    }
+    *reinterpret_cast<double2 *>(rhs + o) = r;
+    acc += r.x * r.x;
+    acc += r.y * r.y;
+  }
+  if (!partial) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < GT / 64; ++i) t += sh[i];
+    partial[blockIdx.x] = t;
+  }
 }
 
 template <int DEG>
@@ -1403,13 +1430,12 @@ hipError_t launch_res_apply(int deg, const MeshDev &M, const Material &mat, cons
   return mf_launch<2, double, double, true>(M, mat, nullptr, U, n_cells, M.inst_active, ycell, s);
 }
 
-hipError_t launch_res_gather(int n_nodes, const int *ptr, const int *idx, const double *ycell, const uint32_t *mask,
-                             const int *row_seg, const int *active, double *rhs, hipStream_t s)
+hipError_t launch_res_gather(const SegInfo &S, const int *ptr, const int *idx, const double *ycell,
+                             const uint32_t *mask, const int *active, double *rhs, double *partial, hipStream_t s)
 {
-  if (n_nodes <= 0) return hipSuccess;
-  const long long n = (long long)n_nodes * 9;
-  hipLaunchKernelGGL(k_res_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n_nodes, ptr, idx, ycell, mask,
-                     row_seg, active, rhs);
+  if (S.n_chunks <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_res_gather, dim3(S.n_chunks), dim3(GT), 0, s, S.chunks, ptr, idx, ycell, mask, active, rhs,
+                     partial);
   return hipGetLastError();
 }
 

@@ -1387,6 +1387,14 @@ hipError_t launch_seg_mdot(const SegInfo &S, int k, const T *V, size_t ldv, cons
   return hipGetLastError();
 }
 
+hipError_t launch_seg_final(const SegInfo &S, const double *partial, double *out, hipStream_t s)
+{
+  if (S.n_chunks <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_seg_final<double>), dim3(seg_grid(S), 1), dim3(RT), 0, s, S.seg_chunk, S.n_seg, S.act, 1,
+                     partial, out, 1, 0, 0, (const int *)nullptr);
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_seg_sub_lincomb_norm(const SegInfo &S, int k, const T *V, size_t ldv, T *h, int ldh, T *w,
                                        T *partial, T *norm2, int ldo, int off, hipStream_t s, const int *flag,

@@ -407,15 +407,46 @@ int norm64(glh_ctx *c, const double *v, double *out)
 
 // system_rhs = -R at U into out, condensed on a constrained mesh: the cell
 // loop of compute_residual (residual.cc:164-289) in the cell slots, summed
-// per node in a fixed order (no colours, no fill: every row is written)
-int residual_cells(glh_ctx *c, const double *U, double *out)
+// per node in a fixed order (no colours, no fill: every row is written).
+// With norm2 (device, n_seg values) also ||R_s||^2, through the chunk
+// partials part.
+int residual_cells(glh_ctx *c, const double *U, double *out, double *part = nullptr, double *norm2 = nullptr)
 {
   const glh::MeshDev M = c->meshdev();
-  double *rcell = c->constrained ? c->rfull.p : out;
-  HIPCHK(c, glh::launch_res_apply(c->deg, M, c->mat, U, c->n_cells, c->mf_ycell.p, c->stream));
-  HIPCHK(c, glh::launch_res_gather(c->n_nodes, c->n2c_ptr.p, c->n2c_idx.p, c->mf_ycell.p, c->node_mask.p,
-                                   c->row_seg.p, M.inst_active, rcell, c->stream));
-  if (c->constrained) HIPCHK(c, glh::launch_condense_rhs(c->cons, c->rfull.p, out, c->stream));
+  const glh::SegInfo S = c->seg();
+  hipStream_t s = c->stream;
+  HIPCHK(c, glh::launch_res_apply(c->deg, M, c->mat, U, c->n_cells, c->mf_ycell.p, s));
+  HIPCHK(c, glh::launch_res_gather(S, c->n2c_ptr.p, c->n2c_idx.p, c->mf_ycell.p, c->node_mask.p, M.inst_active,
+                                   c->constrained ? c->rfull.p : out, c->constrained ? nullptr : part, s));
+  if (c->constrained) {
+    HIPCHK(c, glh::launch_condense_rhs(c->cons, c->rfull.p, out, s));
+    if (norm2) HIPCHK(c, glh::launch_seg_mdot<double>(S, 1, out, ndofs(c), out, part, norm2, 1, 0, false, s));
+  } else if (norm2) {
+    HIPCHK(c, glh::launch_seg_final(S, part, norm2, s));
+  }
+  return GLH_OK;
+}
+
+// -R at U into out and its per-instance ||R_s||^2 on the host
+int residual_norms(glh_ctx *c, const double *U, double *out, std::vector<double> &n2)
+{
+  HIPCHK(c, c->s_part.alloc((size_t)std::max(1, c->n_chunks)));
+  HIPCHK(c, c->s_norm.alloc(c->n_seg));
+  HIPCHK(c, c->pinv.alloc(c->n_seg));
+  if (c->timing) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
+  RCHK(residual_cells(c, U, out, c->s_part.p, c->s_norm.p));
+  if (c->timing) HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->pinv.p, c->s_norm.p, c->n_seg * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  n2.assign(c->pinv.p, c->pinv.p + c->n_seg);
+  if (c->timing) {
+    float ms = 0;
+    HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    c->asm_ms = ms;
+    c->asm_launches = 2;
+    c->rasm_ms_total += ms;
+    c->rasm_count += 1;
+  }
   return GLH_OK;
 }
 
@@ -1027,8 +1058,7 @@ int newton_step_impl(glh_ctx *c, double step, int damped, const std::vector<char
     HIPCHK(c, hipMemcpyAsync(c->s_alpha.p, c->pinv.p, S * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, glh::launch_seg_trial(c->seg(), c->U.p, c->dU.p, c->s_alpha.p, c->node_mask.p, c->X.p, c->stream));
     if (c->constrained) HIPCHK(c, glh::launch_distribute(c->cons, c->X.p, c->stream));  // iteration.cc:180
-    RCHK(assemble_at(c, c->X.p, false, true, false, c->res.p, false));
-    RCHK(seg_norm2(c, c->res.p, c2));
+    RCHK(residual_norms(c, c->X.p, c->res.p, c2));
     bool all = true;
     for (int i = 0; i < S; ++i) {
       cur[i] = std::sqrt(c2[i]);
@@ -1914,8 +1944,12 @@ int glh_rhs_norm(glh_ctx *c, double *nrm)
 int glh_residual(glh_ctx *c, double *nrm)
 {
   RCHK(check_ready(c));
-  RCHK(assemble_at(c, c->U.p, false, true, false, c->res.p, false));
-  return norm64(c, c->res.p, nrm);
+  std::vector<double> r2;
+  RCHK(residual_norms(c, c->U.p, c->res.p, r2));
+  double t = 0;
+  for (double x : r2) t += x;
+  *nrm = std::sqrt(t);
+  return GLH_OK;
 }
 
 int glh_residual_into(glh_ctx *c, const double *U, double *R, double *norm2)
@@ -1926,14 +1960,10 @@ int glh_residual_into(glh_ctx *c, const double *U, double *R, double *norm2)
     return fail(c, GLH_ERR_ARG,
                 "the mesh needs " + std::to_string(c->n_chunks) + " reduction chunks; glh_residual_into holds " +
                     std::to_string(glh::SCRATCH_DOUBLES) + " (use glh_residual)");
-  const size_t n = ndofs(c);
-  hipStream_t s = c->stream;
   // the residual at U into R (through the context's cell slots, allocated
-  // with the mesh)
-  RCHK(residual_cells(c, U, R));
-  // per-instance ||R_s||^2 with the chunk partials in the scratch array
-  HIPCHK(c, glh::launch_seg_mdot<double>(c->seg(), 1, R, n, R, c->scratch, norm2, 1, 0, false, s));
-  return GLH_OK;
+  // with the mesh) and per-instance ||R_s||^2 with the chunk partials in the
+  // scratch array
+  return residual_cells(c, U, R, c->scratch, norm2);
 }
 
 int glh_solve(glh_ctx *c, double rtol, int maxit, int restart, double stats[2])
@@ -1986,9 +2016,8 @@ int glh_instance_residuals(glh_ctx *c, double *R)
 {
   RCHK(check_ready(c));
   if (!R) return fail(c, GLH_ERR_ARG, "null output");
-  RCHK(assemble_at(c, c->U.p, false, true, false, c->res.p, false));
   std::vector<double> r2;
-  RCHK(seg_norm2(c, c->res.p, r2));
+  RCHK(residual_norms(c, c->U.p, c->res.p, r2));
   for (int i = 0; i < c->n_seg; ++i) R[i] = std::sqrt(r2[i]);
   return GLH_OK;
 }
@@ -2011,9 +2040,8 @@ int glh_newton_solve(glh_ctx *c, double rtol, int max_newton, double lin_tol, in
   int lin_total = 0, k = 0, trials_total = 0;
   const double t_start = now_s();
   double t0 = t_start;
-  RCHK(assemble_at(c, c->U.p, false, true, false, c->rhs.p, false));
   std::vector<double> r0(S), rcur(S), r2;
-  RCHK(seg_norm2(c, c->rhs.p, r2));
+  RCHK(residual_norms(c, c->U.p, c->rhs.p, r2));
   for (int i = 0; i < S; ++i) r0[i] = rcur[i] = std::sqrt(r2[i]);
   t_asm += now_s() - t0;
   std::vector<double> &st = c->inst_stats;

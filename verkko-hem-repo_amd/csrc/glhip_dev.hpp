@@ -141,8 +141,6 @@ hipError_t launch_mf_gather(int n_nodes, const int *ptr, const int *idx, const v
 // Dirichlet components and on the rows of instances that are not active.
 hipError_t launch_res_apply(int deg, const MeshDev &M, const Material &mat, const double *U, int n_cells,
                             double *ycell, hipStream_t s);
-hipError_t launch_res_gather(int n_nodes, const int *ptr, const int *idx, const double *ycell, const uint32_t *mask,
-                             const int *row_seg, const int *active, double *rhs, hipStream_t s);
 // Per-cell free energy into Fcell[cell] for cells [0, n_cells).
 hipError_t launch_energy(int deg, const RefTables &T, const MeshDev &M, const Material &mat, const double *U,
                          int n_cells, double *Fcell, hipStream_t s);
@@ -243,6 +241,12 @@ struct SegInfo {
   // it is most of the cost
   int cap = 0;
 };
+// rhs = -R from the residual's cell slots (launch_res_apply); with partial,
+// the chunks' sums of squares of rhs there (for launch_seg_final).
+hipError_t launch_res_gather(const SegInfo &S, const int *ptr, const int *idx, const double *ycell,
+                             const uint32_t *mask, const int *active, double *rhs, double *partial, hipStream_t s);
+// out[s] = sum of the partials of instance s's chunks (one value per chunk)
+hipError_t launch_seg_final(const SegInfo &S, const double *partial, double *out, hipStream_t s);
 template <typename T>
 struct GmresCtl;
 
