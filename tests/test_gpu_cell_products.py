@@ -55,3 +55,25 @@ def test_residual_and_product_match_the_oracle_cell_loop(ctx, deg, n, sides, bt)
         ctx.assemble(J=True, R=True, matrix_free=True, fp32=fp32)
         assert np.abs(ctx.rhs() - r).max() <= 1e-12 * np.abs(r).max()
         assert np.abs(ctx.apply_jacobian(x) - y).max() <= tol * np.abs(y).max()
+
+
+# cells of a colour below and above the counts at which its pairs go to
+# several workgroups
+ASM_CASES = [(1, (3, 2, 2)), (1, (20, 18, 16)), (2, (2, 2, 1)), (2, (9, 9, 9)), (2, (18, 16, 29))]
+
+
+@pytest.mark.parametrize("deg,n", ASM_CASES, ids=["q%d_%dx%dx%d" % (c[0], *c[1]) for c in ASM_CASES])
+def test_assembled_product_matches_the_oracle_cell_loop(ctx, deg, n):
+    p, t, bt = 24.0, 0.75, 2.0
+    hi = np.array([1.3, 1.1, 0.9]) * deg * np.array(n) / 2
+    mesh = G.Mesh(deg, n, -hi, hi, WALLS)
+    print("cells", mesh.n_cells, flush=True)
+    ctx.set_material_pt(p, t, bt=bt)
+    ctx.upload_mesh(mesh)
+    ctx.set_solution(initial_state(mesh.n_nodes, p, t, 0.05, 1))
+    U = ctx.solution()
+    x = np.random.default_rng(3).standard_normal(U.size)
+    _, (y,) = O.cells_apply(deg, mesh.arrays(), mesh.n_nodes, O.coef(p, t, bt=bt), U, X=[x], rhs=False)
+    for fp32, tol in ((False, 1e-12), (True, 2e-6)):
+        ctx.assemble(J=True, R=False, fp32=fp32)
+        assert np.abs(ctx.apply_jacobian(x) - y).max() <= tol * np.abs(y).max()

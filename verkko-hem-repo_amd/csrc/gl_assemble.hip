@@ -17,14 +17,10 @@
 // factorises the same way.  H is evaluated in closed form from six 3x3 Gram
 // matrices per quadrature point.
 //
-// One workgroup (3 wavefronts) owns one cell.  Thread t < 171 owns one
-// unique (c <= d) component pair, keeps H_cd(q) for all q in registers and
-// contracts it against the (a <= b) node-pair weights, which the workgroup
-// stages in LDS 32 pairs at a time (the whole table, 82 KB for Q2, does not
-// fit the scalar cache).  It writes entries [c][d] and [d][c] of block (a,b)
-// and of its transpose (b,a) straight to the BSR values, one node pair after
-// another, with the old values of the next two pairs already requested; the
-// block codes and node masks of the cell sit in LDS as well.
+// A workgroup owns one cell of a colour, or a part of its node pairs.  Q2
+// (k_assemble_q2) contracts the pair weights with H on the FP64 matrix cores,
+// Q1 (k_assemble_q1) in registers; both write whole blocks, 16 bytes (FP64)
+// per lane and consecutive lanes at consecutive entries.
 // Cells of one colour share no node, so the read-modify-write scatter needs
 // no atomics and the result is bit-deterministic; the first colour to touch
 // a block stores instead of accumulating, so J needs no zero fill.
@@ -33,6 +29,7 @@
 // deal.II's AffineConstraints::distribute_local_to_global).
 #include "glhip_dev.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace glh {
@@ -113,192 +110,391 @@ template <typename T> struct Vec2;
 template <> struct Vec2<double> { using type = double2; };
 template <> struct Vec2<float> { using type = float2; };
 
-template <int DEG, typename TJ, bool HANG = false>
-__global__ __launch_bounds__(NT) void k_assemble(RefTables T, MeshDev Mh, Material M0, const double *__restrict__ U,
-                                                 const int *__restrict__ cells, TJ *__restrict__ J)
+// Sizes of the cell contraction of Q2 assembly as a matrix product
+//   OUT[p][col] = sum_k A[p][k] B[k][col]
+// over node pairs p = (a <= b) and block entries col: the 171 entries c <= d,
+// then the 18 entries [d][c] of the same part and spin (the only others that
+// differ from their transposes); k: the NQ points (A = w N_a N_b, B = vol H_cd),
+// the 9 derivative pairs (A = stiffness integrals, B = K1 and K23 factors) and
+// the 6 faces (A = face masses, B = Robin factors; only cells that have one
+// run those steps).  A is uniform over the cells, a table in the lane order of
+// v_mfma_f64_16x16x4_f64 (RefTables::At).
+struct AsmQ2 {
+  static constexpr int NS = 27, NQ = NS, NPAIR = NS * (NS + 1) / 2;
+  static constexpr int NTILE = (NPAIR + 15) / 16;               // row tiles of 16 pairs
+  static constexpr int KB = (NQ + 9 + 3) / 4, KT = (NQ + 15 + 3) / 4;  // k steps of 4, without and with faces
+  static constexpr int TS = 208;                                // LDS row stride of an output tile (192 columns)
+  static constexpr int NW = 6, NTH = 64 * NW;                   // waves (2 column tiles each), threads
+  // phase 0: U, X, Gram and half of B; then two output tiles
+  static constexpr int P0 = NS * 18 + NQ * 18 + NQ * GRAM + 4 * KT * 96, LT = 2 * 16 * TS;
+  static constexpr int LDS = P0 > LT ? P0 : LT;
+};
+
+// column of block entry [r][c] in OUT
+__device__ inline int asm_col(int r, int c)
 {
-  constexpr int N1 = DEG + 1, NS = N1 * N1 * N1, NQ = NS, NPAIR = NS * (NS + 1) / 2;
-  __shared__ double sU[NS * 18];
-  __shared__ double sX[NQ * 18];
-  __shared__ double sGram[NQ * GRAM];
-  // per-cell scatter data staged once: block codes and node constraint masks
-  __shared__ int sBlk[NS * NS];
-  // node-pair weights of the current chunk of pairs (the whole table does not
-  // fit the scalar cache)
-  constexpr int PCH = 32;
-  __shared__ double sWp[PCH * NQ];
-  __shared__ double sSp[PCH * 9];
-  __shared__ uint32_t sMask[NS];
-
-  const int tid = threadIdx.x;
-  const int e = cells[blockIdx.x];
-  if (Mh.inst_active && !Mh.inst_active[Mh.cell_inst[e]]) return;  // finished instance of a batch
-  const Material M = Mh.mats ? Mh.mats[Mh.cell_mat[e]] : M0;  // per-instance (T, p) in a batch
-  const int *cn = Mh.cell_nodes + (size_t)e * NS;
-  double h[3], ih[3];
-  for (int k = 0; k < 3; ++k) { h[k] = Mh.cell_h[3 * e + k]; ih[k] = 1.0 / h[k]; }
-  const double vol = h[0] * h[1] * h[2];
-  const uint32_t cface = Mh.cell_face[e];
-
-  // gather the cell's 18 components at its NS nodes
-  for (int i = tid; i < NS * 18; i += NT) sU[i] = U[(size_t)cn[i / 18] * 18 + (i % 18)];
-  {
-    const int *cb = Mh.cell_blk + (size_t)e * NS * NS;
-    for (int i = tid; i < NS * NS; i += NT) sBlk[i] = cb[i];
-    for (int i = tid; i < NS; i += NT) sMask[i] = Mh.node_mask[cn[i]];
+  if (r > c) {
+    if (r / 3 == c / 3) return 171 + (r / 3) * 3 + (r % 3 == 1 ? 0 : 1 + c % 3);
+    const int t = r;
+    r = c;
+    c = t;
   }
+  return r * 18 - r * (r - 1) / 2 + (c - r);
+}
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// The B operands of the cell: lane l of wave w gets B[4 s + l / 16][16 (w + 6 t)
+// + l % 16] in Br[t][s].  S: AsmQ2::LDS doubles.
+__device__ inline void asm_operands(const RefTables &T, const Material &M, const double *__restrict__ U,
+                                    const int *__restrict__ cn, const double *h, uint32_t cface, bool rb, double *S,
+                                    double (*Br)[AsmQ2::KT])
+{
+  using D = AsmQ2;
+  constexpr int NS = D::NS, NQ = D::NQ;
+  double *sU = S, *sX = sU + NS * 18, *sGram = sX + NQ * 18, *sB = sGram + NQ * GRAM;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const double ih[3] = {1.0 / h[0], 1.0 / h[1], 1.0 / h[2]}, vol = h[0] * h[1] * h[2];
+  for (int i = tid; i < NS * 18; i += D::NTH) sU[i] = U[(size_t)cn[i / 18] * 18 + (i % 18)];
   __syncthreads();
   // the iterate at the quadrature points (s_vector2matrix.cc:116-217)
-  for (int i = tid; i < NQ * 18; i += NT) {
+  for (int i = tid; i < NQ * 18; i += D::NTH) {
     const int q = i / 18, c = i % 18;
     double xv = 0;
     for (int a = 0; a < NS; ++a) xv += T.N[q * NS + a] * sU[a * 18 + c];
     sX[i] = xv;
   }
   __syncthreads();
-  for (int i = tid; i < NQ * GRAM; i += NT) {
+#pragma unroll 1
+  for (int i = tid; i < NQ * GRAM; i += D::NTH) {
+    const int q = i / GRAM, g = i % GRAM;
+    sGram[i] = gram_entry(sX + q * 18, g);
+  }
+  const int nk = 4 * (rb ? D::KT : D::KB);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    // the entry [r][c] of this thread's column (192 columns, 189 used)
+    const int lc = tid % 96, col = 96 * t + lc;
+    int r = 0, c = 0;
+    const bool used = col < 189;
+    if (col < 171) {
+      int k = col;
+      while (k >= 18 - r) { k -= 18 - r; ++r; }
+      c = r + k;
+    } else if (used) {
+      const int g = (col - 171) / 3, k = (col - 171) % 3;
+      r = 3 * g + (k == 0 ? 1 : 2);
+      c = 3 * g + (k == 2 ? 1 : 0);
+    }
+    const bool grad = r / 3 == c / 3;
+    __syncthreads();  // Gram, or the first half of B has been read
+#pragma unroll 1
+    for (int k = tid / 96; k < nk; k += D::NTH / 96) {
+      double v = 0.0;
+      if (used && k < NQ) {
+        v = vol * hess_entry(sGram + k * GRAM, sX + k * 18, r < c ? r : c, r < c ? c : r, M);
+      } else if (used && k < NQ + 9) {
+        const int kk = (k - NQ) / 3, kl = (k - NQ) % 3;
+        if (r == c && kk == kl) v += M.K1 * (vol * ih[kk] * ih[kk]);
+        if (grad && r % 3 == kk && c % 3 == kl) v += M.K23 * vol * ih[kk] * ih[kl];
+      } else if (rb && used && r == c && k < NQ + 15) {
+        const int lf = k - NQ - 9, bid = (int)((cface >> (3 * lf)) & 7u) - 1;
+        if (bid >= 2 && bid <= 4 && !face_zeroed(bid, c)) v = M.robin * face_area(lf, h);
+      }
+      sB[k * 96 + lc] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < D::KT; ++s)
+      Br[t][s] = 4 * s < nk ? sB[(4 * s + (lane >> 4)) * 96 + 16 * w + (lane & 15)] : 0.0;
+  }
+}
+
+// One workgroup of 6 waves per cell of a colour (and per part blockIdx.y of
+// its row tiles, where a colour has too few cells to fill the device).  The
+// contraction of the bulk Hessian, the gradient terms and the Robin masses is
+// one product on the FP64 matrix cores per 16 node pairs, whose result goes
+// to LDS.  From there waves 0-2 write the pairs' blocks (a, b) and waves 3-5
+// the transposed (b, a), 16 bytes per lane: a thread keeps its two entries
+// of a block through all of them, so that the block's address and masks are
+// scalar and its LDS offset constant (about 10 vector instructions a block,
+// against 60 with the blocks' entries dealt over all threads).  The old
+// values of blocks shared with earlier colours are requested before the
+// product; one barrier per 16 pairs.  Jacobian of the 32^3 cube (82 GB moved,
+// 44 GB of it the result: blocks shared between colours are read and written
+// again): 34.4 -> 21.3 ms FP64 (3.9 TB/s), 28.0 -> 22.8 ms FP32, against one
+// thread per component pair storing single values.
+template <typename TJ, bool HANG>
+__global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, MeshDev Mh, Material M0,
+                                                     const double *__restrict__ U, const int *__restrict__ cells,
+                                                     TJ *__restrict__ J)
+{
+  using D = AsmQ2;
+  using J2 = typename Vec2<TJ>::type;
+  constexpr int NS = D::NS, NPAIR = D::NPAIR, KB = D::KB, KT = D::KT, TS = D::TS;
+  __shared__ __attribute__((aligned(16))) double S[D::LDS];
+  __shared__ int sBlk[NS * NS];
+  __shared__ uint32_t sMask[NS];
+  __shared__ uint16_t sPab[D::NTILE * 16];  // a | b << 8 of a pair, ~0 beyond the last
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int e = cells[blockIdx.x];
+  if (Mh.inst_active && !Mh.inst_active[Mh.cell_inst[e]]) return;  // finished instance of a batch
+  const Material M = Mh.mats ? Mh.mats[Mh.cell_mat[e]] : M0;       // per-instance (T, p) in a batch
+  const int *cn = Mh.cell_nodes + (size_t)e * NS;
+  double h[3];
+  for (int k = 0; k < 3; ++k) h[k] = Mh.cell_h[3 * e + k];
+  const uint32_t cface = Mh.cell_face[e];
+  const bool rb = M.robin != 0.0 && cface != 0u;
+  {
+    const int *cb = Mh.cell_blk + (size_t)e * NS * NS;
+    for (int i = tid; i < NS * NS; i += D::NTH) sBlk[i] = cb[i];
+    for (int i = tid; i < NS; i += D::NTH) sMask[i] = Mh.node_mask[cn[i]];
+    for (int i = tid; i < D::NTILE * 16; i += D::NTH)
+      sPab[i] = i < NPAIR ? (uint16_t)(T.pa[i] | (T.pb[i] << 8)) : (uint16_t)0xffff;
+  }
+  double B[2][KT];
+  asm_operands(T, M, U, cn, h, cface, rb, S, B);
+  __syncthreads();  // B has been read: S takes the output tiles
+  // this thread's entries [r][c], [r][c + 1] of a block, and their columns
+  // in OUT: of (a, b), or transposed of (b, a)
+  const bool tr = w >= 3;
+  const int pos = 64 * (tr ? w - 3 : w) + lane;
+  const bool own = pos < 162;
+  const int r = own ? pos / 9 : 0, c = own ? 2 * (pos % 9) : 0;
+  const int o0 = tr ? asm_col(c, r) : asm_col(r, c), o1 = tr ? asm_col(c + 1, r) : asm_col(r, c + 1);
+  const int t0 = D::NTILE * blockIdx.y / gridDim.y, t1 = D::NTILE * (blockIdx.y + 1) / gridDim.y;
+  double A[KT];
+  auto load_a = [&](int t) {
+#pragma unroll
+    for (int s = 0; s < KT; ++s) A[s] = (s < KB || rb) ? T.At[((size_t)t * KT + s) * 64 + lane] : 0.0;
+  };
+  load_a(t0);
+  for (int t = t0; t < t1; ++t) {
+    // lane p < 16: block code of pair 16 t + p for this wave's orientation
+    // (no block: INT_MAX), its row and column masks, and whether a == b
+    int code = 0x7fffffff, mr = 0, mc = 0, dg = -1;
+    if (lane < 16) {
+      const int ab = sPab[16 * t + lane], a = ab & 255, b = ab >> 8;
+      if (ab != 0xffff && !(tr && a == b)) {
+        code = tr ? sBlk[b * NS + a] : sBlk[a * NS + b];
+        mr = (int)sMask[tr ? b : a];
+        mc = (int)sMask[tr ? a : b];
+        dg = a == b ? a : -1;
+      }
+    }
+    J2 old[16];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      const int cd = __builtin_amdgcn_readlane(code, p);
+      old[p] = J2{0, 0};
+      if (cd >= 0 && cd != 0x7fffffff && own) old[p] = reinterpret_cast<const J2 *>(J + (size_t)cd * 324)[pos];
+    }
+    f64x4 acc[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) acc[k] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < KB; ++s)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[s], B[k][s], acc[k], 0, 0, 0);
+    if (rb)
+#pragma unroll
+      for (int s = KB; s < KT; ++s)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[s], B[k][s], acc[k], 0, 0, 0);
+    if (t + 1 < t1) load_a(t + 1);
+    double *O = S + (t & 1) * 16 * TS;
+    // D layout: lane l holds rows 4 q + l / 16, column l % 16
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) O[(4 * q + (lane >> 4)) * TS + 16 * (w + 6 * k) + (lane & 15)] = acc[k][q];
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      const int cd = __builtin_amdgcn_readlane(code, p);
+      if (cd == 0x7fffffff) continue;
+      const uint32_t ur = (uint32_t)__builtin_amdgcn_readlane(mr, p), uc = (uint32_t)__builtin_amdgcn_readlane(mc, p);
+      double v0 = O[p * TS + o0], v1 = O[p * TS + o1];
+      if (ur | uc) {
+        const int na = __builtin_amdgcn_readlane(dg, p);  // the node of a diagonal block
+        // hanging nodes (adaptive meshes): the condensed row keeps the sum
+        // over cells of |local diagonal|
+        if (HANG && na >= 0 && (ur & HANG_BIT) && own && (c == r || c + 1 == r))
+          Mh.hdiag[(size_t)cn[na] * 18 + r] += fabs(c == r ? v0 : v1);
+        const bool rm = (ur >> r) & 1u;
+        if (rm || ((uc >> c) & 1u)) v0 = (na >= 0 && rm && c == r) ? fabs(v0) : 0.0;
+        if (rm || ((uc >> (c + 1)) & 1u)) v1 = (na >= 0 && rm && c + 1 == r) ? fabs(v1) : 0.0;
+      }
+      const int blk = cd < 0 ? -cd - 1 : cd;
+      if (own)
+        reinterpret_cast<J2 *>(J + (size_t)blk * 324)[pos] = J2{(TJ)((double)old[p].x + v0), (TJ)((double)old[p].y + v1)};
+    }
+  }
+}
+
+// The same for Q1 (8 points, 36 node pairs): one workgroup of 3 waves per
+// cell and part of its pairs.  A thread owns entries [r][c], [r][c + 1] of
+// every block, keeps their Hessian at the 8 points in registers and contracts
+// it with the uniform node-pair weights; the block (a, b) and the transposed
+// (b, a) take the same sums (the K2 + K3 term aside), so nothing goes through
+// LDS after the Gram matrices, and a dozen cells run on a CU.  The block
+// codes and masks of the cell sit in lanes, the old values of the next pairs
+// are on their way.  48^3 cells: 11.3 -> 7.7 ms FP64, 9.5 -> 4.4 ms FP32;
+// 8^3 cells (64 a colour): 0.37 -> 0.12 ms.
+template <typename TJ, bool HANG>
+__global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemble_q1(RefTables T, MeshDev Mh, Material M0,
+                                                        const double *__restrict__ U, const int *__restrict__ cells,
+                                                        TJ *__restrict__ J)
+{
+  using J2 = typename Vec2<TJ>::type;
+  constexpr int NS = 8, NQ = 8, NPAIR = 36;
+  __shared__ double sU[NS * 18], sX[NQ * 18], sGram[NQ * GRAM], sSp[NPAIR * 9], sH[NQ * NUPAIR];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int e = cells[blockIdx.x];
+  if (Mh.inst_active && !Mh.inst_active[Mh.cell_inst[e]]) return;  // finished instance of a batch
+  const Material M = Mh.mats ? Mh.mats[Mh.cell_mat[e]] : M0;       // per-instance (T, p) in a batch
+  const int *cn = Mh.cell_nodes + (size_t)e * NS;
+  double h[3], ih[3];
+  for (int k = 0; k < 3; ++k) { h[k] = Mh.cell_h[3 * e + k]; ih[k] = 1.0 / h[k]; }
+  const double vol = h[0] * h[1] * h[2];
+  const uint32_t cface = Mh.cell_face[e];
+  const bool rb = M.robin != 0.0 && cface != 0u;
+  // lane l: the code of block (l / 8, l % 8), the mask of node l % 8
+  const int codes = Mh.cell_blk[(size_t)e * NS * NS + lane];
+  const int masks = (int)Mh.node_mask[cn[lane & 7]];
+  if (tid < NS * 18) sU[tid] = U[(size_t)cn[tid / 18] * 18 + (tid % 18)];
+  for (int i = tid; i < NPAIR * 9; i += 192) sSp[i] = T.Sp[i];
+  __syncthreads();
+  if (tid < NQ * 18) {  // the iterate at the quadrature points (s_vector2matrix.cc:116-217)
+    const int q = tid / 18, c = tid % 18;
+    double xv = 0;
+#pragma unroll
+    for (int a = 0; a < NS; ++a) xv += T.N[q * NS + a] * sU[a * 18 + c];
+    sX[tid] = xv;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int i = tid; i < NQ * GRAM; i += 192) {
     const int q = i / GRAM, g = i % GRAM;
     sGram[i] = gram_entry(sX + q * 18, g);
   }
   __syncthreads();
-
-  {
-    // Thread t < 171 owns the unique component pair (c <= d).  For every node
-    // pair (a <= b) it forms block(a,b)[c][d], block(a,b)[d][c] and writes them,
-    // with the transposed block(b,a), straight to the BSR values (no staging
-    // of the output, so each wavefront keeps many stores in flight; L2 merges
-    // the lanes' 8-byte stores into lines).  All 192 threads load each chunk
-    // of node-pair weights into LDS between two barriers.
-    const bool owner = tid < NUPAIR;
-    int c = 0, d = 0;
-    {
-      int t = owner ? tid : 0;
-      while (t >= 18 - c) { t -= 18 - c; ++c; }
-      d = c + t;
-    }
-    double Hq[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) Hq[q] = hess_entry(sGram + q * GRAM, sX + q * 18, c, d, M);
-    const bool grad_cd = (c / 9 == d / 9) && ((c % 9) / 3 == (d % 9) / 3);
-    const int kc = c % 3, kd = d % 3;
-    const double lap0 = vol * ih[0] * ih[0], lap1 = vol * ih[1] * ih[1], lap2 = vol * ih[2] * ih[2];
-    const double k23_cd = M.K23 * vol * ih[kc] * ih[kd];
-    const uint32_t *mask = Mh.node_mask;
-    const int *cblk = sBlk;
-    const int o_cd = c * 18 + d, o_dc = d * 18 + c;
-    // Robin diagonal weight of this component on each local face (0 if off)
-    double rob[6];
-#pragma unroll
-    for (int lf = 0; lf < 6; ++lf) {
-      const int bid = (int)((cface >> (3 * lf)) & 7u) - 1;
-      rob[lf] = (c == d && M.robin != 0.0 && bid >= 2 && bid <= 4 && !face_zeroed(bid, c))
-                    ? M.robin * face_area(lf, h) : 0.0;
-    }
-    // Old values of blocks shared with earlier colours are loaded one node pair
-    // ahead, so their latency overlaps the contraction of the current pair.
-    auto blk_ptr = [&](int code) -> TJ * { return J + (size_t)(code < 0 ? -code - 1 : code) * 324; };
-    auto prefetch = [&](int p, double *o) {
-      const int a = T.pa[p], b = T.pb[p];
-      const int cab = cblk[a * NS + b];
-      o[0] = o[1] = o[2] = o[3] = 0.0;
-      if (cab >= 0) {
-        const TJ *B = J + (size_t)cab * 324;
-        o[0] = (double)B[o_cd];
-        if (c != d) o[1] = (double)B[o_dc];
-      }
-      if (a != b) {
-        const int cba = cblk[b * NS + a];
-        if (cba >= 0) {
-          const TJ *B = J + (size_t)cba * 324;
-          o[2] = (double)B[o_dc];
-          if (c != d) o[3] = (double)B[o_cd];
-        }
-      }
-    };
-    // entries [c][d] (e1) and [d][c] (e2) of the local block of node pair p
-    auto pair_values = [&](int p, const double *wp, const double *sp, double &e1, double &e2) {
-      double sym = 0.0;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) sym += wp[q] * Hq[q];
-      sym *= vol;
-      const int a = T.pa[p], b = T.pb[p];
-      if (c == d) {
-        sym += M.K1 * (sp[0] * lap0 + sp[4] * lap1 + sp[8] * lap2);
-#pragma unroll
-        for (int lf = 0; lf < 6; ++lf)
-          if (rob[lf] != 0.0) sym += rob[lf] * T.Mf[(lf * NS + a) * NS + b];
-      }
-      e1 = sym;
-      e2 = sym;
-      if (grad_cd) {
-        e1 += k23_cd * sp[kc * 3 + kd];
-        e2 += k23_cd * sp[kd * 3 + kc];
-      }
-    };
-    auto process = [&](int p, const double *ol) {
-      double e1, e2;
-      pair_values(p, sWp + (p % PCH) * NQ, sSp + (p % PCH) * 9, e1, e2);
-      const int a = T.pa[p], b = T.pb[p];
-      const uint32_t ma = sMask[a], mb = sMask[b];
-      {  // block (a,b): rows of node a, columns of node b
-        TJ *B = blk_ptr(cblk[a * NS + b]);
-        double v1 = e1, v2 = e2;
-        const bool r1 = (ma >> c) & 1u, c1 = (mb >> d) & 1u, r2 = (ma >> d) & 1u, c2 = (mb >> c) & 1u;
-        if (r1 || c1) v1 = (a == b && r1 && c == d) ? fabs(v1) : 0.0;
-        if (r2 || c2) v2 = (a == b && r2 && c == d) ? fabs(v2) : 0.0;
-        B[o_cd] = (TJ)(ol[0] + v1);
-        if (c != d) B[o_dc] = (TJ)(ol[1] + v2);
-      }
-      if (a != b) {  // block (b,a) = block(a,b)^T: [d][c] = e1, [c][d] = e2
-        TJ *B = blk_ptr(cblk[b * NS + a]);
-        double v1 = e1, v2 = e2;
-        const bool r1 = (mb >> d) & 1u, c1 = (ma >> c) & 1u, r2 = (mb >> c) & 1u, c2 = (ma >> d) & 1u;
-        if (r1 || c1) v1 = 0.0;
-        if (r2 || c2) v2 = 0.0;
-        B[o_dc] = (TJ)(ol[2] + v1);
-        if (c != d) B[o_cd] = (TJ)(ol[3] + v2);
-      }
-    };
-    // PD node pairs in flight: the old values of pair p + PD are requested
-    // before pair p is contracted and stored (PD = 2 measured fastest with
-    // the block codes and masks in LDS; the registers stay at 3 waves/SIMD)
-    constexpr int PD = 2;
-    double ob[PD][4];
-    if (owner) {
-#pragma unroll
-      for (int k = 0; k < PD; ++k) prefetch(k < NPAIR ? k : NPAIR - 1, ob[k]);
-    }
-    for (int c0 = 0; c0 < NPAIR; c0 += PCH) {
-      const int np = NPAIR - c0 < PCH ? NPAIR - c0 : PCH;
-      __syncthreads();  // the previous chunk has been used
-      for (int i = tid; i < np * NQ; i += NT) sWp[i] = T.Wp[(size_t)c0 * NQ + i];
-      for (int i = tid; i < np * 9; i += NT) sSp[i] = T.Sp[(size_t)c0 * 9 + i];
-      __syncthreads();
-      if (!owner) continue;
-      for (int p0 = c0; p0 < c0 + np; p0 += PD) {
-#pragma unroll
-        for (int k = 0; k < PD; ++k) {
-          const int p = p0 + k;
-          if (p < c0 + np) {
-            double ol[4] = {ob[k][0], ob[k][1], ob[k][2], ob[k][3]};
-            if (p + PD < NPAIR) prefetch(p + PD, ob[k]);
-            process(p, ol);
-          }
-        }
-      }
-    }
-    if (!owner) return;
-    // hanging nodes (adaptive meshes only): the condensed row keeps the sum
-    // over cells of |local diagonal|, gathered outside the hot loop
-    if (HANG && c == d)
-      for (int p = 0; p < NPAIR; ++p) {
-        const int a = T.pa[p];
-        if (a != T.pb[p] || !(mask[cn[a]] & HANG_BIT)) continue;
-        double e1, e2;
-        pair_values(p, T.Wp + p * NQ, T.Sp + p * 9, e1, e2);
-        Mh.hdiag[(size_t)cn[a] * 18 + c] += fabs(e1);
-      }
+  // lanes beyond 162 repeat the last thread's work and store nothing (all
+  // lanes stay active: the codes and masks are read across them)
+  const bool own = tid < 162;
+  const int pos = own ? tid : 161, r = pos / 9, c0 = 2 * (pos % 9);
+  if (tid < NUPAIR) {  // H_cd, c <= d, once per cell
+    int c = 0, t = tid;
+    while (t >= 18 - c) { t -= 18 - c; ++c; }
+#pragma unroll 2
+    for (int q = 0; q < NQ; ++q)
+      sH[q * NUPAIR + tid] = vol * hess_entry(sGram + q * GRAM, sX + q * 18, c, c + t, M);
   }
+  __syncthreads();
+  double H[2][NQ];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = c0 + k, lo = r < c ? r : c, hi = r < c ? c : r, i = lo * 18 - lo * (lo - 1) / 2 + hi - lo;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) H[k][q] = sH[q * NUPAIR + i];
+  }
+  const double lap0 = M.K1 * vol * ih[0] * ih[0], lap1 = M.K1 * vol * ih[1] * ih[1], lap2 = M.K1 * vol * ih[2] * ih[2];
+  // K2 + K3 of [r][c] (the same part and spin) and where its integrals are:
+  // of (a, b) and transposed of (b, a)
+  double k23[2];
+  int ks[2], kt[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = c0 + k;
+    k23[k] = r / 3 == c / 3 ? M.K23 * vol * ih[r % 3] * ih[c % 3] : 0.0;
+    ks[k] = 3 * (r % 3) + c % 3;
+    kt[k] = 3 * (c % 3) + r % 3;
+  }
+  const bool d0 = c0 == r, d1 = c0 + 1 == r;
+  constexpr int PD = 4;  // pairs whose old values are on their way
+  J2 old[PD][2];
+  const int p0 = NPAIR * blockIdx.y / gridDim.y, p1 = NPAIR * (blockIdx.y + 1) / gridDim.y;
+  // pair p = (a, b), stepped in the order of the tables (uniform)
+  struct Pair {
+    int a, b;
+    __device__ inline Pair(int p) : a(0)
+    {
+      while (p >= NS - a) { p -= NS - a; ++a; }
+      b = a + p;
+    }
+    __device__ inline void next()
+    {
+      if (++b == NS) b = ++a;
+    }
+  };
+  auto load_old = [&](const Pair &P, J2 *o) {
+    const int cab = __builtin_amdgcn_readlane(codes, P.a * NS + P.b),
+              cba = __builtin_amdgcn_readlane(codes, P.b * NS + P.a);
+    o[0] = o[1] = J2{0, 0};
+    if (cab >= 0) o[0] = reinterpret_cast<const J2 *>(J + (size_t)cab * 324)[pos];
+    if (P.a != P.b && cba >= 0) o[1] = reinterpret_cast<const J2 *>(J + (size_t)cba * 324)[pos];
+  };
+  auto store = [&](int code, const J2 &o, double v0, double v1) {
+    const int blk = code < 0 ? -code - 1 : code;
+    const J2 v = {(TJ)((double)o.x + v0), (TJ)((double)o.y + v1)};
+    if (own) reinterpret_cast<J2 *>(J + (size_t)blk * 324)[pos] = v;
+  };
+  Pair P(p0), F(p0);
+#pragma unroll
+  for (int k = 0; k < PD; ++k)
+    if (p0 + k < p1) {
+      load_old(F, old[k]);
+      F.next();
+    }
+  // (rolled: 36 unrolled pairs are 40 KB of code, fetched once per wave)
+#pragma unroll 1
+  for (int pb = p0; pb < p1; pb += PD)
+#pragma unroll
+    for (int k = 0; k < PD; ++k) {
+      const int p = pb + k;
+      if (p >= p1) break;
+      const int a = P.a, b = P.b;
+      P.next();
+      const J2 o0 = old[k][0], o1 = old[k][1];
+      if (p + PD < p1) {
+        load_old(F, old[k]);
+        F.next();
+      }
+      double v0 = 0.0, v1 = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const double wq = T.Wp[p * NQ + q];
+        v0 += wq * H[0][q];
+        v1 += wq * H[1][q];
+      }
+      double lap = T.Sp[p * 9] * lap0 + T.Sp[p * 9 + 4] * lap1 + T.Sp[p * 9 + 8] * lap2;
+      if (rb)
+        for (int lf = 0; lf < 6; ++lf) {
+          const int bid = (int)((cface >> (3 * lf)) & 7u) - 1;
+          if (bid >= 2 && bid <= 4 && !face_zeroed(bid, r))
+            lap += M.robin * face_area(lf, h) * T.Mf[(lf * NS + a) * NS + b];
+        }
+      v0 += d0 ? lap : 0.0;
+      v1 += d1 ? lap : 0.0;
+      double t0 = v0 + k23[0] * sSp[p * 9 + kt[0]], t1 = v1 + k23[1] * sSp[p * 9 + kt[1]];  // of (b, a)
+      v0 += k23[0] * sSp[p * 9 + ks[0]];
+      v1 += k23[1] * sSp[p * 9 + ks[1]];
+      const uint32_t ma = (uint32_t)__builtin_amdgcn_readlane(masks, a),
+                     mb = (uint32_t)__builtin_amdgcn_readlane(masks, b);
+      if (ma | mb) {
+        // hanging nodes (adaptive meshes): the condensed row keeps the sum
+        // over cells of |local diagonal|
+        if (HANG && a == b && (ma & HANG_BIT) && own && (d0 || d1))
+          Mh.hdiag[(size_t)cn[a] * 18 + r] += fabs(d0 ? v0 : v1);
+        const bool ra = (ma >> r) & 1u, rbm = (mb >> r) & 1u;  // row r of node a, of node b
+        if (ra || ((mb >> c0) & 1u)) v0 = (a == b && ra && d0) ? fabs(v0) : 0.0;
+        if (ra || ((mb >> (c0 + 1)) & 1u)) v1 = (a == b && ra && d1) ? fabs(v1) : 0.0;
+        if (rbm || ((ma >> c0) & 1u)) t0 = 0.0;
+        if (rbm || ((ma >> (c0 + 1)) & 1u)) t1 = 0.0;
+      }
+      store(__builtin_amdgcn_readlane(codes, a * NS + b), o0, v0, v1);
+      if (a != b) store(__builtin_amdgcn_readlane(codes, b * NS + a), o1, t0, t1);
+    }
 }
 
 // ------------------------------------------------ matrix-free Jacobian
@@ -1346,16 +1542,21 @@ hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDe
                            const double *U, const int *cells, int n, void *J, hipStream_t s)
 {
   if (n <= 0) return hipSuccess;
-  dim3 g(n), b(NT);
-#define GLH_ASM(D, TJ, HG) hipLaunchKernelGGL((k_assemble<D, TJ, HG>), g, b, 0, s, T, M, mat, U, cells, (TJ *)J)
+  // a colour of few cells: the pairs of a cell go to several workgroups, which
+  // each form H again (Q2 colours of 287 cells: 253 us in one part, 245 in
+  // three; Q1 of 64: 15.9 us in four parts, 15.5 in six)
+  const int parts = std::max(1, std::min(deg == 1 ? 6 : AsmQ2::NTILE / 3, 1024 / n));
+  const dim3 g(n, parts);
   // the hanging-node variant (adaptive meshes) also gathers the constrained diagonals
   const bool hang = M.hdiag != nullptr;
+#define GLH_ASM(K, TJ, HG, B) hipLaunchKernelGGL((K<TJ, HG>), g, dim3(B), 0, s, T, M, mat, U, cells, (TJ *)J)
   if (deg == 1) {
-    if (hang) { if (jfp32) GLH_ASM(1, float, true); else GLH_ASM(1, double, true); }
-    else { if (jfp32) GLH_ASM(1, float, false); else GLH_ASM(1, double, false); }
+    if (hang) { if (jfp32) GLH_ASM(k_assemble_q1, float, true, 192); else GLH_ASM(k_assemble_q1, double, true, 192); }
+    else { if (jfp32) GLH_ASM(k_assemble_q1, float, false, 192); else GLH_ASM(k_assemble_q1, double, false, 192); }
   } else {
-    if (hang) { if (jfp32) GLH_ASM(2, float, true); else GLH_ASM(2, double, true); }
-    else { if (jfp32) GLH_ASM(2, float, false); else GLH_ASM(2, double, false); }
+    constexpr int B = AsmQ2::NTH;
+    if (hang) { if (jfp32) GLH_ASM(k_assemble_q2, float, true, B); else GLH_ASM(k_assemble_q2, double, true, B); }
+    else { if (jfp32) GLH_ASM(k_assemble_q2, float, false, B); else GLH_ASM(k_assemble_q2, double, false, B); }
   }
 #undef GLH_ASM
   return hipGetLastError();

@@ -109,7 +109,7 @@ struct glh_ctx {
   int n_seg = 1, n_chunks = 0;
   int max_seg_chunks = 0;  // reduction chunks of the largest instance
   // reference tables
-  DBuf<double> tN, tdN, tw, tWp, tSp, tMf;
+  DBuf<double> tN, tdN, tw, tWp, tSp, tMf, tAt;
   DBuf<int> tpa, tpb;
   // mesh arrays
   DBuf<int> cell_nodes, row_ptr, col, diag, cell_blk, color_cells, cell_mat, seg_chunk;
@@ -213,7 +213,7 @@ struct glh_ctx {
 
   glh::RefTables tables() const
   {
-    return glh::RefTables{tN.p, tdN.p, tw.p, tWp.p, tSp.p, tMf.p, tpa.p, tpb.p};
+    return glh::RefTables{tN.p, tdN.p, tw.p, tWp.p, tSp.p, tMf.p, tpa.p, tpb.p, tAt.p};
   }
   glh::MeshDev meshdev() const
   {
@@ -363,6 +363,23 @@ int build_tables(glh_ctx *c, int deg)
   HIPCHK(c, upload(c->tMf, Mf.data(), Mf.size(), s));
   HIPCHK(c, upload(c->tpa, pa.data(), pa.size(), s));
   HIPCHK(c, upload(c->tpb, pb.data(), pb.size(), s));
+  // the pair tables as matrix-core operands: row tile t, k step s, lane l hold
+  // pair 16 t + l % 16 and k = 4 s + l / 16 (points, derivative pairs, faces)
+  // (Q2; the Q1 assembly reads the pair tables themselves)
+  const int nt = deg == 2 ? (npair + 15) / 16 : 0, kt = (nq + 15 + 3) / 4;
+  std::vector<double> At((size_t)nt * kt * 64, 0.0);
+  for (int t = 0; t < nt; ++t)
+    for (int k4 = 0; k4 < kt; ++k4)
+      for (int l = 0; l < 64; ++l) {
+        const int pr = 16 * t + l % 16, k = 4 * k4 + l / 16;
+        if (pr >= npair) continue;
+        double v = 0.0;
+        if (k < nq) v = Wp[(size_t)pr * nq + k];
+        else if (k < nq + 9) v = Sp[(size_t)pr * 9 + k - nq];
+        else if (k < nq + 15) v = Mf[((size_t)(k - nq - 9) * ns + pa[pr]) * ns + pb[pr]];
+        At[((size_t)t * kt + k4) * 64 + l] = v;
+      }
+  HIPCHK(c, upload(c->tAt, At.data(), At.size(), s));
   HIPCHK(c, hipStreamSynchronize(s));
   c->deg = deg; c->ns = ns; c->nq = nq; c->npair = npair;
   return GLH_OK;
@@ -1135,7 +1152,7 @@ int glh_destroy(glh_ctx *c)
   if (!c) return GLH_OK;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  DBuf<double> *dbs[] = {&c->tN,     &c->tdN,  &c->tw,   &c->tWp,  &c->tSp,   &c->tMf,   &c->cell_h,
+  DBuf<double> *dbs[] = {&c->tN,     &c->tdN,  &c->tw,   &c->tWp,  &c->tSp,   &c->tMf,   &c->tAt,   &c->cell_h,
                          &c->U,      &c->U0,   &c->dU,   &c->X,    &c->rhs,   &c->res,   &c->Fcell,
                          &c->s_norm, &c->s_alpha, &c->s_part, &c->J64, &c->D64, &c->gV64, &c->gZ64,
                          &c->gW64,   &c->gh64, &c->gp64, &c->gy64, &c->gs64,  &c->gq64,  &c->ir_r, &c->gn64};

@@ -19,6 +19,7 @@ struct RefTables {
   const double *Sp;   // [NPAIR*9]  sum_q w_q dN_a/dxi_k dN_b/dxi_l, index k*3+l
   const double *Mf;   // [6*NS*NS]  face mass on each unit face
   const int *pa, *pb; // [NPAIR]    pair list (a <= b)
+  const double *At;   // the pairs' tables as MFMA operands (see k_assemble): [row tile][k step][lane]
 };
 
 struct Material {
