@@ -382,10 +382,7 @@ __global__ __launch_bounds__(256) void k_bj_apply(int n_rows, const TJ *__restri
 // -------------------------------------------------------------- reductions
 constexpr int RT = 256;
 constexpr int KCH = 8;  // vectors per multi-dot pass (4 measured the same, 16 slower)
-// pairs of values per thread of the Gram-Schmidt update: a chunk holds at
-// most GS_MAX_CHUNK values
-constexpr int GS_PAIRS = GS_MAX_CHUNK / (2 * RT);
-static_assert(GS_PAIRS * 2 * RT == GS_MAX_CHUNK, "chunk bound in whole pairs per thread");
+static_assert(GS_MAX_CHUNK == 8 * 2 * RT, "8 FP64 loads per thread cover the longest chunk");
 
 // Sum over the 64 lanes of a wave (butterfly: every lane gets the same,
 // order-fixed result).
@@ -610,20 +607,133 @@ __global__ void k_set_scalar(T *p, T v)
 // workgroups).  Per-chunk partials are reduced per instance in fixed order
 // (deterministic).
 
-// Chunk bounds are even (an instance holds 18 values per node and chunks are
-// 1024 values long), so the Gram-Schmidt kernels below read pairs of values:
-// the basis vectors with non-temporal loads (a cycle's basis is far larger
-// than the caches and is streamed), w with ordinary loads (every group of
-// basis vectors reads it again).
-template <typename T>
-__device__ inline typename NV2<T>::type ld2nt(const T *__restrict__ p)
+// The Gram-Schmidt kernels below read 16 bytes per thread (2 values in FP64,
+// 4 in FP32; 8-byte loads left the FP32 passes at 2.2 TB/s).  Chunk bounds are even (an instance holds 18 values per node and
+// chunks are multiples of 1024 values long), so a load is aligned to 8 bytes
+// at least, and an FP32 chunk may end with a pair.
+template <typename T> struct Quad;
+template <> struct Quad<double> {
+  typedef double type __attribute__((ext_vector_type(2)));
+  static constexpr int N = 2;
+};
+template <> struct Quad<float> {
+  typedef float type __attribute__((ext_vector_type(4), aligned(8)));
+  static constexpr int N = 4;
+};
+// the values at i of p, 0 from end on (i and end even); FULL: all are there
+template <bool NTL, bool FULL, typename T>
+__device__ inline typename Quad<T>::type ldc(const T *__restrict__ p, long long i, long long end)
 {
-  return __builtin_nontemporal_load(reinterpret_cast<const typename NV2<T>::type *>(p));
+  using Q = typename Quad<T>::type;
+  if (FULL || i + Quad<T>::N <= end) {
+    if constexpr (NTL) return __builtin_nontemporal_load(reinterpret_cast<const Q *>(p + i));
+    return *reinterpret_cast<const Q *>(p + i);
+  }
+  Q v{};
+  if (Quad<T>::N == 4 && i < end) {
+    const typename NV2<T>::type h = *reinterpret_cast<const typename NV2<T>::type *>(p + i);
+    v[0] = h.x;
+    v[1] = h.y;
+  }
+  return v;
 }
-template <typename T>
-__device__ inline typename NV2<T>::type ld2(const T *__restrict__ p)
+template <bool FULL, typename T>
+__device__ inline void stc(T *p, long long i, long long end, const typename Quad<T>::type &v)
 {
-  return *reinterpret_cast<const typename NV2<T>::type *>(p);
+  if (FULL || i + Quad<T>::N <= end) *reinterpret_cast<typename Quad<T>::type *>(p + i) = v;
+  else if (Quad<T>::N == 4 && i < end)
+    *reinterpret_cast<typename NV2<T>::type *>(p + i) = typename NV2<T>::type{v[0], v[1]};
+}
+// A thread holds NQ such loads of its chunk (NQ * N * RT values cover it), of
+// several basis vectors at a time: up to 16 loads in flight, and the workgroup
+// reads a whole chunk of one vector (32 KB for chunks of 4096 in FP64) before
+// the next.
+constexpr int gs_flight(int tile, int nq) { return tile / nq < 1 ? 1 : tile / nq; }
+
+// Whether k basis vectors are read past the caches (non-temporal loads): when
+// they do not fit the 256 MB memory-side cache, whose contents the passes of
+// one column otherwise share.
+template <typename T>
+__device__ inline bool gs_stream(int k, size_t ldv) { return (size_t)k * ldv * sizeof(T) > ((size_t)256 << 20); }
+
+// acc[j] += V_j . w over the chunk [beg, end) for j < kk; vector `self` is w
+template <bool NTL, bool FULL, typename T, int G, int NQ>
+__device__ inline void mdot_chunk(const T *__restrict__ V, size_t ldv, const T *__restrict__ w, long long beg,
+                                  long long end, int kk, int self, T *acc)
+{
+  constexpr int QN = Quad<T>::N, U = gs_flight(2 * G, NQ) < G ? gs_flight(2 * G, NQ) : G;
+  using Q = typename Quad<T>::type;
+  const long long idx = beg + QN * threadIdx.x;
+  Q x[NQ];
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) x[t] = ldc<false, FULL>(w, idx + t * QN * RT, end);
+#pragma unroll
+  for (int j = 0; j < G; j += U) {
+    if (j >= kk) break;
+    Q v[U][NQ];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (j + u < kk && j + u != self)
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) v[u][t] = ldc<NTL, FULL>(V + (size_t)(j + u) * ldv, idx + t * QN * RT, end);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (j + u < kk) {
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) {
+          const Q y = j + u == self ? x[t] : v[u][t];
+#pragma unroll
+          for (int q = 0; q < QN; ++q) acc[j + u] += y[q] * x[t][q];
+        }
+      }
+  }
+}
+
+// w -= sum_{i < k} hs[i] V_i over the chunk; returns this thread's share of
+// ||w||^2 after it
+template <bool NTL, bool FULL, typename T, int UF, int NQ>
+__device__ inline T update_chunk(const T *__restrict__ V, size_t ldv, const T *hs, int k, T *__restrict__ w,
+                                 long long beg, long long end)
+{
+  constexpr int QN = Quad<T>::N, U = gs_flight(2 * UF, NQ);
+  using Q = typename Quad<T>::type;
+  const long long idx = beg + QN * threadIdx.x;
+  Q out[NQ];
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) out[t] = ldc<false, FULL>(w, idx + t * QN * RT, end);
+  int i = 0;
+  for (; i + U <= k; i += U) {
+    Q v[U][NQ];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) v[u][t] = ldc<NTL, FULL>(V + (size_t)(i + u) * ldv, idx + t * QN * RT, end);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) out[t] -= hs[i + u] * v[u][t];
+  }
+  if (i < k) {  // the last vectors, their loads together
+    Q v[U][NQ];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u < k)
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) v[u][t] = ldc<NTL, FULL>(V + (size_t)(i + u) * ldv, idx + t * QN * RT, end);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u < k)
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) out[t] -= hs[i + u] * v[u][t];
+  }
+  T acc = 0;
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+#pragma unroll
+    for (int q = 0; q < QN; ++q) acc += out[t][q] * out[t][q];
+    stc<FULL>(w, idx + t * QN * RT, end, out[t]);
+  }
+  return acc;
 }
 
 // 2D grid: x = chunks (or the active list), y = groups of G vectors.
@@ -632,7 +742,7 @@ __device__ inline typename NV2<T>::type ld2(const T *__restrict__ p)
 // 8 (r / groups) + x, group r % groups, and every group of a chunk runs on
 // the XCD of that chunk, whose L2 then serves w to all but the first
 // (gridDim.x is a multiple of 8 there).
-template <typename T, int G>
+template <typename T, int G, int NQ>
 __global__ __launch_bounds__(RT) void k_seg_mdot_partial(const long long *__restrict__ ch, int n_chunks,
                                                          ActiveSet act, int k, const T *__restrict__ V, size_t ldv,
                                                          const T *__restrict__ w, T *__restrict__ partial,
@@ -687,16 +797,12 @@ __global__ __launch_bounds__(RT) void k_seg_mdot_partial(const long long *__rest
     T acc[G];
 #pragma unroll
     for (int j = 0; j < G; ++j) acc[j] = 0;
-    for (long long idx = beg + 2 * threadIdx.x; idx < end; idx += 2 * RT) {
-      const auto x = ld2(w + idx);
-#pragma unroll
-      for (int j = 0; j < G; ++j)
-        if (j < kk) {
-          const auto v = ld2nt(V + (size_t)(i0 + j) * ldv + idx);
-          acc[j] += v.x * x.x;
-          acc[j] += v.y * x.y;
-        }
-    }
+    // the vector that is w itself (the norm beside the products) is not read again
+    const int self = w == V + (size_t)(k - 1) * ldv ? k - 1 - i0 : -1;
+    const T *Vg = V + (size_t)i0 * ldv;
+    if (end - beg != NQ * Quad<T>::N * RT) mdot_chunk<false, false, T, G, NQ>(Vg, ldv, w, beg, end, kk, self, acc);
+    else if (gs_stream<T>(k, ldv)) mdot_chunk<true, true, T, G, NQ>(Vg, ldv, w, beg, end, kk, self, acc);
+    else mdot_chunk<false, true, T, G, NQ>(Vg, ldv, w, beg, end, kk, self, acc);
 #pragma unroll
     for (int j = 0; j < G; ++j) {
       const T r = wave_sum(acc[j]);
@@ -735,7 +841,7 @@ __global__ __launch_bounds__(RT) void k_seg_final(const int *__restrict__ seg_ch
   }
 }
 
-template <typename T, int UF>
+template <typename T, int UF, int NQ>
 __global__ __launch_bounds__(RT) void k_seg_sub_lincomb_norm(const long long *__restrict__ ch, int n_chunks,
                                                              ActiveSet act, int k, const T *__restrict__ V,
                                                              size_t ldv, T *h, int ldh, T *__restrict__ w,
@@ -750,7 +856,6 @@ __global__ __launch_bounds__(RT) void k_seg_sub_lincomb_norm(const long long *__
     const int cb = work_chunk(act, wi);
     const long long sg = ch[3 * cb], beg = ch[3 * cb + 1], end = ch[3 * cb + 2];
     if (flag && !flag[sg]) continue;
-    const T *hs = h + sg * ldh;
     if (hpart) {
       // the instance's hk multi-dot values from its chunk partials, in chunk
       // order (every workgroup of the instance forms the same sums); the
@@ -762,47 +867,14 @@ __global__ __launch_bounds__(RT) void k_seg_sub_lincomb_norm(const long long *__
         shh[i] = acc;
         if (cb == c0) h[sg * ldh + i] = acc;
       }
-      __syncthreads();
-      hs = shh;
+    } else {
+      for (int i = threadIdx.x; i < k; i += RT) shh[i] = h[sg * ldh + i];
     }
-    T acc = 0;
-    // the updated pairs are stored once the whole chunk is done: a store
-    // between the loads of the next pair holds them back (loads and stores
-    // share one counter), and the stores then go out in one burst
-    typename NV2<T>::type out[GS_PAIRS];
-#pragma unroll
-    for (int it = 0; it < GS_PAIRS; ++it) {
-      const long long idx = beg + 2 * threadIdx.x + (long long)it * 2 * RT;
-      if (idx >= end) break;
-      const auto w2 = ld2(w + idx);
-      T s0 = w2.x, s1 = w2.y;
-      const T *vp = V + idx;
-      int i = 0;
-      for (; i + UF <= k; i += UF) {  // UF basis vectors in flight
-        typename NV2<T>::type v[UF];
-#pragma unroll
-        for (int u = 0; u < UF; ++u) v[u] = ld2nt(vp + (size_t)(i + u) * ldv);
-#pragma unroll
-        for (int u = 0; u < UF; ++u) {
-          s0 -= hs[i + u] * v[u].x;
-          s1 -= hs[i + u] * v[u].y;
-        }
-      }
-      for (; i < k; ++i) {
-        const auto v = ld2nt(vp + (size_t)i * ldv);
-        s0 -= hs[i] * v.x;
-        s1 -= hs[i] * v.y;
-      }
-      out[it].x = s0;
-      out[it].y = s1;
-      acc += s0 * s0;
-      acc += s1 * s1;
-    }
-#pragma unroll
-    for (int it = 0; it < GS_PAIRS; ++it) {
-      const long long idx = beg + 2 * threadIdx.x + (long long)it * 2 * RT;
-      if (idx < end) *reinterpret_cast<typename NV2<T>::type *>(w + idx) = out[it];
-    }
+    __syncthreads();
+    T acc;
+    if (end - beg != NQ * Quad<T>::N * RT) acc = update_chunk<false, false, T, UF, NQ>(V, ldv, shh, k, w, beg, end);
+    else if (gs_stream<T>(k, ldv)) acc = update_chunk<true, true, T, UF, NQ>(V, ldv, shh, k, w, beg, end);
+    else acc = update_chunk<false, true, T, UF, NQ>(V, ldv, shh, k, w, beg, end);
     const T r = block_reduce(acc, sh);
     if (threadIdx.x == 0) partial[cb] = r;
   }
@@ -1365,21 +1437,35 @@ inline int seg_grid(const SegInfo &S)
   return S.act.counts ? std::max(1, std::min(S.n_seg, ACT_SEG_GRID) >> S.act.shift) : S.n_seg;
 }
 
+// 16-byte loads per thread that cover the longest chunk
+template <typename T>
+inline int gs_quads(const SegInfo &S)
+{
+  const long long per = Quad<T>::N * RT;
+  const int n = (int)((S.len + per - 1) / per);
+  return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : 8;
+}
+
 template <typename T>
 hipError_t launch_seg_mdot(const SegInfo &S, int k, const T *V, size_t ldv, const T *w, T *partial, T *out, int ldo,
                            int off, bool accumulate, hipStream_t s, const int *flag, bool reduce, const Op1In<T> &O)
 {
   if (k <= 0 || S.n_chunks <= 0) return hipSuccess;
+  if (S.len < 2 || S.len > GS_MAX_CHUNK) return hipErrorInvalidValue;
   if (O.npart && (!O.norm2 || O.norm2 != O.C.nrm2 || O.npart == partial || reduce)) return hipErrorInvalidValue;
   int gx = S.act.counts ? chunk_grid(S) : (S.n_chunks + 7) / 8 * 8;  // XCD-numbered: a multiple of 8
   if (!S.act.counts && S.cap > 0 && S.cap < S.n_chunks) gx = S.cap;  // grid-stride over the chunks
-#define GLH_MDOT(G)                                                                                              \
-  hipLaunchKernelGGL((k_seg_mdot_partial<T, G>), dim3(gx, (k + G - 1) / G), dim3(RT), 0, s, S.chunks, S.n_chunks, \
-                     S.act, k, V, ldv, w, partial, flag, O)
-  if (S.gs == 4) GLH_MDOT(4);
-  else if (S.gs == 8) GLH_MDOT(8);
-  else if (S.gs == 16) GLH_MDOT(16);
+  const int nq = gs_quads<T>(S);
+#define GLH_MDOT(G, NQ)                                                                                         \
+  hipLaunchKernelGGL((k_seg_mdot_partial<T, G, NQ>), dim3(gx, (k + G - 1) / G), dim3(RT), 0, s, S.chunks,        \
+                     S.n_chunks, S.act, k, V, ldv, w, partial, flag, O)
+#define GLH_MDOT2(G) \
+  if (nq == 1) GLH_MDOT(G, 1); else if (nq == 2) GLH_MDOT(G, 2); else if (nq == 4) GLH_MDOT(G, 4); else if constexpr (sizeof(T) == 8) GLH_MDOT(G, 8)
+  if (S.gs == 4) { GLH_MDOT2(4); }
+  else if (S.gs == 8) { GLH_MDOT2(8); }
+  else if (S.gs == 16) { GLH_MDOT2(16); }
   else return hipErrorInvalidValue;
+#undef GLH_MDOT2
 #undef GLH_MDOT
   if (!reduce) return hipGetLastError();  // the consumer sums the chunk partials itself
   hipLaunchKernelGGL((k_seg_final<T>), dim3(seg_grid(S), k), dim3(RT), 0, s, S.seg_chunk, S.n_seg, S.act, k, partial,
@@ -1401,14 +1487,19 @@ hipError_t launch_seg_sub_lincomb_norm(const SegInfo &S, int k, const T *V, size
                                        const GmresCtl<T> *ctl, int op, int j, const T *hpart, int hk, bool reduce)
 {
   if (S.n_chunks <= 0) return hipSuccess;
-  if (hpart && (hk < k || hk > 128 || hpart == partial)) return hipErrorInvalidValue;
-#define GLH_SLN(UF)                                                                                              \
-  hipLaunchKernelGGL((k_seg_sub_lincomb_norm<T, UF>), dim3(chunk_grid(S)), dim3(RT), 0, s, S.chunks, S.n_chunks, \
-                     S.act, k, V, ldv, h, ldh, w, partial, flag, S.seg_chunk, hpart, hk)
-  if (S.gs == 4) GLH_SLN(4);
-  else if (S.gs == 8) GLH_SLN(8);
-  else if (S.gs == 16) GLH_SLN(16);
+  if (S.len < 2 || S.len > GS_MAX_CHUNK || (hpart && (hk < k || hk > 128 || hpart == partial)))
+    return hipErrorInvalidValue;
+  const int nq = gs_quads<T>(S);
+#define GLH_SLN(UF, NQ)                                                                                          \
+  hipLaunchKernelGGL((k_seg_sub_lincomb_norm<T, UF, NQ>), dim3(chunk_grid(S)), dim3(RT), 0, s, S.chunks,         \
+                     S.n_chunks, S.act, k, V, ldv, h, ldh, w, partial, flag, S.seg_chunk, hpart, hk)
+#define GLH_SLN2(UF) \
+  if (nq == 1) GLH_SLN(UF, 1); else if (nq == 2) GLH_SLN(UF, 2); else if (nq == 4) GLH_SLN(UF, 4); else if constexpr (sizeof(T) == 8) GLH_SLN(UF, 8)
+  if (S.gs == 4) { GLH_SLN2(4); }
+  else if (S.gs == 8) { GLH_SLN2(8); }
+  else if (S.gs == 16) { GLH_SLN2(16); }
   else return hipErrorInvalidValue;
+#undef GLH_SLN2
 #undef GLH_SLN
   if (!reduce) return hipGetLastError();  // the norm partials go to a later launch
   if (ctl) {

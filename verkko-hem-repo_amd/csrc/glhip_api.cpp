@@ -108,6 +108,7 @@ struct glh_ctx {
   std::vector<int> node_off, cell_off;  // instance ranges
   int n_seg = 1, n_chunks = 0;
   int max_seg_chunks = 0;  // reduction chunks of the largest instance
+  int chunk_len = (int)glh::GS_MAX_CHUNK;  // the longest chunk
   // reference tables
   DBuf<double> tN, tdN, tw, tWp, tSp, tMf, tAt;
   DBuf<int> tpa, tpb;
@@ -226,6 +227,7 @@ struct glh_ctx {
   {
     glh::SegInfo S{chunks.p, seg_chunk.p, n_chunks, n_seg};
     S.gs = gs_tile;
+    S.len = chunk_len;
     return S;
   }
 };
@@ -397,6 +399,8 @@ int check_ready(glh_ctx *c, bool need_mat = true)
 }
 
 size_t ndofs(const glh_ctx *c) { return (size_t)c->n_nodes * NC; }
+// values between two vectors of the Krylov basis: every vector starts at 16 bytes
+size_t basis_stride(const glh_ctx *c) { return (ndofs(c) + 3) / 4 * 4; }
 
 // per-instance ||v_s||^2 of an FP64 device vector into out (host, n_seg values)
 int seg_norm2(glh_ctx *c, const double *v, std::vector<double> &out)
@@ -701,7 +705,7 @@ template <typename TJ, typename TV>
 int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, int m, const glh::GmresCtl<TV> &C,
                   bool timed, int part, int j0 = 0, int j1 = 0, int shift = 0)
 {
-  const size_t n = ndofs(c);
+  const size_t n = ndofs(c), ldv = basis_stride(c);
   const int ldh = m + 2;
   const glh::SegInfo SI = c->seg();
   hipStream_t s = c->stream;
@@ -743,7 +747,7 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
   }
   if (part == 2) {  // tail: x += M^-1 V y
     HIPCHK(c, glh::launch_gmres_ctl<TV>(C, 3, 0, s));
-    HIPCHK(c, glh::launch_seg_lincomb<TV>(SA, m, V.p, n, C.y, ldh, W.p, s, C.jseg));
+    HIPCHK(c, glh::launch_seg_lincomb<TV>(SA, m, V.p, ldv, C.y, ldh, W.p, s, C.jseg));
     HIPCHK(c, (glh::launch_bj_apply<TJ, TV>(c->n_nodes, Dinv, W.p, Z.p, s, rs, nullptr, act)));
     if (use_act) HIPCHK(c, glh::launch_seg_add<TV>(SA, Z.p, x, s));
     else HIPCHK(c, (glh::launch_axpy<TV, TV>(n, 1.0, Z.p, x, s)));
@@ -752,7 +756,7 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
   // body block: Arnoldi steps j0 <= j < j1
   if (j0 == 0) HIPCHK(c, glh::launch_seg_scale<TV>(SA, V.p, nrm2, 1, V.p, s, cyc, true));
   for (int j = j0; j < j1; ++j) {
-    TV *vj = V.p + n * j, *wv = V.p + n * (j + 1);
+    TV *vj = V.p + ldv * j, *wv = V.p + ldv * (j + 1);
     HIPCHK(c, (glh::launch_bj_apply<TJ, TV>(c->n_nodes, Dinv, vj, Z.p, s, rs, cyc, act)));
     RCHK(mv(Z.p, wv, cyc, act));
     // each pass's norm reduction runs the control op of its instance
@@ -761,8 +765,8 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
     // (batches of small instances: each update workgroup sums its instance's
     // multi-dot partials itself, instead of a reduction launch per pass)
     if (fold) {
-      HIPCHK(c, glh::launch_seg_mdot<TV>(SA, j + 2, V.p, n, wv, pt.p, hs, ldh, 0, false, s, cyc, false));
-      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, n, hs, ldh, wv, np, nrm2, 1, 0, s, cyc, nullptr,
+      HIPCHK(c, glh::launch_seg_mdot<TV>(SA, j + 2, V.p, ldv, wv, pt.p, hs, ldh, 0, false, s, cyc, false));
+      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, ldv, hs, ldh, wv, np, nrm2, 1, 0, s, cyc, nullptr,
                                                      0, j, pt.p, j + 2, false));
       // op 1 (the second pass's flag) formed by the second pass's multi-dot
       // workgroups from the first pass's norm partials: no launch of its own
@@ -772,16 +776,16 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
       o1.seg_chunk = SR.seg_chunk;
       o1.C = C;
       o1.j = j;
-      HIPCHK(c, glh::launch_seg_mdot<TV>(SR, j + 1, V.p, n, wv, pt.p, hq, ldh, 0, false, s, ro, false, o1));
-      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, n, hq, ldh, wv, np, nrm2, 1, 0, s, ro, nullptr, 0,
+      HIPCHK(c, glh::launch_seg_mdot<TV>(SR, j + 1, V.p, ldv, wv, pt.p, hq, ldh, 0, false, s, ro, false, o1));
+      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, ldv, hq, ldh, wv, np, nrm2, 1, 0, s, ro, nullptr, 0,
                                                      j, pt.p, j + 1, false));
       // the pass's norm reduction, op 2 and the normalisation in one launch
       HIPCHK(c, glh::launch_seg_ctl2_scale<TV>(SA, np, nrm2, C, j, wv, s));
     } else {
-      HIPCHK(c, glh::launch_seg_mdot<TV>(SA, j + 2, V.p, n, wv, pt.p, hs, ldh, 0, false, s, cyc));
-      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, n, hs, ldh, wv, pt.p, nrm2, 1, 0, s, cyc, &C, 1, j));
-      HIPCHK(c, glh::launch_seg_mdot<TV>(SR, j + 1, V.p, n, wv, pt.p, hq, ldh, 0, false, s, ro));
-      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, n, hq, ldh, wv, pt.p, nrm2, 1, 0, s, ro, nullptr,
+      HIPCHK(c, glh::launch_seg_mdot<TV>(SA, j + 2, V.p, ldv, wv, pt.p, hs, ldh, 0, false, s, cyc));
+      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, ldv, hs, ldh, wv, pt.p, nrm2, 1, 0, s, cyc, &C, 1, j));
+      HIPCHK(c, glh::launch_seg_mdot<TV>(SR, j + 1, V.p, ldv, wv, pt.p, hq, ldh, 0, false, s, ro));
+      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SA, j + 1, V.p, ldv, hq, ldh, wv, pt.p, nrm2, 1, 0, s, ro, nullptr,
                                                      0, j, nullptr, 0, false));
       // as above: the pass's norm reduction (its partials where it ran), op 2
       // and the normalisation in one launch
@@ -808,7 +812,7 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   auto &pt = Work<TV>::part(c);
   auto &yb = Work<TV>::y(c);
   auto &sc = Work<TV>::sc(c);
-  HIPCHK(c, V.alloc(n * (m + 1)));
+  HIPCHK(c, V.alloc(basis_stride(c) * (m + 1)));
   HIPCHK(c, Z.alloc(n));
   HIPCHK(c, W.alloc(n));
   HIPCHK(c, hs.alloc((size_t)S * ldh));
@@ -1763,6 +1767,9 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
     segch.push_back((int)(ch.size() / 3));
   }
   c->n_chunks = (int)(ch.size() / 3);
+  long long clen = 2;
+  for (int i = 0; i < c->n_chunks; ++i) clen = std::max(clen, ch[3 * i + 2] - ch[3 * i + 1]);
+  c->chunk_len = (int)clen;
   c->max_seg_chunks = 0;
   for (int sg = 0; sg < c->n_seg; ++sg) c->max_seg_chunks = std::max(c->max_seg_chunks, segch[sg + 1] - segch[sg]);
   HIPCHK(c, upload(c->cell_nodes, m.cell_nodes.data(), m.cell_nodes.size(), s));

@@ -241,6 +241,7 @@ struct SegInfo {
   // Gram-Schmidt pass), where dispatching a workgroup per chunk only to skip
   // it is most of the cost
   int cap = 0;
+  int len = (int)GS_MAX_CHUNK;  // no chunk is longer
 };
 // rhs = -R from the residual's cell slots (launch_res_apply); with partial,
 // the chunks' sums of squares of rhs there (for launch_seg_final).
