@@ -1147,6 +1147,49 @@ __global__ __launch_bounds__(RT) void k_seg_final_ctl(const int *__restrict__ se
   }
 }
 
+// Control op 2 of one instance by a whole workgroup: the new column (both
+// passes summed) and the previous rotations are staged in LDS, so that the
+// rotation loop of one thread reads LDS, not a chain of global loads (same
+// arithmetic and order as gmres_ctl_op).  nrm: ||w||^2 after the passes.
+// Returns (thread 0) whether the instance goes on.
+template <typename T>
+__device__ inline int ctl2_column(const GmresCtl<T> &C, int sg, int j, T nrm, bool ro, double *s_col, double *s_cs,
+                                  double *s_sn)
+{
+  const size_t so = (size_t)sg * C.ldh, sr = (size_t)sg * C.m;
+  for (int r = threadIdx.x; r <= j; r += RT) s_col[r] = (double)C.hs[so + r] + (ro ? (double)C.hq[so + r] : 0.0);
+  for (int r = threadIdx.x; r < j; r += RT) {
+    s_cs[r] = C.cs[sr + r];
+    s_sn[r] = C.sn[sr + r];
+  }
+  __syncthreads();
+  int on = 0;
+  if (threadIdx.x == 0) {
+    const int m = C.m;
+    double *g = C.g + (size_t)sg * (m + 1);
+    double *H = C.H + (size_t)sg * (m + 1) * m;
+    const double hn = nrm > (T)0 ? sqrt((double)nrm) : 0.0;
+    double cur = s_col[0];
+    for (int r = 0; r < j; ++r) {
+      const double nxt = s_col[r + 1], c_ = s_cs[r], s_ = s_sn[r];
+      H[(size_t)r * m + j] = c_ * cur + s_ * nxt;
+      cur = -s_ * cur + c_ * nxt;
+    }
+    const double rr = hypot(cur, hn);
+    const double c_ = rr > 0 ? cur / rr : 1.0, s_ = rr > 0 ? hn / rr : 0.0, gj = g[j];
+    C.cs[sr + j] = c_;
+    C.sn[sr + j] = s_;
+    H[(size_t)j * m + j] = rr;
+    g[j + 1] = -s_ * gj;
+    g[j] = c_ * gj;
+    C.jseg[sg] = j + 1;
+    C.its[sg] += 1;
+    on = !(fabs(-s_ * gj) <= C.target[sg] || hn == 0.0);
+    C.cyc[sg] = on;
+  }
+  return on;
+}
+
 // After the second Gram-Schmidt pass: its norm reduction, control op 2 and
 // the normalisation of V_{j+1} in one launch over the chunks (the second
 // pass rarely runs; where it did not, the first pass's norm is read).  Every workgroup of an iterating instance forms
@@ -1191,41 +1234,8 @@ __global__ __launch_bounds__(RT) void k_seg_ctl2_scale(const long long *__restri
       nrm = block_reduce(acc, sh);
     }
     if (cb == seg_chunk[sg]) {
-      // op 2 with the new column (both passes summed) and the previous
-      // rotations staged in LDS by the workgroup: the rotation loop of one
-      // thread then reads LDS, not a chain of global loads (same arithmetic
-      // and order as gmres_ctl_op)
-      const size_t so = (size_t)sg * C.ldh, sr = (size_t)sg * C.m;
-      for (int r = threadIdx.x; r <= j; r += RT)
-        s_col[r] = (double)C.hs[so + r] + (ro ? (double)C.hq[so + r] : 0.0);
-      for (int r = threadIdx.x; r < j; r += RT) {
-        s_cs[r] = C.cs[sr + r];
-        s_sn[r] = C.sn[sr + r];
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        if (ro) norm2[sg] = nrm;
-        const int m = C.m;
-        double *g = C.g + (size_t)sg * (m + 1);
-        double *H = C.H + (size_t)sg * (m + 1) * m;
-        double *cs = C.cs + sr, *sn = C.sn + sr;
-        const double hn = nrm > (T)0 ? sqrt((double)nrm) : 0.0;
-        double cur = s_col[0];
-        for (int r = 0; r < j; ++r) {
-          const double nxt = s_col[r + 1], c_ = s_cs[r], s_ = s_sn[r];
-          H[(size_t)r * m + j] = c_ * cur + s_ * nxt;
-          cur = -s_ * cur + c_ * nxt;
-        }
-        const double rr = hypot(cur, hn);
-        cs[j] = rr > 0 ? cur / rr : 1.0;
-        sn[j] = rr > 0 ? hn / rr : 0.0;
-        H[(size_t)j * m + j] = rr;
-        g[j + 1] = -sn[j] * g[j];
-        g[j] = cs[j] * g[j];
-        C.jseg[sg] = j + 1;
-        C.its[sg] += 1;
-        if (fabs(g[j + 1]) <= C.target[sg] || hn == 0.0) C.cyc[sg] = 0;
-      }
+      ctl2_column(C, (int)sg, j, nrm, ro, s_col, s_cs, s_sn);
+      if (threadIdx.x == 0 && ro) norm2[sg] = nrm;
     }
     const T a = nrm > (T)0 ? sqrt(nrm) : (T)0;
     const T inv = a != (T)0 ? (T)1 / a : (T)1;
@@ -1233,6 +1243,60 @@ __global__ __launch_bounds__(RT) void k_seg_ctl2_scale(const long long *__restri
   }
 }
 
+
+// The end of an Arnoldi step of a single instance: the norm after the first
+// Gram-Schmidt pass from its chunk partials (every workgroup forms it, in
+// k_seg_final_ctl's order), op 1, and where no second pass is needed op 2 and
+// the normalisation.  A column that needs the second pass stops the instance
+// (cyc 0, ro 1) until the host has enqueued that pass and this kernel again
+// with resume set, which takes the second pass's partials: steps enqueued
+// ahead in the meantime find nothing to do.  status (host memory): 0 stopped,
+// 1 goes on, 2 second pass needed.
+template <typename T>
+__global__ __launch_bounds__(RT) void k_step_end(const long long *__restrict__ ch, int n_chunks,
+                                                 const T *__restrict__ partial, T *norm2, GmresCtl<T> C, int j,
+                                                 T *__restrict__ w, int resume, int *status)
+{
+  __shared__ T sh[RT];
+  __shared__ int s_it;
+  __shared__ double s_col[128], s_cs[128], s_sn[128];  // j < m <= 126
+  const int cb = blockIdx.x;
+  // read once per workgroup: the first workgroup's op may clear it meanwhile
+  if (threadIdx.x == 0) s_it = resume ? C.ro[0] : C.cyc[0];
+  T acc = 0;
+  for (int b = threadIdx.x; b < n_chunks; b += RT) acc += partial[b];
+  const T nrm = block_reduce(acc, sh);  // (its barriers cover s_it)
+  const bool first = cb == 0 && threadIdx.x == 0;
+  if (!s_it) {
+    if (first) __hip_atomic_store(status, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  if (!resume && (double)nrm < C.dgks * (double)C.hs[j + 1]) {
+    if (first) {
+      norm2[0] = nrm;
+      C.ro[0] = 1;
+      C.cyc[0] = 0;
+      __hip_atomic_store(status, 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return;
+  }
+  if (cb == 0) {
+    const int on = ctl2_column(C, 0, j, nrm, resume != 0, s_col, s_cs, s_sn);
+    if (first) {
+      norm2[0] = nrm;
+      if (!resume) C.ro[0] = 0;
+      __hip_atomic_store(status, on, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  const T a = nrm > (T)0 ? sqrt(nrm) : (T)0;
+  const T inv = a != (T)0 ? (T)1 / a : (T)1;
+  const long long beg = ch[3 * cb + 1], end = ch[3 * cb + 2];
+  for (long long i = beg + Quad<T>::N * threadIdx.x; i < end; i += Quad<T>::N * RT) {
+    auto v = ldc<false, false>(w, i, end);
+    v *= inv;
+    stc<false>(w, i, end, v);
+  }
+}
 
 template <typename T>
 __global__ __launch_bounds__(RT) void k_fill(size_t n, T v, T *__restrict__ d)
@@ -1525,6 +1589,16 @@ hipError_t launch_seg_ctl2_scale(const SegInfo &S, const T *partial, T *norm2, c
 }
 
 template <typename T>
+hipError_t launch_step_end(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, T *w,
+                           bool resume, int *status, hipStream_t s)
+{
+  if (S.n_seg != 1 || S.n_chunks <= 0 || norm2 != C.nrm2 || !status) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_step_end<T>), dim3(S.n_chunks), dim3(RT), 0, s, S.chunks, S.n_chunks, partial, norm2, C, j, w,
+                     resume ? 1 : 0, status);
+  return hipGetLastError();
+}
+
+template <typename T>
 hipError_t launch_seg_lincomb(const SegInfo &S, int k, const T *V, size_t ldv, const T *y, int ldy, T *w,
                               hipStream_t s, const int *kseg)
 {
@@ -1608,6 +1682,8 @@ hipError_t launch_seg_residual(const SegInfo &S, const T *b, const T *w, T *r, T
                                                      const GmresCtl<T> *, int, int, const T *, int, bool);         \
   template hipError_t launch_seg_ctl2_scale<T>(const SegInfo &, const T *, T *, const GmresCtl<T> &, int, T *,     \
                                                hipStream_t);                                                       \
+  template hipError_t launch_step_end<T>(const SegInfo &, const T *, T *, const GmresCtl<T> &, int, T *, bool, int *, \
+                                         hipStream_t);                                                             \
   template hipError_t launch_seg_lincomb<T>(const SegInfo &, int, const T *, size_t, const T *, int, T *,          \
                                             hipStream_t, const int *);                                             \
   template hipError_t launch_seg_scale<T>(const SegInfo &, const T *, const T *, int, T *, hipStream_t,            \

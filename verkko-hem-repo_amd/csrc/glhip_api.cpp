@@ -176,6 +176,8 @@ struct glh_ctx {
     int q = 1;
   } graph64, graph32;
   HBuf<float> pin32;
+  HBuf<int> pin_st;  // status of each step of a single instance's cycle, written by the device
+  hipEvent_t ev_step[2] = {nullptr, nullptr};  // the two last steps enqueued
   HBuf<int> pin_i, pin_fl;  // pinned staging of the per-instance flags and counters
   DBuf<double> ir_r;
   // per-instance results of the last Newton solve: 8 values per instance
@@ -753,6 +755,32 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
     else HIPCHK(c, (glh::launch_axpy<TV, TV>(n, 1.0, Z.p, x, s)));
     return GLH_OK;
   }
+  if (c->n_seg == 1) {
+    // one step (part 1), or the second Gram-Schmidt pass of step j0 (part 3),
+    // which a column rarely needs: the host enqueues it when the step's
+    // status asks for it.  The updates of a small instance sum the multi-dot
+    // partials themselves.
+    const int j = j0;
+    TV *wv = V.p + ldv * (j + 1);
+    int *st = c->pin_st.p + j;
+    const bool small = c->n_chunks <= FOLD_MAX_CHUNKS;
+    if (part == 3) {
+      HIPCHK(c, glh::launch_seg_mdot<TV>(SI, j + 1, V.p, ldv, wv, pt.p, hq, ldh, 0, false, s, ro, !small));
+      HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SI, j + 1, V.p, ldv, hq, ldh, wv, np, nrm2, 1, 0, s, ro, nullptr,
+                                                     0, j, small ? pt.p : nullptr, small ? j + 1 : 0, false));
+      HIPCHK(c, glh::launch_step_end<TV>(SI, np, nrm2, C, j, wv, true, st, s));
+      return GLH_OK;
+    }
+    TV *vj = V.p + ldv * j;
+    if (j == 0) HIPCHK(c, glh::launch_seg_scale<TV>(SI, V.p, nrm2, 1, V.p, s, cyc, true));
+    HIPCHK(c, (glh::launch_bj_apply<TJ, TV>(c->n_nodes, Dinv, vj, Z.p, s, rs, cyc, act)));
+    RCHK(mv(Z.p, wv, cyc, act));
+    HIPCHK(c, glh::launch_seg_mdot<TV>(SI, j + 2, V.p, ldv, wv, pt.p, hs, ldh, 0, false, s, cyc, !small));
+    HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SI, j + 1, V.p, ldv, hs, ldh, wv, np, nrm2, 1, 0, s, cyc, nullptr,
+                                                   0, j, small ? pt.p : nullptr, small ? j + 2 : 0, false));
+    HIPCHK(c, glh::launch_step_end<TV>(SI, np, nrm2, C, j, wv, false, st, s));
+    return GLH_OK;
+  }
   // body block: Arnoldi steps j0 <= j < j1
   if (j0 == 0) HIPCHK(c, glh::launch_seg_scale<TV>(SA, V.p, nrm2, 1, V.p, s, cyc, true));
   for (int j = j0; j < j1; ++j) {
@@ -833,6 +861,7 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   HIPCHK(c, c->act_counts.alloc(4));
   // every host <-> device copy of the loop below goes through pinned memory
   HIPCHK(c, c->pin_i.alloc(2 * (size_t)S + 4));
+  HIPCHK(c, c->pin_st.alloc(128));
   HIPCHK(c, Work<TV>::pin(c).alloc(S));
   HIPCHK(c, c->act_seg.alloc(S));
   HIPCHK(c, c->act_rpref.alloc(S + 1));
@@ -887,12 +916,15 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   if (!timed && gc.key != key) {
     for (auto e : gc.exec)
       if (e) (void)hipGraphExecDestroy(e);
-    gc.exec.assign(1 + NLEV * (1 + nblk), nullptr);
+    gc.exec.assign(1 + NLEV * (1 + nblk) + nblk, nullptr);
     gc.key = key;
     gc.q = q;
   }
-  // graph slot: 0 head; per level L: tail, then the body blocks
-  auto slot = [&](int part, int lev, int blk) { return part == 0 ? 0 : 1 + lev * (1 + nblk) + (part == 2 ? 0 : 1 + blk); };
+  // graph slot: 0 head; per level L: tail, then the body blocks; then the
+  // second passes of a single instance's steps
+  auto slot = [&](int part, int lev, int blk) {
+    return part == 0 ? 0 : part == 3 ? 1 + NLEV * (1 + nblk) + blk : 1 + lev * (1 + nblk) + (part == 2 ? 0 : 1 + blk);
+  };
   auto launch = [&](int part, int lev, int blk) -> int {
     const int j0 = blk * q, j1 = std::min(m, j0 + q), shift = 3 * lev;
     if (timed) return enqueue_cycle<TJ, TV>(c, J, Dinv, b, x, m, C, true, part, j0, j1, shift);
@@ -940,6 +972,38 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
     if (S > 1) {
       const double f = (double)hcnt[2] / std::max(1, c->n_nodes);
       lev = f > 1.0 / 8 ? 0 : f > 1.0 / 64 ? 1 : 2;
+    }
+    if (S == 1) {
+      // A step ahead: while step j runs, step j + 1 is enqueued (it skips
+      // itself if j turns out to be the last, or to need its second pass), so
+      // the device does not wait for the host to read j's status.  With
+      // kernel timing on, each step is waited for, so that no skipped product
+      // is counted.
+      for (auto &e : c->ev_step)
+        if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      volatile int *st = c->pin_st.p;
+      auto step = [&](int j) -> int {
+        RCHK(launch(1, lev, j));
+        HIPCHK(c, hipEventRecord(c->ev_step[j & 1], s));
+        return GLH_OK;
+      };
+      RCHK(step(0));
+      for (int j = 0; j < nblk; ++j) {
+        const bool ahead = !timed && j + 1 < nblk;
+        if (ahead) RCHK(step(j + 1));
+        HIPCHK(c, hipEventSynchronize(c->ev_step[j & 1]));
+        int v = st[j];
+        if (v == 2) {
+          RCHK(launch(3, lev, j));
+          HIPCHK(c, hipStreamSynchronize(s));
+          v = st[j];
+          if (v == 1 && ahead) RCHK(step(j + 1));  // the one enqueued before has skipped itself
+        }
+        if (v != 1) break;
+        if (!ahead && j + 1 < nblk) RCHK(step(j + 1));
+      }
+      RCHK(launch(2, lev, 0));
+      continue;
     }
     for (int blk = 0; blk < nblk; ++blk) {
       RCHK(launch(1, lev, blk));
@@ -1196,6 +1260,9 @@ int glh_destroy(glh_ctx *c)
   c->pinv.release();
   c->pin32.release();
   c->pin_i.release();
+  c->pin_st.release();
+  for (auto e : c->ev_step)
+    if (e) (void)hipEventDestroy(e);
   c->pin_fl.release();
   for (auto e : c->ev_pool)
     if (e) (void)hipEventDestroy(e);
