@@ -58,8 +58,9 @@ struct Buf {
   }
 };
 
-constexpr int OUTP = 64;       // padded width of the output layer
+constexpr int OUTP = glh::mlp::MLP_OUTP;  // padded width of the output layer
 constexpr int DW_SPLITS = 64;  // K splits of the weight-gradient products
+constexpr int PREDICT_ROWS = 65536;  // points of an inference pass
 
 }  // namespace
 
@@ -68,11 +69,13 @@ struct glh_mlp {
   hipStream_t stream = nullptr;
   std::string err;
   int F = 64, width = 256, depth = 5, n_out = 18;
+  bool tiled = false;                    // layers fit a tile of rows in LDS (mlp_pass.hip)
   std::vector<int> K, N, Np;             // per layer
   std::vector<long long> woff, boff;     // offsets in the flat parameters
   long long n_params = 0;
   Buf<float> P, G, Mo, Vo, Bf;
-  std::vector<Buf<bf16>> Wb, WbT;  // BF16 weights, K x Np and transposed Np x K
+  // BF16 weights: K x Np and transposed Np x K, or (tiled) the fragments of both
+  std::vector<Buf<bf16>> Wb, WbT;
   Buf<float> Xall, Yall;
   long long n_data = 0;
   // batch workspace
@@ -81,6 +84,8 @@ struct glh_mlp {
   std::vector<Buf<bf16>> H;
   std::vector<Buf<float>> Z;
   Buf<bf16> dY, dZa, dZb;
+  std::vector<Buf<bf16>> dZ;  // tiled: every layer's, kept for the weight gradients
+  Buf<float> Xp, Yp;          // inference: points of a pass, outputs
   Buf<int> step;
   hipGraphExec_t graph = nullptr;
   int graph_nb = 0;
@@ -109,9 +114,46 @@ int fail(glh_mlp *m, int code, const std::string &msg)
 
 int pack_all(glh_mlp *m)
 {
+  const auto pack = m->tiled ? glh::mlp::pack_frag : glh::mlp::pack_w;
   for (int l = 0; l <= m->depth; ++l)
-    MCHK(m, glh::mlp::pack_w(m->K[l], m->N[l], m->Np[l], m->P.p + m->woff[l], m->Wb[l].p, m->WbT[l].p,
-                             m->stream));
+    MCHK(m, pack(m->K[l], m->N[l], m->Np[l], m->P.p + m->woff[l], m->Wb[l].p, m->WbT[l].p, m->stream));
+  return GLH_OK;
+}
+
+// Splits of a gradient's 32-sample steps outside training (which keeps
+// dw_splits: its parameters would otherwise drift apart in the rounding).  A
+// sum is steps / splits products long and then splits long: shortest, in time
+// and in rounding, near the square root, whole splits to every XCD above 8.
+int grad_splits(int steps)
+{
+  const int sp = std::max(1, (int)std::sqrt((double)steps));
+  return sp > 8 ? std::min(sp / 8 * 8, DW_SPLITS) : sp;
+}
+
+// workspaces of a gradient over nb rows, for tiles of up to 128 rows
+int ensure_tiled(glh_mlp *m, int nb)
+{
+  const size_t rows = ((size_t)nb + 127) / 128 * 128;
+  m->H.resize(m->depth + 1);
+  m->Z.resize(m->depth);
+  m->dZ.resize(m->depth + 1);
+  MCHK(m, m->Xb.alloc((size_t)nb * 6));
+  MCHK(m, m->Yb.alloc((size_t)nb * m->n_out));
+  size_t ptot = 0, ctot = 0;
+  for (int l = 0; l <= m->depth; ++l) {
+    MCHK(m, m->H[l].alloc(rows * m->K[l]));
+    MCHK(m, m->dZ[l].alloc(rows * m->Np[l]));
+    if (l < m->depth) MCHK(m, m->Z[l].alloc(rows * m->width));
+    ptot += (size_t)m->K[l] * m->Np[l];
+    ctot += (size_t)m->Np[l];
+  }
+  MCHK(m, m->part.alloc(ptot * DW_SPLITS));
+  MCHK(m, m->cpart.alloc(ctot * DW_SPLITS));
+  MCHK(m, m->lpart.alloc(rows / 32));
+  MCHK(m, m->loss.alloc(1));
+  m->nb = nb;
+  if (m->graph) (void)hipGraphExecDestroy(m->graph);
+  m->graph = nullptr;
   return GLH_OK;
 }
 
@@ -119,6 +161,7 @@ int ensure_batch(glh_mlp *m, int nb)
 {
   if (nb % 64 || nb < 64) return fail(m, GLH_ERR_ARG, "batch must be a positive multiple of 64");
   if (m->nb == nb) return GLH_OK;
+  if (m->tiled) return ensure_tiled(m, nb);
   m->H.resize(m->depth + 1);
   m->Z.resize(m->depth);
   MCHK(m, m->Xb.alloc((size_t)nb * 6));
@@ -238,9 +281,94 @@ int forward_backward(glh_mlp *m, int n_real, bool grad)
   return GLH_OK;
 }
 
+glh::mlp::PassArgs pass_args(glh_mlp *m, int n_real)
+{
+  glh::mlp::PassArgs A;
+  A.depth = m->depth; A.F = m->F; A.width = m->width; A.n_out = m->n_out; A.n_real = n_real;
+  A.Bf = m->Bf.p;
+  A.P = m->P.p;
+  for (int l = 0; l <= m->depth; ++l) {
+    A.boff[l] = m->boff[l];
+    A.WT[l] = m->WbT[l].p;
+    A.Wb[l] = m->Wb[l].p;
+  }
+  return A;
+}
+
+// Tiled networks: loss and gradient of n_real rows of X, T into loss and G,
+// or (adam) a training step over n_real rows drawn from them.  Three launches.
+int tiled_step(glh_mlp *m, int n_real, const float *X, const float *T, bool adam, uint64_t seed, float lr)
+{
+  hipStream_t s = m->stream;
+  const int D = m->depth;
+  glh::mlp::PassArgs A = pass_args(m, n_real);
+  A.X = X;
+  A.T = T;
+  A.lpart = m->lpart.p;
+  if (adam) {
+    A.step = m->step.p;
+    A.seed = seed;
+    A.n_data = m->n_data;
+  }
+  A.n_rows = m->nb;
+  const int steps = m->nb / 32, sp0 = adam ? dw_splits(m->nb) : grad_splits(steps), per = (steps + sp0 - 1) / sp0,
+            sp = (steps + per - 1) / per;
+  glh::mlp::WgradArgs Wg;
+  glh::mlp::UpdateArgs U;
+  Wg.n_layers = U.n_layers = D + 1;
+  Wg.splits = U.splits = sp;
+  Wg.ksteps = steps;
+  Wg.per = per;
+  Wg.part = m->part.p;
+  Wg.cpart = m->cpart.p;
+  U.part = m->part.p;
+  U.cpart = m->cpart.p;
+  long long po = 0, co = 0;
+  int unit = 0;
+  for (int l = 0; l <= D; ++l) {
+    A.H[l] = m->H[l].p;
+    A.dZ[l] = m->dZ[l].p;
+    if (l < D) A.Z[l] = m->Z[l].p;
+    Wg.H[l] = m->H[l].p;
+    Wg.dZ[l] = m->dZ[l].p;
+    const int nA = m->K[l] / 16, nB = l < D ? m->width / 16 : (m->n_out + 31) / 32 * 2;
+    Wg.nA[l] = U.nA[l] = nA;
+    Wg.nB[l] = U.nB[l] = nB;
+    U.N[l] = m->N[l];
+    U.Np[l] = m->Np[l];
+    U.woff[l] = m->woff[l];
+    U.boff[l] = m->boff[l];
+    U.WT[l] = m->WbT[l].p;
+    U.Wb[l] = m->Wb[l].p;
+    Wg.poff[l] = U.poff[l] = po;
+    Wg.coff[l] = U.coff[l] = co;
+    po += (long long)sp * nA * nB * 256;
+    co += (long long)sp * nB * 16;
+    U.unit0[l] = unit;
+    unit += nA * nB * 64 + m->N[l];
+  }
+  U.unit0[D + 1] = unit;
+  Wg.step = adam ? m->step.p : nullptr;
+  U.lpart = m->lpart.p;
+  const int pr = glh::mlp::pass_rows(n_real, m->width);
+  U.n_lpart = (m->nb + pr - 1) / pr;
+  U.loss = m->loss.p;
+  U.G = m->G.p;
+  U.P = m->P.p;
+  U.m = m->Mo.p;
+  U.v = m->Vo.p;
+  U.lr = lr; U.b1 = 0.9f; U.b2 = 0.999f; U.eps = 1e-8f;
+  U.step = m->step.p;
+  MCHK(m, glh::mlp::pass(A, true, s));
+  MCHK(m, glh::mlp::wgrad(Wg, s));
+  MCHK(m, glh::mlp::update(U, adam, s));
+  return GLH_OK;
+}
+
 int train_step(glh_mlp *m, uint64_t seed, float lr)
 {
   hipStream_t s = m->stream;
+  if (m->tiled) return tiled_step(m, m->nb, m->Xall.p, m->Yall.p, true, seed, lr);
   MCHK(m, glh::mlp::step_inc(m->step.p, s));
   MCHK(m, glh::mlp::gather(m->nb, m->n_data, seed, m->step.p, m->Xall.p, m->Yall.p, m->n_out, m->Xb.p, m->Yb.p, s));
   RCHK(forward_backward(m, m->nb, true));
@@ -271,6 +399,7 @@ int glh_mlp_create(int device, int n_freq, double sigma, int width, int depth, i
   auto *m = new glh_mlp();
   m->device = device;
   m->F = n_freq; m->width = width; m->depth = depth; m->n_out = n_out;
+  m->tiled = width <= glh::mlp::MLP_PASS_MAX && 2 * n_freq <= glh::mlp::MLP_PASS_MAX;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) {
     delete m;
     return GLH_ERR_HIP;
@@ -340,12 +469,13 @@ int glh_mlp_destroy(glh_mlp *m)
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   if (m->graph) (void)hipGraphExecDestroy(m->graph);
   Buf<float> *fb[] = {&m->P, &m->G, &m->Mo, &m->Vo, &m->Bf, &m->Xall, &m->Yall, &m->Xb, &m->Yb,
-                      &m->Yo, &m->part, &m->cpart, &m->lpart, &m->loss};
+                      &m->Yo, &m->part, &m->cpart, &m->lpart, &m->loss, &m->Xp, &m->Yp};
   for (auto *b : fb) b->release();
   for (auto &b : m->Wb) b.release();
   for (auto &b : m->WbT) b.release();
   for (auto &b : m->H) b.release();
   for (auto &b : m->Z) b.release();
+  for (auto &b : m->dZ) b.release();
   m->dY.release();
   m->dZa.release();
   m->dZb.release();
@@ -435,11 +565,14 @@ int glh_mlp_loss_grad(glh_mlp *m, int n, const float *X, const float *Y, float *
   const int nb = (n + 63) / 64 * 64;
   RCHK(ensure_batch(m, nb));
   hipStream_t s = m->stream;
-  MCHK(m, hipMemsetAsync(m->Xb.p, 0, (size_t)nb * 6 * sizeof(float), s));
-  MCHK(m, hipMemsetAsync(m->Yb.p, 0, (size_t)nb * m->n_out * sizeof(float), s));
+  if (!m->tiled) {  // the products run over the padding rows too
+    MCHK(m, hipMemsetAsync(m->Xb.p, 0, (size_t)nb * 6 * sizeof(float), s));
+    MCHK(m, hipMemsetAsync(m->Yb.p, 0, (size_t)nb * m->n_out * sizeof(float), s));
+  }
   MCHK(m, hipMemcpyAsync(m->Xb.p, X, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, s));
   MCHK(m, hipMemcpyAsync(m->Yb.p, Y, (size_t)n * m->n_out * sizeof(float), hipMemcpyHostToDevice, s));
-  RCHK(forward_backward(m, n, true));
+  if (m->tiled) RCHK(tiled_step(m, n, m->Xb.p, m->Yb.p, false, 0, 0.f));
+  else RCHK(forward_backward(m, n, true));
   float L = 0.f;
   MCHK(m, hipMemcpyAsync(&L, m->loss.p, sizeof(float), hipMemcpyDeviceToHost, s));
   if (grad) MCHK(m, hipMemcpyAsync(grad, m->G.p, m->n_params * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -452,31 +585,29 @@ int glh_mlp_predict(glh_mlp *m, int64_t n, const float *X, float *Y)
 {
   if (!m || n < 1 || !X || !Y) return GLH_ERR_ARG;
   hipStream_t s = m->stream;
-  // in chunks of at most 65536 points
-  const int chunk = 65536;
-  Buf<float> Yt;
-  MCHK(m, Yt.alloc((size_t)chunk * m->n_out));
+  const int chunk = (int)std::min<int64_t>(n, PREDICT_ROWS);
+  if (m->tiled) MCHK(m, m->Xp.alloc((size_t)chunk * 6));
+  MCHK(m, m->Yp.alloc((size_t)chunk * m->n_out));
   for (int64_t i0 = 0; i0 < n; i0 += chunk) {
     const int nr = (int)std::min<int64_t>(chunk, n - i0);
-    const int nb = (nr + 63) / 64 * 64;
-    if (m->nb < nb) {
-      const int rc = ensure_batch(m, nb);
-      if (rc) { Yt.release(); return rc; }
+    if (m->tiled) {
+      MCHK(m, hipMemcpyAsync(m->Xp.p, X + i0 * 6, (size_t)nr * 6 * sizeof(float), hipMemcpyHostToDevice, s));
+      glh::mlp::PassArgs A = pass_args(m, nr);
+      A.X = m->Xp.p;
+      A.Y = m->Yp.p;
+      MCHK(m, glh::mlp::pass(A, false, s));
+    } else {
+      const int nb = (nr + 63) / 64 * 64;
+      if (m->nb < nb) RCHK(ensure_batch(m, nb));
+      // forward over the allocated batch rows (rows beyond nr are zero inputs)
+      MCHK(m, hipMemsetAsync(m->Xb.p, 0, (size_t)m->nb * 6 * sizeof(float), s));
+      MCHK(m, hipMemcpyAsync(m->Xb.p, X + i0 * 6, (size_t)nr * 6 * sizeof(float), hipMemcpyHostToDevice, s));
+      RCHK(forward_backward(m, nr, false));
+      MCHK(m, glh::mlp::take_out(nr, m->n_out, OUTP, m->Yo.p, m->Yp.p, s));
     }
-    hipError_t e = hipMemsetAsync(m->Xb.p, 0, (size_t)m->nb * 6 * sizeof(float), s);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(m->Xb.p, X + i0 * 6, (size_t)nr * 6 * sizeof(float), hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) { Yt.release(); return fail(m, GLH_ERR_HIP, hipGetErrorString(e)); }
-    // forward over the allocated batch rows (rows beyond nr are zero inputs)
-    const int rc = forward_backward(m, nr, false);
-    if (rc) { Yt.release(); return rc; }
-    e = glh::mlp::take_out(nr, m->n_out, OUTP, m->Yo.p, Yt.p, s);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(Y + i0 * m->n_out, Yt.p, (size_t)nr * m->n_out * sizeof(float), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) { Yt.release(); return fail(m, GLH_ERR_HIP, hipGetErrorString(e)); }
+    MCHK(m, hipMemcpyAsync(Y + i0 * m->n_out, m->Yp.p, (size_t)nr * m->n_out * sizeof(float), hipMemcpyDeviceToHost, s));
+    MCHK(m, hipStreamSynchronize(s));
   }
-  Yt.release();
   return GLH_OK;
 }
 

@@ -7,6 +7,9 @@
 // product accumulates in FP32 (v_mfma_f32_16x16x32_bf16); master weights,
 // gradients and Adam moments are FP32.
 //
+// These kernels serve networks with a layer of more than 256 features, and
+// the general products; narrower networks run in mlp_pass.hip.
+//
 // GEMM: C (FP32) = A B with A (M x K) and B (K x N) in BF16, 64 x 64 tiles,
 // 4 wavefronts of 2 x 2 MFMA 16 x 16 blocks, M, N multiples of 64 and K a
 // multiple of 32 (the host pads).  The network's products run in two

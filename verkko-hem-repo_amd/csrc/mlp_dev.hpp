@@ -70,5 +70,61 @@ hipError_t gather(int nb, long long n_data, uint64_t seed, const int *step, cons
 hipError_t take_out(int n, int n_out, int ldy, const float *Yp, float *Y, hipStream_t s);
 hipError_t step_inc(int *step, hipStream_t s);
 
+
+// ------------------------------------------------------------------------
+// Networks of at most MLP_PASS_MAX features a layer (mlp_pass.hip): the
+// operands as MFMA fragments, three launches a training step.
+constexpr int MLP_PASS_MAX = 256;
+constexpr int MLP_OUTP = 64;  // padded width of the output layer
+struct PassArgs {
+  int depth = 0, F = 0, width = 0, n_out = 0, n_real = 0;
+  int n_rows = 0;  // gradient: n_real rounded up to whole steps of 32
+  const float *X = nullptr, *T = nullptr, *Bf = nullptr, *P = nullptr;
+  long long boff[MLP_MAX_LAYERS];
+  const bf16 *WT[MLP_MAX_LAYERS], *Wb[MLP_MAX_LAYERS];
+  float *Y = nullptr;  // inference: n_real x n_out
+  // gradient: what the weight gradients and the backward sweep read, in rows
+  // padded to pass_rows
+  bf16 *H[MLP_MAX_LAYERS], *dZ[MLP_MAX_LAYERS];
+  float *Z[MLP_MAX_LAYERS];
+  float *lpart = nullptr;  // sums of squares, one per pass_rows
+  // n_data > 0: row i is the point hash(seed, step + 1, i) mod n_data of X, T
+  const int *step = nullptr;
+  uint64_t seed = 0;
+  long long n_data = 0;
+};
+int pass_rows(int n, int width);  // rows of a workgroup's tile at n rows
+// forward over n_real rows; with grad also the loss and dZ of every layer
+hipError_t pass(const PassArgs &A, bool grad, hipStream_t s);
+
+// Layer l: nA x nB blocks of 16 x 16; split z takes the 32-sample steps
+// z per .. + per - 1 of ksteps and writes nA nB blocks (64 lanes x 4 FP32) at
+// part + poff[l] + z nA nB 256 and its column sums at cpart + coff[l] + z nB 16.
+struct WgradArgs {
+  int n_layers = 0, splits = 1, per = 1, ksteps = 0;
+  int nA[MLP_MAX_LAYERS], nB[MLP_MAX_LAYERS], tile0[MLP_MAX_LAYERS + 1];  // tile0: set by wgrad()
+  const bf16 *H[MLP_MAX_LAYERS], *dZ[MLP_MAX_LAYERS];
+  float *part = nullptr, *cpart = nullptr;
+  long long poff[MLP_MAX_LAYERS], coff[MLP_MAX_LAYERS];
+  int *step = nullptr;  // incremented when set
+};
+hipError_t wgrad(const WgradArgs &A, hipStream_t s);
+
+struct UpdateArgs {
+  int n_layers = 0, splits = 1, n_lpart = 0;
+  int nA[MLP_MAX_LAYERS], nB[MLP_MAX_LAYERS], N[MLP_MAX_LAYERS], Np[MLP_MAX_LAYERS], unit0[MLP_MAX_LAYERS + 1];
+  const float *part = nullptr, *cpart = nullptr, *lpart = nullptr;
+  long long poff[MLP_MAX_LAYERS], coff[MLP_MAX_LAYERS], woff[MLP_MAX_LAYERS], boff[MLP_MAX_LAYERS];
+  float *G = nullptr, *loss = nullptr;
+  float *P = nullptr, *m = nullptr, *v = nullptr;
+  float lr = 0.f, b1 = 0.f, b2 = 0.f, eps = 0.f;
+  const int *step = nullptr;
+  bf16 *WT[MLP_MAX_LAYERS], *Wb[MLP_MAX_LAYERS];
+};
+// loss = the sum of lpart; G = the gradient, or with adam the parameter step
+hipError_t update(const UpdateArgs &A, bool adam, hipStream_t s);
+// fragment copies of W (K x N, zeros up to Np): WT of W, Wb of its transpose
+hipError_t pack_frag(int K, int N, int Np, const float *W, bf16 *Wb, bf16 *WT, hipStream_t s);
+
 }  // namespace mlp
 }  // namespace glh
