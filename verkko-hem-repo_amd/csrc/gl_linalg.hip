@@ -66,6 +66,15 @@ __device__ inline void pair_ld(const T *__restrict__ p, double &a, double &b)
   b = v.y;
 }
 
+// Order the LDS accesses of one wavefront around a point where its lanes
+// exchange values (the wavefront runs in step; no workgroup barrier).
+__device__ inline void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Block-row layout of the SpMV and the block-Jacobi apply: one wavefront per
 // block row.  The 324 row-major values of a block are read as 162 consecutive
 // pairs; lane l < 54 takes pairs k*54 + l (k < 3), i.e. row 6k + l/9 at
@@ -212,13 +221,190 @@ __global__ __launch_bounds__(256) void k_res_spmv(int n_rows, const int *__restr
   if (lane < 18) r[(size_t)row * 18 + lane] = bv[(size_t)row * 18 + lane] - t;
 }
 
-// Order the LDS accesses of one wavefront around a point where its lanes
-// exchange values (the wavefront runs in step; no workgroup barrier).
-__device__ inline void wave_lds_sync()
+// The same products from the upper triangle only: the Jacobian is the Hessian
+// of a free energy, masked and condensed symmetrically, so block (j, i) is the
+// transpose of block (i, j).  A wavefront reads the blocks of its row from the
+// diagonal on; each gives its row sums as above and, from the same registers,
+// x_row times the block for the row of its column.  Those 18 values go to the
+// block's slot of T in FP64 (nothing is rounded before the row's sum), the
+// row sums to the diagonal's slot, and k_spmv_low sums a row's slots in column
+// order.  Reading the matrix bounds the product: 3.1 GB FP64 (20615 Q2 nodes)
+// 531 us whole at 5.9 TB/s; the half and the slots (1.6 GB read, 0.09 written
+// and read) 329 + 22 us.  FP32, 15625 Q2 nodes: 249 -> 173 us.
+template <typename TJ>
+__device__ inline void pair_raw(const TJ *__restrict__ p, typename V2t<TJ>::type &v)
 {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  typedef TJ vec2 __attribute__((ext_vector_type(2)));
+  const vec2 t = __builtin_nontemporal_load(reinterpret_cast<const vec2 *>(p));
+  v.x = t.x;
+  v.y = t.y;
+}
+template <typename TJ, typename TX>
+__device__ inline void spmv_up_row(int row, int lane, const int *__restrict__ rp, const int *__restrict__ diag,
+                                   const int *__restrict__ col, const TJ *__restrict__ val, const TX *__restrict__ x,
+                                   double *__restrict__ T, double *red)
+{
+  constexpr int U = 3;   // blocks per step: 54 lanes = 3 x 18 sums
+  constexpr int CB = 63; // columns held by the wavefront's lanes at a time
+  RowAcc acc;
+  const int b0 = diag[row], b1 = rp[row + 1];
+  const int ln = lane < 54 ? lane : 53, m = ln / 9, cp = 2 * (ln % 9);
+  double xr[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) xr[k] = (double)x[(size_t)row * 18 + 6 * k + m];
+  const int us = lane / 18, uc = lane - 18 * us;
+  struct Step {
+    typename V2t<TJ>::type v[U][3];
+    typename V2t<TX>::type w[U];
+  } A, B;
+  for (int c0 = b0; c0 < b1; c0 += CB) {
+    const int nb = b1 - c0 < CB ? b1 - c0 : CB;
+    const int cl = col[c0 + (lane < nb ? lane : nb - 1)];
+    const auto load = [&](Step &S, int i) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i + u >= nb) continue;
+        const int s = __builtin_amdgcn_readlane(cl, i + u);
+        S.w[u] = *reinterpret_cast<const typename V2t<TX>::type *>(x + (size_t)s * 18 + cp);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) pair_raw(val + (size_t)(c0 + i + u) * 324 + 2 * (54 * k + ln), S.v[u][k]);
+      }
+    };
+    const auto step = [&](const Step &S, int i, double *rd) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i + u >= nb) continue;
+        const double w0 = (double)S.w[u].x, w1 = (double)S.w[u].y;
+        acc.a0 += (double)S.v[u][0].x * w0;
+        acc.a0 += (double)S.v[u][0].y * w1;
+        acc.a1 += (double)S.v[u][1].x * w0;
+        acc.a1 += (double)S.v[u][1].y * w1;
+        acc.a2 += (double)S.v[u][2].x * w0;
+        acc.a2 += (double)S.v[u][2].y * w1;
+        double t0 = (double)S.v[u][0].x * xr[0], t1 = (double)S.v[u][0].y * xr[0];
+        t0 += (double)S.v[u][1].x * xr[1];
+        t1 += (double)S.v[u][1].y * xr[1];
+        t0 += (double)S.v[u][2].x * xr[2];
+        t1 += (double)S.v[u][2].y * xr[2];
+        if (lane < 54) *reinterpret_cast<double2 *>(rd + u * 108 + 2 * lane) = double2{t0, t1};
+      }
+      wave_lds_sync();
+      if (lane < 54 && i + us < nb) {
+        double t = 0.0;
+#pragma unroll
+        for (int g = 0; g < 6; ++g) t += rd[us * 108 + 18 * g + uc];
+        T[(size_t)(c0 + i + us) * 18 + uc] = t;
+      }
+    };
+    // the next step's blocks are on their way while this one's sums go
+    // through LDS (two buffers: a step writes one while the last is read)
+    load(A, 0);
+    for (int i = 0; i < nb; i += 2 * U) {
+      if (i + U < nb) load(B, i + U);
+      step(A, i, red);
+      if (i + U >= nb) break;
+      if (i + 2 * U < nb) load(A, i + 2 * U);
+      step(B, i + U, red + 324);
+    }
+    wave_lds_sync();
+  }
+  const double t = acc.row_sum(lane, red);
+  if (lane < 18) T[(size_t)b0 * 18 + lane] = t;  // after the diagonal's own slot, by the same lanes
+}
+
+template <typename TJ, typename TX>
+__global__ __launch_bounds__(256) void k_spmv_up(int n_rows, const int *__restrict__ rp, const int *__restrict__ diag,
+                                                 const int *__restrict__ col, const TJ *__restrict__ val,
+                                                 const TX *__restrict__ x, double *__restrict__ T,
+                                                 const int *__restrict__ row_seg, const int *__restrict__ seg_flag,
+                                                 ActiveSet act)
+{
+  __shared__ __attribute__((aligned(16))) double red[4][648];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (!act.counts) {
+    const int row = xcd_block(blockIdx.x, gridDim.x) * 4 + wv;
+    if (row >= n_rows) return;
+    if (seg_flag && !seg_flag[row_seg[row]]) return;
+    spmv_up_row(row, lane, rp, diag, col, val, x, T, red[wv]);
+    return;
+  }
+  const int total = act.counts[2];
+  for (int gi = blockIdx.x * 4 + wv; gi < total; gi += gridDim.x * 4) {
+    const int row = active_row(act, gi);
+    if (seg_flag && !seg_flag[row_seg[row]]) continue;
+    spmv_up_row(row, lane, rp, diag, col, val, x, T, red[wv]);
+  }
+}
+
+// y_row = T[diagonal] + the slots of the row's lower blocks (lo[b]: the block
+// that block b is the transpose of); with bv, y = bv - that.  Three rows per
+// wavefront, a lane per component.
+template <typename TX>
+__device__ inline void spmv_low_row(int row, int c, const int *__restrict__ rp, const int *__restrict__ diag,
+                                    const int *__restrict__ lo, const double *__restrict__ T,
+                                    const double *__restrict__ bv, TX *__restrict__ y)
+{
+  const int b0 = rp[row], b1 = diag[row];
+  constexpr int U = 8;  // slots in flight, with the next ones' positions
+  double s = T[(size_t)b1 * 18 + c];
+  int p[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) p[u] = b0 + u < b1 ? lo[b0 + u] : 0;
+  for (int b = b0; b < b1; b += U) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = b + u < b1 ? T[(size_t)p[u] * 18 + c] : 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) p[u] = b + U + u < b1 ? lo[b + U + u] : 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += v[u];
+  }
+  const size_t i = (size_t)row * 18 + c;
+  y[i] = (TX)(bv ? bv[i] - s : s);
+}
+
+template <typename TX>
+__global__ __launch_bounds__(256) void k_spmv_low(int n_rows, const int *__restrict__ rp, const int *__restrict__ diag,
+                                                  const int *__restrict__ lo, const double *__restrict__ T,
+                                                  const double *__restrict__ bv, TX *__restrict__ y,
+                                                  const int *__restrict__ row_seg, const int *__restrict__ seg_flag,
+                                                  ActiveSet act)
+{
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane / 18, c = lane - 18 * sub;
+  if (lane >= 54) return;
+  if (!act.counts) {
+    const int row = (xcd_block(blockIdx.x, gridDim.x) * 4 + wv) * 3 + sub;
+    if (row >= n_rows || (seg_flag && !seg_flag[row_seg[row]])) return;
+    spmv_low_row(row, c, rp, diag, lo, T, bv, y);
+    return;
+  }
+  const int total = act.counts[2];
+  for (int gi = (blockIdx.x * 4 + wv) * 3 + sub; gi < total; gi += gridDim.x * 12) {
+    const int row = active_row(act, gi);
+    if (seg_flag && !seg_flag[row_seg[row]]) continue;
+    spmv_low_row(row, c, rp, diag, lo, T, bv, y);
+  }
+}
+
+// lo[b] of every block below the diagonal; bad[0] = 1 if the pattern has a
+// block without its transpose
+__global__ __launch_bounds__(256) void k_sym_map(int n_rows, const int *__restrict__ rp, const int *__restrict__ col,
+                                                 int *__restrict__ lo, int *__restrict__ bad)
+{
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= n_rows) return;
+  for (int b = rp[row] + lane; b < rp[row + 1]; b += 64) {
+    const int i = col[b];
+    int l = rp[i], h = rp[i + 1] - 1;
+    while (l < h) {
+      const int mid = (l + h) >> 1;
+      if (col[mid] < row) l = mid + 1;
+      else h = mid;
+    }
+    const bool found = l <= h && col[l] == row;
+    if (!found) bad[0] = 1;
+    lo[b] = found ? l : 0;
+  }
 }
 
 // Gauss-Jordan inverse of the 18x18 diagonal blocks with partial pivoting,
@@ -1354,6 +1540,27 @@ hipError_t launch_residual_spmv(int n_rows, const int *row_ptr, const int *col, 
   return hipGetLastError();
 }
 
+hipError_t launch_sym_map(int n_rows, const int *row_ptr, const int *col, int *lo, int *bad, hipStream_t s)
+{
+  if (n_rows <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_sym_map, dim3((n_rows + 3) / 4), dim3(256), 0, s, n_rows, row_ptr, col, lo, bad);
+  return hipGetLastError();
+}
+
+template <typename TJ, typename TX>
+hipError_t launch_spmv_sym(int n_rows, const int *row_ptr, const int *diag, const int *col, const int *lo,
+                           const TJ *val, const TX *x, const double *b, TX *y, double *T, hipStream_t s,
+                           const int *row_seg, const int *seg_flag, ActiveSet act)
+{
+  if (n_rows <= 0) return hipSuccess;
+  const int cap = act.row_cap > 0 ? act.row_cap : ACT_ROW_GRID, g4 = (n_rows + 3) / 4, g12 = (n_rows + 11) / 12;
+  hipLaunchKernelGGL((k_spmv_up<TJ, TX>), dim3(act.counts ? std::max(1, std::min(g4, cap) >> act.shift) : g4),
+                     dim3(256), 0, s, n_rows, row_ptr, diag, col, val, x, T, row_seg, seg_flag, act);
+  hipLaunchKernelGGL((k_spmv_low<TX>), dim3(act.counts ? std::max(1, std::min(g12, cap) >> act.shift) : g12),
+                     dim3(256), 0, s, n_rows, row_ptr, diag, lo, T, b, y, row_seg, seg_flag, act);
+  return hipGetLastError();
+}
+
 template <typename TJ>
 hipError_t launch_bj_invert(int n_rows, const int *diag_blk, const TJ *val, TJ *Dinv, int *status, hipStream_t s)
 {
@@ -1720,6 +1927,15 @@ template hipError_t launch_spmv<double, double>(int, const int *, const int *, c
                                                 double *, hipStream_t, const int *, const int *, ActiveSet);
 template hipError_t launch_spmv<float, float>(int, const int *, const int *, const float *, const float *, float *,
                                               hipStream_t, const int *, const int *, ActiveSet);
+template hipError_t launch_spmv_sym<double, double>(int, const int *, const int *, const int *, const int *,
+                                                    const double *, const double *, const double *, double *, double *,
+                                                    hipStream_t, const int *, const int *, ActiveSet);
+template hipError_t launch_spmv_sym<float, float>(int, const int *, const int *, const int *, const int *,
+                                                  const float *, const float *, const double *, float *, double *,
+                                                  hipStream_t, const int *, const int *, ActiveSet);
+template hipError_t launch_spmv_sym<float, double>(int, const int *, const int *, const int *, const int *,
+                                                   const float *, const double *, const double *, double *, double *,
+                                                   hipStream_t, const int *, const int *, ActiveSet);
 template hipError_t launch_residual_spmv<double>(int, const int *, const int *, const double *, const double *,
                                                  const double *, double *, hipStream_t);
 template hipError_t launch_residual_spmv<float>(int, const int *, const int *, const float *, const double *,

@@ -119,6 +119,11 @@ struct glh_ctx {
   // system matrix J and rhs
   bool constrained = false;
   int nnzb_a = 0, n_hang = 0;
+  // upper-triangle products of the assembled Jacobian: 1 usable, -1 not,
+  // 0 not looked at on this mesh
+  int sym_state = 0;
+  DBuf<int> sym_lo;
+  DBuf<double> sym_T;
   glh::ConstraintDev cons;
   DBuf<int> c_gptr, c_gsrc, c_brow, c_rptr, c_rsrc, c_hnode, c_hptr, c_hm;
   DBuf<double> c_gw, c_rw, c_hw, hdiag, rfull;
@@ -561,8 +566,37 @@ int distribute(glh_ctx *c, double *v)
   return GLH_OK;
 }
 
+// From this many blocks of the assembled matrix on the products read its upper
+// triangle (launch_spmv_sym).  A second launch costs 3 us: 1000 blocks 8.1 us
+// against 5.5 whole; 4913 (rows of up to 125) 23 against 43, 6859 9.1 against
+// 10.7.
+constexpr int SYM_MIN_BLOCKS = 4096;
+
+// the upper-triangle product's map and scratch, once per mesh; without the
+// memory for them (or on a pattern that is not symmetric) the products read
+// the whole matrix
+int ensure_sym(glh_ctx *c)
+{
+  if (c->sym_state || c->j_mf || c->nnzb < SYM_MIN_BLOCKS) return GLH_OK;
+  c->sym_state = -1;
+  if (c->sym_lo.alloc(c->nnzb) != hipSuccess || c->sym_T.alloc((size_t)c->nnzb * NC) != hipSuccess) {
+    (void)hipGetLastError();
+    c->sym_lo.release();
+    c->sym_T.release();
+    return GLH_OK;
+  }
+  HIPCHK(c, c->status.alloc(1));
+  HIPCHK(c, glh::launch_fill<int>(1, 0, c->status.p, c->stream));
+  HIPCHK(c, glh::launch_sym_map(c->n_nodes, c->row_ptr.p, c->col.p, c->sym_lo.p, c->status.p, c->stream));
+  int bad = 0;
+  HIPCHK(c, hipMemcpyAsync(&bad, c->status.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->sym_state = bad ? -1 : 1;
+  return GLH_OK;
+}
 int ensure_precond(glh_ctx *c)
 {
+  RCHK(ensure_sym(c));
   if (c->d_valid) return GLH_OK;
   HIPCHK(c, c->status.alloc(1));
   HIPCHK(c, hipMemsetAsync(c->status.p, 0, sizeof(int), c->stream));
@@ -668,8 +702,12 @@ int apply_j(glh_ctx *c, const TJ *J, const TV *x, TV *y, const int *flag, glh::A
     RCHK(mf_product<TV>(c, x, nullptr, y, flag));
     return GLH_OK;
   }
-  HIPCHK(c, glh::launch_spmv<TJ, TV>(c->n_nodes, c->row_ptr.p, c->col.p, J, x, y, c->stream, c->row_seg.p, flag,
-                                     act));
+  if (c->sym_state == 1)
+    HIPCHK(c, (glh::launch_spmv_sym<TJ, TV>(c->n_nodes, c->row_ptr.p, c->diag.p, c->col.p, c->sym_lo.p, J, x, nullptr,
+                                            y, c->sym_T.p, c->stream, c->row_seg.p, flag, act)));
+  else
+    HIPCHK(c, glh::launch_spmv<TJ, TV>(c->n_nodes, c->row_ptr.p, c->col.p, J, x, y, c->stream, c->row_seg.p, flag,
+                                       act));
   return GLH_OK;
 }
 
@@ -1089,6 +1127,9 @@ int solve_impl(glh_ctx *c, const std::vector<double> &rtolv, int maxit, int rest
       if (rc && rc != GLH_ERR_NOCONV) return rc;
       HIPCHK(c, (glh::launch_axpy<float, double>(n, 1.0, c->gx32.p, c->dU.p, s)));
       if (c->j_mf) RCHK(mf_product<double>(c, c->dU.p, c->rhs.p, c->ir_r.p));
+      else if (c->sym_state == 1)
+        HIPCHK(c, (glh::launch_spmv_sym<float, double>(c->n_nodes, c->row_ptr.p, c->diag.p, c->col.p, c->sym_lo.p,
+                                                       c->J32.p, c->dU.p, c->rhs.p, c->ir_r.p, c->sym_T.p, s)));
       else
         HIPCHK(c, glh::launch_residual_spmv<float>(c->n_nodes, c->row_ptr.p, c->col.p, c->J32.p, c->dU.p, c->rhs.p,
                                                    c->ir_r.p, s));
@@ -1223,13 +1264,13 @@ int glh_destroy(glh_ctx *c)
   DBuf<double> *dbs[] = {&c->tN,     &c->tdN,  &c->tw,   &c->tWp,  &c->tSp,   &c->tMf,   &c->tAt,   &c->cell_h,
                          &c->U,      &c->U0,   &c->dU,   &c->X,    &c->rhs,   &c->res,   &c->Fcell,
                          &c->s_norm, &c->s_alpha, &c->s_part, &c->J64, &c->D64, &c->gV64, &c->gZ64,
-                         &c->gW64,   &c->gh64, &c->gp64, &c->gy64, &c->gs64,  &c->gq64,  &c->ir_r, &c->gn64};
+                         &c->gW64,   &c->gh64, &c->gp64, &c->gy64, &c->gs64,  &c->gq64,  &c->ir_r, &c->gn64, &c->sym_T};
   for (auto *b : dbs) b->release();
   DBuf<float> *fbs[] = {&c->J32,  &c->D32,  &c->gV32, &c->gZ32, &c->gW32, &c->gh32,
                         &c->gp32, &c->gy32, &c->gs32, &c->gq32, &c->gb32, &c->gx32, &c->gn32};
   for (auto *b : fbs) b->release();
   DBuf<int> *ibs[] = {&c->tpa,      &c->tpb,         &c->cell_nodes, &c->row_ptr,  &c->col,       &c->diag,
-                      &c->cell_blk, &c->color_cells, &c->status,     &c->cell_mat, &c->seg_chunk, &c->s_flag};
+                      &c->cell_blk, &c->color_cells, &c->status,     &c->cell_mat, &c->seg_chunk, &c->s_flag, &c->sym_lo};
   for (auto *b : ibs) b->release();
   for (auto *g : {&c->graph64, &c->graph32})
     for (auto e : g->exec)
@@ -1770,6 +1811,7 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   if (c->deg != m.deg || !c->tN.p) RCHK(build_tables(c, m.deg));
   hipStream_t s = c->stream;
   drop_graphs(c);  // captured GMRES graphs refer to the previous mesh's buffers
+  c->sym_state = 0;
   c->n_cells = m.n_cells;
   c->n_nodes = m.n_nodes;
   c->nnzb = m.row_ptr.back();
@@ -1937,6 +1979,7 @@ int glh_apply_jacobian(glh_ctx *c, const double *x, double *y)
   if (!x || !y) return fail(c, GLH_ERR_ARG, "null vector");
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   const size_t n = ndofs(c);
+  RCHK(ensure_sym(c));
   HIPCHK(c, c->gW64.alloc(n));
   HIPCHK(c, c->gZ64.alloc(n));
   HIPCHK(c, hipMemcpyAsync(c->gZ64.p, x, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -2472,6 +2515,7 @@ int glh_bench_spmv(glh_ctx *c, int k, double *ms_avg)
 {
   RCHK(check_ready(c));
   if (!c->j_valid || k < 1 || !ms_avg) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
+  RCHK(ensure_sym(c));
   if (c->j_fp32) {
     HIPCHK(c, c->gW32.alloc(ndofs(c)));
     HIPCHK(c, c->gZ32.alloc(ndofs(c)));

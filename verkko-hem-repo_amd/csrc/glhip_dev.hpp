@@ -174,6 +174,16 @@ hipError_t launch_spmv(int n_rows, const int *row_ptr, const int *col, const TJ 
 template <typename TJ>
 hipError_t launch_residual_spmv(int n_rows, const int *row_ptr, const int *col, const TJ *val, const double *x,
                                 const double *b, double *r, hipStream_t s);
+// The same two products of a symmetric matrix (val(j, i) = val(i, j)^T), reading
+// its blocks from the diagonal on: y = J x, or y = b - J x when b is given.
+// diag: the rows' diagonal blocks; lo (nnzb ints, launch_sym_map): the block
+// each block is the transpose of; T: nnzb * 18 values of scratch.
+// launch_sym_map sets bad[0] = 1 if the pattern is not symmetric.
+hipError_t launch_sym_map(int n_rows, const int *row_ptr, const int *col, int *lo, int *bad, hipStream_t s);
+template <typename TJ, typename TX>
+hipError_t launch_spmv_sym(int n_rows, const int *row_ptr, const int *diag, const int *col, const int *lo,
+                           const TJ *val, const TX *x, const double *b, TX *y, double *T, hipStream_t s,
+                           const int *row_seg = nullptr, const int *seg_flag = nullptr, ActiveSet act = ActiveSet{});
 // Dinv[r] = inverse of the (symmetric) diagonal block of row r (Gauss-Jordan
 // with partial pivoting in FP64), stored as its upper triangle: 171 values
 // row-major over c <= d; status[0] set to 1 if a block is singular.
