@@ -77,3 +77,24 @@ def test_assembled_product_matches_the_oracle_cell_loop(ctx, deg, n):
     for fp32, tol in ((False, 1e-12), (True, 2e-6)):
         ctx.assemble(J=True, R=False, fp32=fp32)
         assert np.abs(ctx.apply_jacobian(x) - y).max() <= tol * np.abs(y).max()
+
+
+# one chunk of cells and several (3640 Q2 or 12300 Q1 cells each): nodes whose
+# cells lie in different chunks are written by one and added to by the others
+DIAG_CASES = [(1, (1, 1, 1)), (1, (24, 23, 23)), (2, (3, 1, 2)), (2, (11, 21, 17))]
+
+
+@pytest.mark.parametrize("deg,n", DIAG_CASES, ids=["q%d_%dx%dx%d" % (c[0], *c[1]) for c in DIAG_CASES])
+def test_matrix_free_diagonal_blocks_match_the_assembled_ones(ctx, deg, n):
+    p, t, bt = 24.0, 0.75, 2.0
+    hi = np.array([1.3, 1.1, 0.9]) * deg * np.array(n) / 2
+    mesh = G.Mesh(deg, n, -hi, hi, WALLS)
+    print("cells", mesh.n_cells, flush=True)
+    ctx.set_material_pt(p, t, bt=bt)
+    ctx.upload_mesh(mesh)
+    ctx.set_solution(initial_state(mesh.n_nodes, p, t, 0.05, 1))
+    ctx.assemble(J=True, R=False)
+    D = ctx.diagonal_blocks()
+    for fp32 in (False, True):  # the blocks are FP64 in both
+        ctx.assemble(J=True, R=False, matrix_free=True, fp32=fp32)
+        assert np.abs(ctx.diagonal_blocks() - D).max() <= 1e-12 * np.abs(D).max()

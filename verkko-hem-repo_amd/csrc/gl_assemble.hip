@@ -30,6 +30,7 @@
 #include "glhip_dev.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace glh {
@@ -516,24 +517,78 @@ __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemb
 // applied as a zero x there, Dirichlet rows keep only their diagonal
 // (k_mf_gather).
 
-// CON: a mesh with constraint lines (the hanging nodes' |local diagonal| and
-// the raw local blocks of X as well)
+// The diagonal blocks are symmetric: a cell's block of a node is its 171
+// entries c <= d, those of the parts (u, u) and (v, v) first (their Hessian
+// entries have one form, the (u, v) entries another, so that most wavefronts
+// evaluate only one).
+__device__ inline void diag_pair(int t, int &c, int &d)
+{
+  if (t >= 90) {
+    c = (t - 90) / 9;
+    d = 9 + (t - 90) % 9;
+    return;
+  }
+  const int part = t / 45;
+  int i = t - 45 * part;
+  c = 0;
+  while (i >= 9 - c) { i -= 9 - c; ++c; }
+  d = 9 * part + c + i;
+  c += 9 * part;
+}
+
+// 1D line of point values h -> sum_i w_i L_a(x_i)^2 h_i of its nodes
+template <int DEG>
+__device__ inline void square_line(double &a, double &b, double &c)
+{
+  if constexpr (DEG == 2) {
+    constexpr double t = 0.38729833462074168852;  // sqrt(3/5) / 2, the outer points' distance from the middle
+    constexpr double w = 5.0 / 18.0, p = w * (0.3 + t) * (0.3 + t), m = w * (0.3 - t) * (0.3 - t);
+    const double h0 = a, h2 = c;
+    a = p * h0 + m * h2;
+    b = (8.0 / 18.0) * b + (w * 0.16) * (h0 + h2);
+    c = m * h0 + p * h2;
+  } else {
+    constexpr double t = 0.28867513459481288225;  // 1 / (2 sqrt 3)
+    constexpr double p = 0.5 * (0.5 + t) * (0.5 + t), m = 0.5 * (0.5 - t) * (0.5 - t);
+    const double h0 = a;
+    a = p * h0 + m * b;
+    b = m * h0 + p * b;
+  }
+}
+template <int DEG>
+__device__ inline void square_lines(double *h)
+{
+  constexpr int N = DEG + 1;
+#pragma unroll
+  for (int s = 1, k = 0; k < 3; ++k, s *= N)
+#pragma unroll
+    for (int l = 0; l < N * N; ++l) {
+      const int o = (l / s) * s * N + l % s;
+      square_line<DEG>(h[o], h[o + s], h[o + (DEG == 2 ? 2 * s : s)]);
+    }
+}
+
+// One workgroup per cell of a chunk of cells: the iterate at the quadrature
+// points, and the cell's share of its nodes' diagonal blocks into slots
+// ([cell][node][171], raw: no Dirichlet rule).  A thread holds one entry's
+// Hessian at the points and contracts it with w N_a^2, a tensor product, by
+// 1D lines (162 operations instead of 729 multiply-adds in Q2).  Bound by the
+// Hessian entries' instructions and LDS reads.  Per Newton step, setup and
+// gather: 32^3 Q2 cells 10 x (114 + 39) us, against 8 colours of 280 us that
+// read and rewrote the nodes' blocks; 5586 Q2 cells FP32 2 x (95 + 30) against
+// 8 x 60; 22528 Q1 cells with hanging nodes 2 x (128 + 32) against 11 x 55.
+// CON: a mesh with constraint lines (the raw local blocks X lists as well)
 template <int DEG, typename TH, bool CON>
 __global__ __launch_bounds__(NT) void k_mf_setup(RefTables T, MeshDev Mh, Material M0, const double *__restrict__ U,
-                                                 const int *__restrict__ cells, TH *__restrict__ Uq,
-                                                 double *__restrict__ Jd, MfCondDev X)
+                                                 int e0, TH *__restrict__ Uq, double *__restrict__ slots, MfCondDev X)
 {
   constexpr int N1 = DEG + 1, NS = N1 * N1 * N1, NQ = NS;
   __shared__ double sU[NS * 18];
   __shared__ double sX[NQ * 18];
   __shared__ double sGram[NQ * GRAM];
-  // per node of the cell: global node, constraint mask, and whether this
-  // cell writes the node's diagonal block first
-  __shared__ int sNode[NS];
-  __shared__ uint32_t sMask[NS];
-  __shared__ int sFirst[NS];
+  __shared__ double sSp[NS * 9];  // the gradient products of the node pairs (a, a)
   const int tid = threadIdx.x;
-  const int e = cells[blockIdx.x];
+  const int e = e0 + blockIdx.x;
   // a finished instance of a batch keeps the iterate and blocks of its last
   // step (all of its cells are skipped together)
   if (Mh.inst_active && !Mh.inst_active[Mh.cell_inst[e]]) return;
@@ -543,13 +598,10 @@ __global__ __launch_bounds__(NT) void k_mf_setup(RefTables T, MeshDev Mh, Materi
   for (int k = 0; k < 3; ++k) { h[k] = Mh.cell_h[3 * e + k]; ih[k] = 1.0 / h[k]; }
   const double vol = h[0] * h[1] * h[2];
   const uint32_t cface = Mh.cell_face[e];
-  const int *cblk = Mh.cell_blk + (size_t)e * NS * NS;
   for (int i = tid; i < NS * 18; i += NT) sU[i] = U[(size_t)cn[i / 18] * 18 + (i % 18)];
-  if (tid < NS) {
-    const int node = cn[tid];
-    sNode[tid] = node;
-    sMask[tid] = Mh.node_mask[node];
-    sFirst[tid] = cblk[tid * NS + tid] < 0;
+  for (int i = tid; i < NS * 9; i += NT) {
+    const int a = i / 9;
+    sSp[i] = T.Sp[(size_t)(a * NS - a * (a - 1) / 2) * 9 + i % 9];
   }
   __syncthreads();
   for (int i = tid; i < NQ * 18; i += NT) {
@@ -566,89 +618,121 @@ __global__ __launch_bounds__(NT) void k_mf_setup(RefTables T, MeshDev Mh, Materi
   }
   __syncthreads();
   if (tid >= NUPAIR) return;
-  int c = 0, d = 0;
-  {
-    int t = tid;
-    while (t >= 18 - c) { t -= 18 - c; ++c; }
-    d = c + t;
-  }
+  int c, d;
+  diag_pair(tid, c, d);
   double Hv[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) Hv[q] = hess_entry(sGram + q * GRAM, sX + q * 18, c, d, M);
-  // diagonal blocks (a,a), as k_assemble forms and masks them
   const bool grad_cd = (c / 9 == d / 9) && ((c % 9) / 3 == (d % 9) / 3);
   const int kc = c % 3, kd = d % 3;
   const double lap0 = vol * ih[0] * ih[0], lap1 = vol * ih[1] * ih[1], lap2 = vol * ih[2] * ih[2];
   const double k23_cd = M.K23 * vol * ih[kc] * ih[kd];
-  const int o_cd = c * 18 + d, o_dc = d * 18 + c;
-  // entries [c][d] (v1) and [d][c] (v2) of the local block of node pair p =
-  // (a <= b), before the Dirichlet rows and columns are applied
-  auto pair_block = [&](int p, int a, int b, double &v1, double &v2) {
-    const double *wp = T.Wp + (size_t)p * NQ, *sp = T.Sp + (size_t)p * 9;
-    double sym = 0.0;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) sym += wp[q] * Hv[q];
-    sym *= vol;
+  // the gradient and Robin terms of entry [c][d] of node pair (a, b), whose
+  // gradient products are sp
+  auto edge_terms = [&](const double *sp, int a, int b) {
+    double v = 0.0;
     if (c == d) {
-      sym += M.K1 * (sp[0] * lap0 + sp[4] * lap1 + sp[8] * lap2);
+      v += M.K1 * (sp[0] * lap0 + sp[4] * lap1 + sp[8] * lap2);
       if (M.robin != 0.0)
         for (int lf = 0; lf < 6; ++lf) {
           const int bid = (int)((cface >> (3 * lf)) & 7u) - 1;
           if (bid >= 2 && bid <= 4 && !face_zeroed(bid, c))
-            sym += (M.robin * face_area(lf, h)) * T.Mf[(lf * NS + a) * NS + b];
+            v += (M.robin * face_area(lf, h)) * T.Mf[(lf * NS + a) * NS + b];
         }
     }
-    v1 = sym;
-    v2 = sym;
-    if (grad_cd) {
-      v1 += k23_cd * sp[kc * 3 + kd];
-      v2 += k23_cd * sp[kd * 3 + kc];
-    }
+    return v;
   };
-  // The nodes' blocks are updated a chunk of nodes at a time: the chunk's
-  // contributions, then all of its old values requested at once, then the
-  // stores, so that one load latency covers the chunk (the nodes of a cell
-  // are distinct, so the chunk's blocks do not overlap).
-  constexpr int AC = DEG == 1 ? 4 : 3;
-  static_assert(NS % AC == 0, "whole chunks of nodes");
-  for (int a0 = 0; a0 < NS; a0 += AC) {
-    double v1[AC], v2[AC], o1[AC], o2[AC];
-#pragma unroll
-    for (int k = 0; k < AC; ++k) {
-      const int a = a0 + k;
-      pair_block(a * NS - a * (a - 1) / 2, a, a, v1[k], v2[k]);  // pair (a, a)
-      const uint32_t ma = sMask[a];
-      // a hanging node's condensed row keeps the sum over cells of |local diagonal|
-      if (CON && c == d && (ma & HANG_BIT)) Mh.hdiag[(size_t)sNode[a] * 18 + c] += fabs(v1[k]);
-      const bool r1 = (ma >> c) & 1u, c1 = (ma >> d) & 1u, r2 = (ma >> d) & 1u, c2 = (ma >> c) & 1u;
-      if (r1 || c1) v1[k] = (r1 && c == d) ? fabs(v1[k]) : 0.0;
-      if (r2 || c2) v2[k] = (r2 && c == d) ? fabs(v2[k]) : 0.0;
-    }
-#pragma unroll
-    for (int k = 0; k < AC; ++k) {
-      const double *B = Jd + (size_t)sNode[a0 + k] * 324;
-      const bool first = sFirst[a0 + k];
-      o1[k] = first ? 0.0 : B[o_cd];
-      o2[k] = (first || c == d) ? 0.0 : B[o_dc];
-    }
-#pragma unroll
-    for (int k = 0; k < AC; ++k) {
-      double *B = Jd + (size_t)sNode[a0 + k] * 324;
-      B[o_cd] = o1[k] + v1[k];
-      if (c != d) B[o_dc] = o2[k] + v2[k];
-    }
-  }
   // constrained meshes: the raw local blocks that constraint lines fold into
   // the condensed diagonal blocks of masters (few cells have any)
   if (CON)
     for (int k = X.xptr[e]; k < X.xptr[e + 1]; ++k) {
-      const int p = X.xpair[k];
-      double v1, v2;
-      pair_block(p, T.pa[p], T.pb[p], v1, v2);
+      const int p = X.xpair[k], a = T.pa[p], b = T.pb[p];
+      const double *wp = T.Wp + (size_t)p * NQ, *sp = T.Sp + (size_t)p * 9;
+      double sym = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) sym += wp[q] * Hv[q];
+      sym = sym * vol + edge_terms(sp, a, b);
+      double v1 = sym, v2 = sym;
+      if (grad_cd) {
+        v1 += k23_cd * sp[kc * 3 + kd];
+        v2 += k23_cd * sp[kd * 3 + kc];
+      }
       double *B = X.LB + (size_t)k * 324;
-      B[o_cd] = v1;
-      if (c != d) B[o_dc] = v2;
+      B[c * 18 + d] = v1;
+      if (c != d) B[d * 18 + c] = v2;
     }
+  square_lines<DEG>(Hv);
+  double *S = slots + (size_t)blockIdx.x * NS * NUPAIR + tid;
+#pragma unroll
+  for (int a = 0; a < NS; ++a) {
+    double v = Hv[a] * vol + edge_terms(sSp + 9 * a, a, a);
+    if (grad_cd) v += k23_cd * sSp[9 * a + 3 * kc + kd];
+    S[a * NUPAIR] = v;
+  }
+}
+
+// The diagonal blocks of the nodes n0 .. n1 - 1 (a range that holds the nodes
+// of cells e0 .. e1 - 1) from their slots, in cell order: the first chunk that
+// holds a cell of the node writes its block, later ones add.  A thread sums
+// one of the 171 entries of DG nodes, 16 slots in flight; the blocks go out
+// whole through LDS.  Dirichlet rows and columns are 0 but for the sum of
+// |local diagonal|, which a hanging node also keeps in hdiag (CON).
+constexpr int DG = 4;
+template <int NS, bool CON>
+__global__ __launch_bounds__(NT) void k_mf_diag_gather(int n0, int n1, int e0, int e1,
+                                                       const int *__restrict__ n2c_ptr,
+                                                       const int *__restrict__ n2c_idx,
+                                                       const double *__restrict__ slots,
+                                                       const uint32_t *__restrict__ node_mask,
+                                                       const int *__restrict__ row_seg,
+                                                       const int *__restrict__ inst_active, double *__restrict__ Jd,
+                                                       double *__restrict__ hdiag)
+{
+  __shared__ double sB[DG][324];
+  const int tid = threadIdx.x, base = n0 + blockIdx.x * DG;
+  const int lo = e0 * NS, hi = e1 * NS;
+  int c = 0, d = 0;
+  if (tid < NUPAIR) diag_pair(tid, c, d);
+  unsigned in = 0, first = 0;  // nodes of the chunk, and those written here first
+#pragma unroll
+  for (int j = 0; j < DG; ++j) {
+    const int n = base + j;
+    if (n >= n1 || (inst_active && !inst_active[row_seg[n]])) continue;
+    const int p0 = n2c_ptr[n], p1 = n2c_ptr[n + 1];
+    if (p0 == p1 || n2c_idx[p0] >= hi || n2c_idx[p1 - 1] < lo) continue;
+    in |= 1u << j;
+    if (n2c_idx[p0] >= lo) first |= 1u << j;
+    if (tid >= NUPAIR) continue;
+    const uint32_t m = node_mask[n];
+    const bool rc = (m >> c) & 1u, rd = (m >> d) & 1u;
+    double acc = 0.0, habs = 0.0;
+    for (int p = p0; p < p1; p += 4) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = p + u < p1 ? n2c_idx[p + u] : -1;
+        v[u] = k >= lo && k < hi ? slots[(size_t)(k - lo) * NUPAIR + tid] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        acc += rc && c == d ? fabs(v[u]) : v[u];
+        if (CON) habs += fabs(v[u]);
+      }
+    }
+    if ((rc || rd) && c != d) acc = 0.0;
+    sB[j][c * 18 + d] = acc;
+    sB[j][d * 18 + c] = acc;
+    if (CON && c == d && (m & HANG_BIT)) hdiag[(size_t)n * 18 + c] += habs;
+  }
+  if (!in) return;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < DG; ++j) {
+    if (!((in >> j) & 1u)) continue;
+    double *B = Jd + (size_t)(base + j) * 324;
+    const bool f = (first >> j) & 1u;
+    for (int i = tid; i < 324; i += NT) B[i] = f ? sB[j][i] : B[i] + sB[j][i];
+  }
 }
 
 // The product in sum-factorised form: N_b(q) = L_bx(x_qx) L_by(x_qy) L_bz(x_qz),
@@ -1562,20 +1646,33 @@ hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDe
   return hipGetLastError();
 }
 
+size_t mf_setup_slots(int deg) { return (size_t)(deg == 1 ? 8 : 27) * NUPAIR; }
+
 hipError_t launch_mf_setup(int deg, bool u32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const double *U, const int *cells, int n, void *Uq, double *Jd, const MfCondDev &X,
-                           hipStream_t s)
+                           const double *U, int n_cells, int chunk, const int *node_range, const int *n2c_ptr,
+                           const int *n2c_idx, const int *row_seg, double *slots, void *Uq, double *Jd,
+                           const MfCondDev &X, hipStream_t s)
 {
-  if (n <= 0) return hipSuccess;
-  if (X.xptr && !M.hdiag) return hipErrorInvalidValue;  // the constrained setup writes hdiag
-#define GLH_MFS(D, TH, CON) \
-  hipLaunchKernelGGL((k_mf_setup<D, TH, CON>), dim3(n), dim3(NT), 0, s, T, M, mat, U, cells, (TH *)Uq, Jd, X)
+  if (n_cells <= 0) return hipSuccess;
+  if (chunk < 1 || (X.xptr && !M.hdiag)) return hipErrorInvalidValue;  // the constrained setup writes hdiag
+  for (int e0 = 0; e0 < n_cells; e0 += chunk) {
+    const int n = n_cells - e0 < chunk ? n_cells - e0 : chunk;
+    int n0 = INT_MAX, n1 = 0;
+    for (int k = e0 / MF_RANGE; k <= (e0 + n - 1) / MF_RANGE; ++k) {
+      n0 = std::min(n0, node_range[2 * k]);
+      n1 = std::max(n1, node_range[2 * k + 1]);
+    }
+#define GLH_MFS(D, TH, CON)                                                                                          \
+  hipLaunchKernelGGL((k_mf_setup<D, TH, CON>), dim3(n), dim3(NT), 0, s, T, M, mat, U, e0, (TH *)Uq, slots, X);       \
+  hipLaunchKernelGGL((k_mf_diag_gather<(D + 1) * (D + 1) * (D + 1), CON>), dim3((n1 - n0 + DG - 1) / DG), dim3(NT),  \
+                     0, s, n0, n1, e0, e0 + n, n2c_ptr, n2c_idx, slots, M.node_mask, row_seg, M.inst_active, Jd, M.hdiag)
 #define GLH_MFS2(D, TH) \
-  if (X.xptr) GLH_MFS(D, TH, true); else GLH_MFS(D, TH, false)
-  if (deg == 1) { if (u32) GLH_MFS2(1, float); else GLH_MFS2(1, double); }
-  else { if (u32) GLH_MFS2(2, float); else GLH_MFS2(2, double); }
+  if (X.xptr) { GLH_MFS(D, TH, true); } else { GLH_MFS(D, TH, false); }
+    if (deg == 1) { if (u32) { GLH_MFS2(1, float) } else { GLH_MFS2(1, double) } }
+    else { if (u32) { GLH_MFS2(2, float) } else { GLH_MFS2(2, double) } }
 #undef GLH_MFS2
 #undef GLH_MFS
+  }
   return hipGetLastError();
 }
 

@@ -93,35 +93,63 @@ __global__ __launch_bounds__(CT) void k_distribute(int n_hang, const int *__rest
 }
 
 // ------------------------------------------------ matrix-free Jacobian
-// Condensed diagonal blocks, in place: thread (t, c, d) adds to block
-// tnode[t] the weighted terms of its list (in list order), each the [c][d]
-// entry of a raw local block with the cell loop's Dirichlet rule applied
-// (row of A or column of B constrained: 0, except |v| on the diagonal of a
-// node's own (a, a) block) and the contributions through a line dropped on
-// the Dirichlet components of the master (as k_condense_j drops them).
-__global__ __launch_bounds__(CT) void k_mf_cond_diag(int n_targets, const int *__restrict__ tnode,
-                                                     const int *__restrict__ tptr, const int *__restrict__ tslot,
-                                                     const int *__restrict__ tA, const int *__restrict__ tB,
-                                                     const double *__restrict__ tw,
-                                                     const unsigned char *__restrict__ tfl,
-                                                     const uint32_t *__restrict__ mask, const double *__restrict__ LB,
-                                                     double *__restrict__ Jd)
+// Condensed diagonal blocks, in place: the workgroup of target t adds to block
+// tnode[t] the weighted terms of its list (in list order), each a raw local
+// block with the cell loop's Dirichlet rule applied (row of A or column of B
+// constrained: 0, except |v| on the diagonal of a node's own (a, a) block) and
+// the contributions through a line dropped on the Dirichlet components of the
+// master (as k_condense_j drops them).  Thread (c, d) of the block; the list
+// entries (position, weight, flags, both masks) are read by the threads
+// together, CL at a time, and the terms eight in flight: with a thread reading
+// the lists by itself a term cost a chain of four loads (305 us for an
+// adaptive slab of 22528 cells, now 110).
+constexpr int CL = 64, CNT = 384;
+__global__ __launch_bounds__(CNT) void k_mf_cond_diag(int n_targets, const int *__restrict__ tnode,
+                                                      const int *__restrict__ tptr, const int *__restrict__ tslot,
+                                                      const int *__restrict__ tA, const int *__restrict__ tB,
+                                                      const double *__restrict__ tw,
+                                                      const unsigned char *__restrict__ tfl,
+                                                      const uint32_t *__restrict__ mask, const double *__restrict__ LB,
+                                                      double *__restrict__ Jd)
 {
-  const long long i = (long long)blockIdx.x * CT + threadIdx.x;
-  if (i >= (long long)n_targets * 324) return;
-  const int t = (int)(i / 324), e = (int)(i % 324), c = e / 18, d = e % 18;
-  const int n = tnode[t];
+  __shared__ int sSlot[CL];
+  __shared__ unsigned sFl[CL];
+  __shared__ uint32_t sA[CL], sB[CL];
+  __shared__ double sW[CL];
+  const int t = blockIdx.x, e = threadIdx.x, c = e / 18, d = e % 18;
+  const int n = tnode[t], k0 = tptr[t], k1 = tptr[t + 1];
   const uint32_t mn = mask[n];
+  const bool own = e < 324, mc = (mn >> c) & 1u, md = (mn >> d) & 1u;
   double acc = 0.0;
-  for (int k = tptr[t]; k < tptr[t + 1]; ++k) {
-    const unsigned f = tfl[k];
-    if (((f & 1u) && ((mn >> c) & 1u)) || ((f & 2u) && ((mn >> d) & 1u))) continue;
-    double v = LB[(size_t)tslot[k] * 324 + ((f & 4u) ? d * 18 + c : e)];
-    const bool rA = (mask[tA[k]] >> c) & 1u, cB = (mask[tB[k]] >> d) & 1u;
-    if (rA || cB) v = ((f & 8u) && rA && c == d) ? fabs(v) : 0.0;
-    acc += tw[k] * v;
+  for (int kb = k0; kb < k1; kb += CL) {
+    const int nk = k1 - kb < CL ? k1 - kb : CL;
+    if (e < nk) {
+      sSlot[e] = tslot[kb + e];
+      sFl[e] = tfl[kb + e];
+      sW[e] = tw[kb + e];
+      sA[e] = mask[tA[kb + e]];
+      sB[e] = mask[tB[kb + e]];
+    }
+    __syncthreads();
+    if (own)
+      for (int k = 0; k < nk; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          v[u] = k + u < nk ? LB[(size_t)sSlot[k + u] * 324 + ((sFl[k + u] & 4u) ? d * 18 + c : e)] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (k + u >= nk) continue;
+          const unsigned f = sFl[k + u];
+          if (((f & 1u) && mc) || ((f & 2u) && md)) continue;
+          const bool rA = (sA[k + u] >> c) & 1u, cB = (sB[k + u] >> d) & 1u;
+          if (rA || cB) v[u] = ((f & 8u) && rA && c == d) ? fabs(v[u]) : 0.0;
+          acc += sW[k + u] * v[u];
+        }
+      }
+    __syncthreads();
   }
-  Jd[(size_t)n * 324 + e] += acc;
+  if (own) Jd[(size_t)n * 324 + e] += acc;
 }
 
 // Block n_nodes + j of the hanging node hnode[j]: its condensed row, the
@@ -297,9 +325,8 @@ hipError_t launch_mf_cond_diag(const ConstraintDev &C, const MfCondDev &X, int n
                                double *Jd, hipStream_t s)
 {
   if (X.n_targets > 0) {
-    const long long nv = (long long)X.n_targets * 324;
-    hipLaunchKernelGGL(k_mf_cond_diag, dim3((unsigned)((nv + CT - 1) / CT)), dim3(CT), 0, s, X.n_targets, X.tnode,
-                       X.tptr, X.tslot, X.tA, X.tB, X.tw, X.tfl, C.mask, X.LB, Jd);
+    hipLaunchKernelGGL(k_mf_cond_diag, dim3((unsigned)X.n_targets), dim3(CNT), 0, s, X.n_targets, X.tnode, X.tptr,
+                       X.tslot, X.tA, X.tB, X.tw, X.tfl, C.mask, X.LB, Jd);
   }
   if (C.n_hang > 0) {
     const long long nv = (long long)C.n_hang * 324;

@@ -155,7 +155,8 @@ struct glh_ctx {
   // into the masters' diagonal blocks), node -> hanging index, and the C x and
   // J C x of a product
   DBuf<int> mfx_ptr, mfx_pair, mft_node, mft_ptr, mft_slot, mft_A, mft_B, c_hidx;
-  DBuf<double> mfx_LB, mft_w, mf_xf, mf_yf;
+  DBuf<double> mfx_LB, mft_w, mf_xf, mf_yf, mf_diag;
+  std::vector<int> mf_range;  // nodes of every MF_RANGE cells (first, one past the last)
   DBuf<unsigned char> mft_fl;
   glh::MfCondDev mfc;
   size_t mfx_slots = 0;
@@ -478,11 +479,15 @@ int residual_norms(glh_ctx *c, const double *U, double *out, std::vector<double>
   return GLH_OK;
 }
 
+// values of the cells' diagonal-block shares held at a time (128 MB)
+constexpr size_t MF_SETUP_VALUES = (size_t)16 << 20;
+
 // assemble (J and/or -R) at state Ustate into (J, rhs_out)
 int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp32, double *rhs_out, bool timed,
                 bool mf = false)
 {
   void *J = nullptr;
+  int mf_chunk = 0;
   if (do_j && mf) {  // matrix-free: H at the quadrature points and the diagonal blocks
     const size_t un = (size_t)c->n_cells * c->nq * NC;
     if (fp32) HIPCHK(c, c->Uq32.alloc(un));
@@ -498,6 +503,19 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
       HIPCHK(c, c->mf_yf.alloc(ndofs(c)));
     }
     c->mf_sh_on = false;
+    // the cells' shares of the diagonal blocks, a chunk of cells at a time:
+    // large enough to fill the device, small enough to stay in the caches;
+    // smaller chunks where the memory is not to be had
+    const size_t per = glh::mf_setup_slots(c->deg);
+    const int most = std::max(1, (int)(MF_SETUP_VALUES / per)), parts = (c->n_cells + most - 1) / most;
+    mf_chunk = (c->n_cells + parts - 1) / parts;
+    hipError_t e = c->mf_diag.alloc((size_t)mf_chunk * per);
+    while (e == hipErrorOutOfMemory && mf_chunk > 1) {
+      (void)hipGetLastError();
+      mf_chunk = (mf_chunk + 1) / 2;
+      e = c->mf_diag.alloc((size_t)mf_chunk * per);
+    }
+    HIPCHK(c, e);
   } else if (do_j) {
     const size_t nv = (size_t)c->nnzb * 324;
     if (fp32) { HIPCHK(c, c->J32.alloc(nv)); J = c->J32.p; }
@@ -517,16 +535,19 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
   const glh::MeshDev M = c->meshdev();
   timed = timed || c->timing;
   if (timed) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-  const int ncol = do_j ? (int)c->color_ptr.size() - 1 : 0;
-  for (int k = 0; k < ncol; ++k) {
-    const int off = c->color_ptr[k], n = c->color_ptr[k + 1] - off;
-    if (mf)
-      HIPCHK(c, glh::launch_mf_setup(c->deg, fp32, T, M, c->mat, Ustate, c->color_cells.p + off, n,
-                                     fp32 ? (void *)c->Uq32.p : (void *)c->Uq64.p, c->Jd64.p,
-                                     c->constrained ? c->mfc : glh::MfCondDev{}, c->stream));
-    else
-      HIPCHK(c, glh::launch_assemble(c->deg, fp32, T, M, c->mat, Ustate, c->color_cells.p + off, n, Jcell,
-                                     c->stream));
+  int launches = 0;
+  if (do_j && mf) {
+    HIPCHK(c, glh::launch_mf_setup(c->deg, fp32, T, M, c->mat, Ustate, c->n_cells, mf_chunk, c->mf_range.data(),
+                                   c->n2c_ptr.p, c->n2c_idx.p, c->row_seg.p, c->mf_diag.p,
+                                   fp32 ? (void *)c->Uq32.p : (void *)c->Uq64.p, c->Jd64.p,
+                                   c->constrained ? c->mfc : glh::MfCondDev{}, c->stream));
+    launches = 2 * ((c->n_cells + mf_chunk - 1) / mf_chunk);
+  } else if (do_j) {
+    launches = (int)c->color_ptr.size() - 1;
+    for (int k = 0; k < launches; ++k) {
+      const int off = c->color_ptr[k], n = c->color_ptr[k + 1] - off;
+      HIPCHK(c, glh::launch_assemble(c->deg, fp32, T, M, c->mat, Ustate, c->color_cells.p + off, n, Jcell, c->stream));
+    }
   }
   if (c->constrained) {
     if (do_j && mf) HIPCHK(c, glh::launch_mf_cond_diag(c->cons, c->mfc, c->n_nodes, c->hdiag.p, c->Jd64.p, c->stream));
@@ -542,7 +563,7 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
     float ms = 0;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->asm_ms = ms;
-    c->asm_launches = ncol + (do_r ? 2 : 0);
+    c->asm_launches = launches + (do_r ? 2 : 0);
     if (c->timing) {
       if (do_j) { c->jasm_ms_total += ms; c->jasm_count += 1; }
       else { c->rasm_ms_total += ms; c->rasm_count += 1; }
@@ -1285,7 +1306,7 @@ int glh_destroy(glh_ctx *c)
                      &c->c_hm,    &c->c_hidx,   &c->mfx_ptr,  &c->mfx_pair, &c->mft_node, &c->mft_ptr, &c->mft_slot,
                      &c->mft_A,   &c->mft_B};
   for (auto *b : ci) b->release();
-  DBuf<double> *cd[] = {&c->c_gw, &c->c_rw, &c->c_hw, &c->hdiag, &c->rfull, &c->Jf64, &c->mfx_LB, &c->mft_w,
+  DBuf<double> *cd[] = {&c->c_gw, &c->c_rw, &c->c_hw, &c->hdiag, &c->rfull, &c->Jf64, &c->mfx_LB, &c->mft_w, &c->mf_diag,
                         &c->mf_xf, &c->mf_yf, &c->mf_sh};
   for (auto *b : cd) b->release();
   c->mft_fl.release();
@@ -1883,7 +1904,15 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   for (int sg = 0; sg < c->n_seg; ++sg) c->max_seg_chunks = std::max(c->max_seg_chunks, segch[sg + 1] - segch[sg]);
   HIPCHK(c, upload(c->cell_nodes, m.cell_nodes.data(), m.cell_nodes.size(), s));
   // node -> (cell * ns + local node) lists in cell order, for the gather of
-  // the matrix-free product
+  // the matrix-free product, and the nodes' range of every MF_RANGE cells
+  c->mf_range.clear();
+  for (int e = 0; e < m.n_cells; e += glh::MF_RANGE) {
+    const auto b = m.cell_nodes.begin() + (size_t)e * ns,
+               l = m.cell_nodes.begin() + (size_t)std::min(m.n_cells, e + glh::MF_RANGE) * ns;
+    const auto nr = std::minmax_element(b, l);
+    c->mf_range.push_back(*nr.first);
+    c->mf_range.push_back(*nr.second + 1);
+  }
   std::vector<int> n2c_ptr(m.n_nodes + 1, 0), n2c_idx(m.cell_nodes.size());
   for (int v : m.cell_nodes) ++n2c_ptr[v + 1];
   for (int i = 0; i < m.n_nodes; ++i) n2c_ptr[i + 1] += n2c_ptr[i];

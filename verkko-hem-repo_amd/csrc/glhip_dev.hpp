@@ -116,7 +116,8 @@ hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDe
 // Matrix-free Jacobian: per cell the iterate at the quadrature points (Uq:
 // [n_cells][18][NQ]; the product forms H(q) X(q) from it) and the diagonal
 // blocks (Jd: [n_nodes][324], one more per hanging node on a constrained
-// mesh), the setup colour-ordered like the assembly; the product writes
+// mesh), summed per node from the cells' shares in slots, chunk cells at a
+// time (mf_setup_slots(deg) values per cell); the product writes
 // each cell's contribution to its slot of ycell ([n_cells][NS][18]),
 // and launch_mf_gather sums them per node (node -> cell*NS + a lists, fixed
 // order) and writes the Dirichlet rows.
@@ -125,8 +126,12 @@ hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDe
 // With X.xptr set (constrained meshes) the setup also stores the raw local
 // blocks X lists and adds the |local diagonal| of hanging nodes to M.hdiag.
 hipError_t launch_mf_setup(int deg, bool u32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const double *U, const int *cells, int n, void *Uq, double *Jd, const MfCondDev &X,
-                           hipStream_t s);
+                           const double *U, int n_cells, int chunk, const int *node_range, const int *n2c_ptr,
+                           const int *n2c_idx, const int *row_seg, double *slots, void *Uq, double *Jd,
+                           const MfCondDev &X, hipStream_t s);
+size_t mf_setup_slots(int deg);
+// node_range (host): first node and one past the last of every MF_RANGE cells
+constexpr int MF_RANGE = 64;
 // flag (per instance, or null): cells and rows of instances whose flag is 0
 // are skipped, as in the batched SpMV.
 hipError_t launch_mf_apply(int deg, bool u32, bool x32, const MeshDev &M, const Material &mat, const void *Uq,
