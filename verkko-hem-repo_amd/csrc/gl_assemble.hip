@@ -225,7 +225,11 @@ __device__ inline void asm_operands(const RefTables &T, const Material &M, const
 // 44 GB of it the result: blocks shared between colours are read and written
 // again): 34.4 -> 21.3 ms FP64 (3.9 TB/s), 28.0 -> 22.8 ms FP32, against one
 // thread per component pair storing single values.
-template <typename TJ, bool HANG>
+// UP: only the blocks on and above the diagonal (the products read no
+// others): of a pair's two blocks the one whose row node is not the larger,
+// waves 0-2 the even pairs and waves 3-5 the odd ones.  Half the bytes:
+// colours of 287 cells 245 -> 182 us FP64.
+template <typename TJ, bool HANG, bool UP>
 __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, MeshDev Mh, Material M0,
                                                      const double *__restrict__ U, const int *__restrict__ cells,
                                                      TJ *__restrict__ J)
@@ -236,6 +240,7 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
   __shared__ __attribute__((aligned(16))) double S[D::LDS];
   __shared__ int sBlk[NS * NS];
   __shared__ uint32_t sMask[NS];
+  __shared__ int sNode[UP ? NS : 1];
   __shared__ uint16_t sPab[D::NTILE * 16];  // a | b << 8 of a pair, ~0 beyond the last
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int e = cells[blockIdx.x];
@@ -250,6 +255,8 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
     const int *cb = Mh.cell_blk + (size_t)e * NS * NS;
     for (int i = tid; i < NS * NS; i += D::NTH) sBlk[i] = cb[i];
     for (int i = tid; i < NS; i += D::NTH) sMask[i] = Mh.node_mask[cn[i]];
+    if (UP)
+      for (int i = tid; i < NS; i += D::NTH) sNode[i] = cn[i];
     for (int i = tid; i < D::NTILE * 16; i += D::NTH)
       sPab[i] = i < NPAIR ? (uint16_t)(T.pa[i] | (T.pb[i] << 8)) : (uint16_t)0xffff;
   }
@@ -262,7 +269,9 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
   const int pos = 64 * (tr ? w - 3 : w) + lane;
   const bool own = pos < 162;
   const int r = own ? pos / 9 : 0, c = own ? 2 * (pos % 9) : 0;
-  const int o0 = tr ? asm_col(c, r) : asm_col(r, c), o1 = tr ? asm_col(c + 1, r) : asm_col(r, c + 1);
+  const int n0 = asm_col(r, c), n1 = asm_col(r, c + 1), r0 = asm_col(c, r), r1 = asm_col(c + 1, r);
+  const int o0 = tr ? r0 : n0, o1 = tr ? r1 : n1;
+  constexpr int NP = UP ? 8 : 16;  // pairs of a tile this wave stores
   const int t0 = D::NTILE * blockIdx.y / gridDim.y, t1 = D::NTILE * (blockIdx.y + 1) / gridDim.y;
   double A[KT];
   auto load_a = [&](int t) {
@@ -273,19 +282,22 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
   for (int t = t0; t < t1; ++t) {
     // lane p < 16: block code of pair 16 t + p for this wave's orientation
     // (no block: INT_MAX), its row and column masks, and whether a == b
-    int code = 0x7fffffff, mr = 0, mc = 0, dg = -1;
-    if (lane < 16) {
-      const int ab = sPab[16 * t + lane], a = ab & 255, b = ab >> 8;
-      if (ab != 0xffff && !(tr && a == b)) {
-        code = tr ? sBlk[b * NS + a] : sBlk[a * NS + b];
-        mr = (int)sMask[tr ? b : a];
-        mc = (int)sMask[tr ? a : b];
+    // (UP: lane i < 8 pair 16 t + 2 i, or + 1, and turn its orientation)
+    int code = 0x7fffffff, mr = 0, mc = 0, dg = -1, turn = 0;
+    if (lane < NP) {
+      const int ab = sPab[16 * t + (UP ? 2 * lane + (tr ? 1 : 0) : lane)], a = ab & 255, b = ab >> 8;
+      if (ab != 0xffff && (UP || !(tr && a == b))) {
+        const bool x = UP ? sNode[a] > sNode[b] : tr;
+        code = x ? sBlk[b * NS + a] : sBlk[a * NS + b];
+        mr = (int)sMask[x ? b : a];
+        mc = (int)sMask[x ? a : b];
         dg = a == b ? a : -1;
+        turn = x;
       }
     }
-    J2 old[16];
+    J2 old[NP];
 #pragma unroll
-    for (int p = 0; p < 16; ++p) {
+    for (int p = 0; p < NP; ++p) {
       const int cd = __builtin_amdgcn_readlane(code, p);
       old[p] = J2{0, 0};
       if (cd >= 0 && cd != 0x7fffffff && own) old[p] = reinterpret_cast<const J2 *>(J + (size_t)cd * 324)[pos];
@@ -311,11 +323,13 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
       for (int q = 0; q < 4; ++q) O[(4 * q + (lane >> 4)) * TS + 16 * (w + 6 * k) + (lane & 15)] = acc[k][q];
     __syncthreads();
 #pragma unroll
-    for (int p = 0; p < 16; ++p) {
+    for (int p = 0; p < NP; ++p) {
       const int cd = __builtin_amdgcn_readlane(code, p);
       if (cd == 0x7fffffff) continue;
       const uint32_t ur = (uint32_t)__builtin_amdgcn_readlane(mr, p), uc = (uint32_t)__builtin_amdgcn_readlane(mc, p);
-      double v0 = O[p * TS + o0], v1 = O[p * TS + o1];
+      const double *row = O + (UP ? 2 * p + (tr ? 1 : 0) : p) * TS;
+      const bool x = UP && __builtin_amdgcn_readlane(turn, p);
+      double v0 = row[UP ? (x ? r0 : n0) : o0], v1 = row[UP ? (x ? r1 : n1) : o1];
       if (ur | uc) {
         const int na = __builtin_amdgcn_readlane(dg, p);  // the node of a diagonal block
         // hanging nodes (adaptive meshes): the condensed row keeps the sum
@@ -342,7 +356,8 @@ __global__ __launch_bounds__(AsmQ2::NTH, 3) void k_assemble_q2(RefTables T, Mesh
 // codes and masks of the cell sit in lanes, the old values of the next pairs
 // are on their way.  48^3 cells: 11.3 -> 7.7 ms FP64, 9.5 -> 4.4 ms FP32;
 // 8^3 cells (64 a colour): 0.37 -> 0.12 ms.
-template <typename TJ, bool HANG>
+// UP: as k_assemble_q2 (batch of 48 slabs FP32, a colour: 156 -> 129 us).
+template <typename TJ, bool HANG, bool UP>
 __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemble_q1(RefTables T, MeshDev Mh, Material M0,
                                                         const double *__restrict__ U, const int *__restrict__ cells,
                                                         TJ *__restrict__ J)
@@ -362,7 +377,11 @@ __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemb
   const bool rb = M.robin != 0.0 && cface != 0u;
   // lane l: the code of block (l / 8, l % 8), the mask of node l % 8
   const int codes = Mh.cell_blk[(size_t)e * NS * NS + lane];
-  const int masks = (int)Mh.node_mask[cn[lane & 7]];
+  const int nodes = cn[lane & 7], masks = (int)Mh.node_mask[nodes];
+  // UP: the block (a, b), or (b, a), of a pair is below the diagonal
+  const auto low = [&](int a, int b) {
+    return UP && __builtin_amdgcn_readlane(nodes, a) > __builtin_amdgcn_readlane(nodes, b);
+  };
   if (tid < NS * 18) sU[tid] = U[(size_t)cn[tid / 18] * 18 + (tid % 18)];
   for (int i = tid; i < NPAIR * 9; i += 192) sSp[i] = T.Sp[i];
   __syncthreads();
@@ -432,8 +451,8 @@ __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemb
     const int cab = __builtin_amdgcn_readlane(codes, P.a * NS + P.b),
               cba = __builtin_amdgcn_readlane(codes, P.b * NS + P.a);
     o[0] = o[1] = J2{0, 0};
-    if (cab >= 0) o[0] = reinterpret_cast<const J2 *>(J + (size_t)cab * 324)[pos];
-    if (P.a != P.b && cba >= 0) o[1] = reinterpret_cast<const J2 *>(J + (size_t)cba * 324)[pos];
+    if (cab >= 0 && !low(P.a, P.b)) o[0] = reinterpret_cast<const J2 *>(J + (size_t)cab * 324)[pos];
+    if (P.a != P.b && cba >= 0 && !low(P.b, P.a)) o[1] = reinterpret_cast<const J2 *>(J + (size_t)cba * 324)[pos];
   };
   auto store = [&](int code, const J2 &o, double v0, double v1) {
     const int blk = code < 0 ? -code - 1 : code;
@@ -493,8 +512,8 @@ __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemb
         if (rbm || ((ma >> c0) & 1u)) t0 = 0.0;
         if (rbm || ((ma >> (c0 + 1)) & 1u)) t1 = 0.0;
       }
-      store(__builtin_amdgcn_readlane(codes, a * NS + b), o0, v0, v1);
-      if (a != b) store(__builtin_amdgcn_readlane(codes, b * NS + a), o1, t0, t1);
+      if (!low(a, b)) store(__builtin_amdgcn_readlane(codes, a * NS + b), o0, v0, v1);
+      if (a != b && !low(b, a)) store(__builtin_amdgcn_readlane(codes, b * NS + a), o1, t0, t1);
     }
 }
 
@@ -1623,7 +1642,7 @@ __global__ __launch_bounds__(NT) void k_energy(RefTables T, MeshDev Mh, Material
 }  // namespace
 
 hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const double *U, const int *cells, int n, void *J, hipStream_t s)
+                           const double *U, const int *cells, int n, void *J, bool upper, hipStream_t s)
 {
   if (n <= 0) return hipSuccess;
   // a colour of few cells: the pairs of a cell go to several workgroups, which
@@ -1633,15 +1652,15 @@ hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDe
   const dim3 g(n, parts);
   // the hanging-node variant (adaptive meshes) also gathers the constrained diagonals
   const bool hang = M.hdiag != nullptr;
-#define GLH_ASM(K, TJ, HG, B) hipLaunchKernelGGL((K<TJ, HG>), g, dim3(B), 0, s, T, M, mat, U, cells, (TJ *)J)
-  if (deg == 1) {
-    if (hang) { if (jfp32) GLH_ASM(k_assemble_q1, float, true, 192); else GLH_ASM(k_assemble_q1, double, true, 192); }
-    else { if (jfp32) GLH_ASM(k_assemble_q1, float, false, 192); else GLH_ASM(k_assemble_q1, double, false, 192); }
-  } else {
-    constexpr int B = AsmQ2::NTH;
-    if (hang) { if (jfp32) GLH_ASM(k_assemble_q2, float, true, B); else GLH_ASM(k_assemble_q2, double, true, B); }
-    else { if (jfp32) GLH_ASM(k_assemble_q2, float, false, B); else GLH_ASM(k_assemble_q2, double, false, B); }
-  }
+  if (upper && hang) return hipErrorInvalidValue;  // the condensation reads both halves
+#define GLH_ASM(K, TJ, HG, UP, B) hipLaunchKernelGGL((K<TJ, HG, UP>), g, dim3(B), 0, s, T, M, mat, U, cells, (TJ *)J)
+#define GLH_ASM2(K, B)                                                                                   \
+  if (hang) { if (jfp32) GLH_ASM(K, float, true, false, B); else GLH_ASM(K, double, true, false, B); }    \
+  else if (upper) { if (jfp32) GLH_ASM(K, float, false, true, B); else GLH_ASM(K, double, false, true, B); } \
+  else { if (jfp32) GLH_ASM(K, float, false, false, B); else GLH_ASM(K, double, false, false, B); }
+  if (deg == 1) { GLH_ASM2(k_assemble_q1, 192) }
+  else { GLH_ASM2(k_assemble_q2, AsmQ2::NTH) }
+#undef GLH_ASM2
 #undef GLH_ASM
   return hipGetLastError();
 }

@@ -407,6 +407,19 @@ __global__ __launch_bounds__(256) void k_sym_map(int n_rows, const int *__restri
   }
 }
 
+// val[b] of every block below the diagonal = the transpose of block lo[b]
+template <typename TJ>
+__global__ __launch_bounds__(256) void k_sym_fill(int n_rows, const int *__restrict__ rp, const int *__restrict__ diag,
+                                                  const int *__restrict__ lo, TJ *__restrict__ val)
+{
+  const int row = blockIdx.x;
+  for (int b = rp[row]; b < diag[row]; ++b) {
+    const TJ *A = val + (size_t)lo[b] * 324;
+    TJ *B = val + (size_t)b * 324;
+    for (int i = threadIdx.x; i < 324; i += 256) B[i] = A[(i % 18) * 18 + i / 18];
+  }
+}
+
 // Gauss-Jordan inverse of the 18x18 diagonal blocks with partial pivoting,
 // in place: three nodes per wavefront, lane j of a node's 18 holding column j
 // of its block in registers.  A pivot step is one division and 17 FMAs per
@@ -1546,6 +1559,16 @@ hipError_t launch_sym_map(int n_rows, const int *row_ptr, const int *col, int *l
   hipLaunchKernelGGL(k_sym_map, dim3((n_rows + 3) / 4), dim3(256), 0, s, n_rows, row_ptr, col, lo, bad);
   return hipGetLastError();
 }
+
+template <typename TJ>
+hipError_t launch_sym_fill(int n_rows, const int *row_ptr, const int *diag, const int *lo, TJ *val, hipStream_t s)
+{
+  if (n_rows <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_sym_fill<TJ>), dim3(n_rows), dim3(256), 0, s, n_rows, row_ptr, diag, lo, val);
+  return hipGetLastError();
+}
+template hipError_t launch_sym_fill<double>(int, const int *, const int *, const int *, double *, hipStream_t);
+template hipError_t launch_sym_fill<float>(int, const int *, const int *, const int *, float *, hipStream_t);
 
 template <typename TJ, typename TX>
 hipError_t launch_spmv_sym(int n_rows, const int *row_ptr, const int *diag, const int *col, const int *lo,

@@ -122,6 +122,7 @@ struct glh_ctx {
   // upper-triangle products of the assembled Jacobian: 1 usable, -1 not,
   // 0 not looked at on this mesh
   int sym_state = 0;
+  bool j_upper = false;  // the assembled values stop at the diagonal
   DBuf<int> sym_lo;
   DBuf<double> sym_T;
   glh::ConstraintDev cons;
@@ -479,6 +480,35 @@ int residual_norms(glh_ctx *c, const double *U, double *out, std::vector<double>
   return GLH_OK;
 }
 
+// From this many blocks of the assembled matrix on the products read its upper
+// triangle (launch_spmv_sym).  A second launch costs 3 us: 1000 blocks 8.1 us
+// against 5.5 whole; 4913 (rows of up to 125) 23 against 43, 6859 9.1 against
+// 10.7.
+constexpr int SYM_MIN_BLOCKS = 4096;
+
+// the upper-triangle product's map and scratch, once per mesh, before its first
+// assembly (without constraint lines only the blocks it reads are assembled); without the
+// memory for them (or on a pattern that is not symmetric) the products read
+// the whole matrix
+int ensure_sym(glh_ctx *c)
+{
+  if (c->sym_state || c->nnzb < SYM_MIN_BLOCKS) return GLH_OK;
+  c->sym_state = -1;
+  if (c->sym_lo.alloc(c->nnzb) != hipSuccess || c->sym_T.alloc((size_t)c->nnzb * NC) != hipSuccess) {
+    (void)hipGetLastError();
+    c->sym_lo.release();
+    c->sym_T.release();
+    return GLH_OK;
+  }
+  HIPCHK(c, c->status.alloc(1));
+  HIPCHK(c, glh::launch_fill<int>(1, 0, c->status.p, c->stream));
+  HIPCHK(c, glh::launch_sym_map(c->n_nodes, c->row_ptr.p, c->col.p, c->sym_lo.p, c->status.p, c->stream));
+  int bad = 0;
+  HIPCHK(c, hipMemcpyAsync(&bad, c->status.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->sym_state = bad ? -1 : 1;
+  return GLH_OK;
+}
 // values of the cells' diagonal-block shares held at a time (128 MB)
 constexpr size_t MF_SETUP_VALUES = (size_t)16 << 20;
 
@@ -517,6 +547,7 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
     }
     HIPCHK(c, e);
   } else if (do_j) {
+    RCHK(ensure_sym(c));
     const size_t nv = (size_t)c->nnzb * 324;
     if (fp32) { HIPCHK(c, c->J32.alloc(nv)); J = c->J32.p; }
     else { HIPCHK(c, c->J64.alloc(nv)); J = c->J64.p; }
@@ -536,6 +567,7 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
   timed = timed || c->timing;
   if (timed) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   int launches = 0;
+  const bool upper = c->sym_state == 1 && !c->constrained;
   if (do_j && mf) {
     HIPCHK(c, glh::launch_mf_setup(c->deg, fp32, T, M, c->mat, Ustate, c->n_cells, mf_chunk, c->mf_range.data(),
                                    c->n2c_ptr.p, c->n2c_idx.p, c->row_seg.p, c->mf_diag.p,
@@ -544,9 +576,11 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
     launches = 2 * ((c->n_cells + mf_chunk - 1) / mf_chunk);
   } else if (do_j) {
     launches = (int)c->color_ptr.size() - 1;
+    c->j_upper = upper;
     for (int k = 0; k < launches; ++k) {
       const int off = c->color_ptr[k], n = c->color_ptr[k + 1] - off;
-      HIPCHK(c, glh::launch_assemble(c->deg, fp32, T, M, c->mat, Ustate, c->color_cells.p + off, n, Jcell, c->stream));
+      HIPCHK(c, glh::launch_assemble(c->deg, fp32, T, M, c->mat, Ustate, c->color_cells.p + off, n, Jcell, upper,
+                                     c->stream));
     }
   }
   if (c->constrained) {
@@ -587,37 +621,8 @@ int distribute(glh_ctx *c, double *v)
   return GLH_OK;
 }
 
-// From this many blocks of the assembled matrix on the products read its upper
-// triangle (launch_spmv_sym).  A second launch costs 3 us: 1000 blocks 8.1 us
-// against 5.5 whole; 4913 (rows of up to 125) 23 against 43, 6859 9.1 against
-// 10.7.
-constexpr int SYM_MIN_BLOCKS = 4096;
-
-// the upper-triangle product's map and scratch, once per mesh; without the
-// memory for them (or on a pattern that is not symmetric) the products read
-// the whole matrix
-int ensure_sym(glh_ctx *c)
-{
-  if (c->sym_state || c->j_mf || c->nnzb < SYM_MIN_BLOCKS) return GLH_OK;
-  c->sym_state = -1;
-  if (c->sym_lo.alloc(c->nnzb) != hipSuccess || c->sym_T.alloc((size_t)c->nnzb * NC) != hipSuccess) {
-    (void)hipGetLastError();
-    c->sym_lo.release();
-    c->sym_T.release();
-    return GLH_OK;
-  }
-  HIPCHK(c, c->status.alloc(1));
-  HIPCHK(c, glh::launch_fill<int>(1, 0, c->status.p, c->stream));
-  HIPCHK(c, glh::launch_sym_map(c->n_nodes, c->row_ptr.p, c->col.p, c->sym_lo.p, c->status.p, c->stream));
-  int bad = 0;
-  HIPCHK(c, hipMemcpyAsync(&bad, c->status.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->sym_state = bad ? -1 : 1;
-  return GLH_OK;
-}
 int ensure_precond(glh_ctx *c)
 {
-  RCHK(ensure_sym(c));
   if (c->d_valid) return GLH_OK;
   HIPCHK(c, c->status.alloc(1));
   HIPCHK(c, hipMemsetAsync(c->status.p, 0, sizeof(int), c->stream));
@@ -2008,7 +2013,6 @@ int glh_apply_jacobian(glh_ctx *c, const double *x, double *y)
   if (!x || !y) return fail(c, GLH_ERR_ARG, "null vector");
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   const size_t n = ndofs(c);
-  RCHK(ensure_sym(c));
   HIPCHK(c, c->gW64.alloc(n));
   HIPCHK(c, c->gZ64.alloc(n));
   HIPCHK(c, hipMemcpyAsync(c->gZ64.p, x, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -2074,6 +2078,10 @@ int glh_get_jacobian(glh_ctx *c, double *val)
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   if (c->j_mf) return fail(c, GLH_ERR_STATE, "the last Jacobian is matrix-free: no assembled values (glh_assemble)");
   const size_t nv = (size_t)c->nnzb * 324;
+  if (c->j_upper && c->j_fp32)
+    HIPCHK(c, glh::launch_sym_fill<float>(c->n_nodes, c->row_ptr.p, c->diag.p, c->sym_lo.p, c->J32.p, c->stream));
+  else if (c->j_upper)
+    HIPCHK(c, glh::launch_sym_fill<double>(c->n_nodes, c->row_ptr.p, c->diag.p, c->sym_lo.p, c->J64.p, c->stream));
   if (!c->j_fp32) {
     HIPCHK(c, hipMemcpyAsync(val, c->J64.p, nv * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2544,7 +2552,6 @@ int glh_bench_spmv(glh_ctx *c, int k, double *ms_avg)
 {
   RCHK(check_ready(c));
   if (!c->j_valid || k < 1 || !ms_avg) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
-  RCHK(ensure_sym(c));
   if (c->j_fp32) {
     HIPCHK(c, c->gW32.alloc(ndofs(c)));
     HIPCHK(c, c->gZ32.alloc(ndofs(c)));

@@ -110,9 +110,10 @@ hipError_t launch_transfer(int n_nodes, int deg, const int *cell, const float *t
 
 // ---------------------------------------------------------------- assembly
 // The Jacobian, one launch per colour; cells[] lists the cells of that
-// colour.  J: double* or float* (jfp32).
+// colour.  J: double* or float* (jfp32).  upper: only the blocks on and above
+// the diagonal (not with M.hdiag).
 hipError_t launch_assemble(int deg, bool jfp32, const RefTables &T, const MeshDev &M, const Material &mat,
-                           const double *U, const int *cells, int n, void *J, hipStream_t s);
+                           const double *U, const int *cells, int n, void *J, bool upper, hipStream_t s);
 // Matrix-free Jacobian: per cell the iterate at the quadrature points (Uq:
 // [n_cells][18][NQ]; the product forms H(q) X(q) from it) and the diagonal
 // blocks (Jd: [n_nodes][324], one more per hanging node on a constrained
@@ -185,6 +186,9 @@ hipError_t launch_residual_spmv(int n_rows, const int *row_ptr, const int *col, 
 // each block is the transpose of; T: nnzb * 18 values of scratch.
 // launch_sym_map sets bad[0] = 1 if the pattern is not symmetric.
 hipError_t launch_sym_map(int n_rows, const int *row_ptr, const int *col, int *lo, int *bad, hipStream_t s);
+// the blocks below the diagonal from those above it
+template <typename TJ>
+hipError_t launch_sym_fill(int n_rows, const int *row_ptr, const int *diag, const int *lo, TJ *val, hipStream_t s);
 template <typename TJ, typename TX>
 hipError_t launch_spmv_sym(int n_rows, const int *row_ptr, const int *diag, const int *col, const int *lo,
                            const TJ *val, const TX *x, const double *b, TX *y, double *T, hipStream_t s,
