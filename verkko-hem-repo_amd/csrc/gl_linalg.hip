@@ -515,45 +515,50 @@ __global__ __launch_bounds__(256) void k_bj_invert(int n_rows, const int *__rest
 // walking the packed index (steps 17 - d while d < c, then 1) in LDS, where
 // the node's 171 values and x of the three nodes are staged.
 template <typename TJ, typename TX>
-__device__ inline void bj_rows(int row, bool valid, int lane, const TJ *__restrict__ Dinv, const TX *__restrict__ x,
-                               TX *__restrict__ y, double *sx)
-{
-  const int sub = lane / 18, c = lane % 18;
-  if (lane < 54) sx[lane] = valid ? (double)x[(size_t)row * 18 + c] : 0.0;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // the node's 171 values staged through LDS by its 18 lanes, each load
-  // instruction covering 18 consecutive values of each node: the row walk
-  // below touches scattered entries, which from memory cost a cache-line
-  // request per lane (bit-identical; 94 -> 80 us FP64, 65 -> 39 us FP32 on
-  // the 32^3 Q2 cube)
-  TJ *sp = reinterpret_cast<TJ *>(sx + 54) + sub * 172;
-  if (lane < 54 && valid) {
+struct BjNode {  // a lane's share of its node: x and every 18th inverse entry
+  TX x;
+  TJ p[10];
+  __device__ inline void load(int row, bool valid, int lane, const TJ *__restrict__ Dinv, const TX *__restrict__ xv)
+  {
+    const int c = lane % 18;
+    x = valid ? xv[(size_t)row * 18 + c] : (TX)0;
+    // the node's 171 values staged through LDS by its 18 lanes, each load
+    // instruction covering 18 consecutive values of each node: the row walk
+    // below touches scattered entries, which from memory cost a cache-line
+    // request per lane (bit-identical; 94 -> 80 us FP64, 65 -> 39 us FP32 on
+    // the 32^3 Q2 cube)
+    if (!valid) return;
     const TJ *P = Dinv + (size_t)row * 171;
 #pragma unroll
     for (int t = 0; t < 10; ++t)
-      if (c + 18 * t < 171) sp[c + 18 * t] = P[c + 18 * t];
+      if (c + 18 * t < 171) p[t] = P[c + 18 * t];
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (lane < 54 && valid) {
-    const TJ *P = sp;
-    const double *xs = sx + sub * 18;
-    double acc = 0.0;
-    int off = c;
+  __device__ inline void apply(int row, bool valid, int lane, TX *__restrict__ y, double *sx) const
+  {
+    const int sub = lane / 18, c = lane % 18;
+    TJ *sp = reinterpret_cast<TJ *>(sx + 54) + sub * 172;
+    if (lane < 54) {
+      sx[lane] = (double)x;
+      if (valid)
 #pragma unroll
-    for (int d = 0; d < 18; ++d) {
-      acc += (double)P[off] * xs[d];
-      off += d < c ? 17 - d : 1;
+        for (int t = 0; t < 10; ++t)
+          if (c + 18 * t < 171) sp[c + 18 * t] = p[t];
     }
-    y[(size_t)row * 18 + c] = (TX)acc;
+    wave_lds_sync();
+    if (lane < 54 && valid) {
+      const double *xs = sx + sub * 18;
+      double acc = 0.0;
+      int off = c;
+#pragma unroll
+      for (int d = 0; d < 18; ++d) {
+        acc += (double)sp[off] * xs[d];
+        off += d < c ? 17 - d : 1;
+      }
+      y[(size_t)row * 18 + c] = (TX)acc;
+    }
+    wave_lds_sync();
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+};
 
 template <typename TJ, typename TX>
 __global__ __launch_bounds__(256) void k_bj_apply(int n_rows, const TJ *__restrict__ Dinv, const TX *__restrict__ x,
@@ -566,7 +571,9 @@ __global__ __launch_bounds__(256) void k_bj_apply(int n_rows, const TJ *__restri
   if (!act.counts) {
     const int row = (blockIdx.x * 4 + wv) * 3 + sub;
     const bool valid = lane < 54 && row < n_rows && live(row);
-    bj_rows(row, valid, lane, Dinv, x, y, sx[wv]);
+    BjNode<TJ, TX> N;
+    N.load(row, valid, lane, Dinv, x);
+    N.apply(row, valid, lane, y, sx[wv]);
     return;
   }
   const int total = act.counts[2];
@@ -574,7 +581,10 @@ __global__ __launch_bounds__(256) void k_bj_apply(int n_rows, const TJ *__restri
     const int gi = 3 * g + sub;
     const bool in = lane < 54 && gi < total;
     const int row = in ? active_row(act, gi) : 0;
-    bj_rows(row, in && live(row), lane, Dinv, x, y, sx[wv]);
+    const bool valid = in && live(row);
+    BjNode<TJ, TX> N;
+    N.load(row, valid, lane, Dinv, x);
+    N.apply(row, valid, lane, y, sx[wv]);
   }
 }
 
@@ -1450,12 +1460,16 @@ __global__ __launch_bounds__(RT) void k_seg_ctl2_scale(const long long *__restri
 // (cyc 0, ro 1) until the host has enqueued that pass and this kernel again
 // with resume set, which takes the second pass's partials: steps enqueued
 // ahead in the meantime find nothing to do.  status (host memory): 0 stopped,
-// 1 goes on, 2 second pass needed.
-template <typename T>
-__global__ __launch_bounds__(RT) void k_step_end(const long long *__restrict__ ch, int n_chunks,
-                                                 const T *__restrict__ partial, T *norm2, GmresCtl<T> C, int j,
-                                                 T *__restrict__ w, int resume, int *status)
+// 1 goes on, 2 second pass needed.  The normalised vector goes straight
+// through the point-block Jacobi for the next step's product (z = D^-1 v):
+// bound by reading the inverses; 15.4 + 83.7 -> 94.7 us FP64 (274625 nodes),
+// 6.4 + 10.9 -> 13.9 us FP32 (48633 nodes), against a launch for each.
+template <typename TJ, typename T>
+__global__ __launch_bounds__(RT) void k_step_end(int n_chunks, const T *__restrict__ partial, T *norm2, GmresCtl<T> C,
+                                                 int j, int n_rows, const TJ *__restrict__ Dinv, T *__restrict__ w,
+                                                 T *__restrict__ z, int resume, int *status)
 {
+  __shared__ double sx[4][54 + 3 * 172];
   __shared__ T sh[RT];
   __shared__ int s_it;
   __shared__ double s_col[128], s_cs[128], s_sn[128];  // j < m <= 126
@@ -1489,11 +1503,33 @@ __global__ __launch_bounds__(RT) void k_step_end(const long long *__restrict__ c
   }
   const T a = nrm > (T)0 ? sqrt(nrm) : (T)0;
   const T inv = a != (T)0 ? (T)1 / a : (T)1;
-  const long long beg = ch[3 * cb + 1], end = ch[3 * cb + 2];
-  for (long long i = beg + Quad<T>::N * threadIdx.x; i < end; i += Quad<T>::N * RT) {
-    auto v = ldc<false, false>(w, i, end);
-    v *= inv;
-    stc<false>(w, i, end, v);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane < 54 ? lane / 18 : 0;
+  // the next three nodes are on their way while these are applied
+  BjNode<TJ, T> N[2];
+  const long long step = gridDim.x * 4;
+  auto load = [&](BjNode<TJ, T> &B, long long g) {
+    const int row = (int)(3 * g) + sub;
+    B.load(row, lane < 54 && row < n_rows, lane, Dinv, w);
+  };
+  auto apply = [&](BjNode<TJ, T> &B, long long g) {
+    const int row = (int)(3 * g) + sub;
+    const bool valid = lane < 54 && row < n_rows;
+    B.x *= inv;
+    if (valid) w[(size_t)row * 18 + lane % 18] = B.x;
+    B.apply(row, valid, lane, z, sx[wv]);
+  };
+  long long g = blockIdx.x * 4 + wv;
+  if (3 * g >= n_rows) return;
+  load(N[0], g);
+  while (true) {
+    if (3 * (g + step) < n_rows) load(N[1], g + step);
+    apply(N[0], g);
+    g += step;
+    if (3 * g >= n_rows) break;
+    if (3 * (g + step) < n_rows) load(N[0], g + step);
+    apply(N[1], g);
+    g += step;
+    if (3 * g >= n_rows) break;
   }
 }
 
@@ -1818,13 +1854,15 @@ hipError_t launch_seg_ctl2_scale(const SegInfo &S, const T *partial, T *norm2, c
   return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_step_end(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, T *w,
-                           bool resume, int *status, hipStream_t s)
+template <typename TJ, typename T>
+hipError_t launch_step_end(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, int n_rows,
+                           const TJ *Dinv, T *w, T *z, bool resume, int *status, hipStream_t s)
 {
   if (S.n_seg != 1 || S.n_chunks <= 0 || norm2 != C.nrm2 || !status) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_step_end<T>), dim3(S.n_chunks), dim3(RT), 0, s, S.chunks, S.n_chunks, partial, norm2, C, j, w,
-                     resume ? 1 : 0, status);
+  // every workgroup sums the norm's partials: no more of them than fit the device
+  const int grid = std::min((n_rows + 11) / 12, 2048);
+  hipLaunchKernelGGL((k_step_end<TJ, T>), dim3(grid), dim3(RT), 0, s, S.n_chunks, partial, norm2, C, j, n_rows, Dinv,
+                     w, z, resume ? 1 : 0, status);
   return hipGetLastError();
 }
 
@@ -1912,8 +1950,8 @@ hipError_t launch_seg_residual(const SegInfo &S, const T *b, const T *w, T *r, T
                                                      const GmresCtl<T> *, int, int, const T *, int, bool);         \
   template hipError_t launch_seg_ctl2_scale<T>(const SegInfo &, const T *, T *, const GmresCtl<T> &, int, T *,     \
                                                hipStream_t);                                                       \
-  template hipError_t launch_step_end<T>(const SegInfo &, const T *, T *, const GmresCtl<T> &, int, T *, bool, int *, \
-                                         hipStream_t);                                                             \
+  template hipError_t launch_step_end<T, T>(const SegInfo &, const T *, T *, const GmresCtl<T> &, int, int,          \
+                                            const T *, T *, T *, bool, int *, hipStream_t);                        \
   template hipError_t launch_seg_lincomb<T>(const SegInfo &, int, const T *, size_t, const T *, int, T *,          \
                                             hipStream_t, const int *);                                             \
   template hipError_t launch_seg_scale<T>(const SegInfo &, const T *, const T *, int, T *, hipStream_t,            \

@@ -832,17 +832,20 @@ int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, i
       HIPCHK(c, glh::launch_seg_mdot<TV>(SI, j + 1, V.p, ldv, wv, pt.p, hq, ldh, 0, false, s, ro, !small));
       HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SI, j + 1, V.p, ldv, hq, ldh, wv, np, nrm2, 1, 0, s, ro, nullptr,
                                                      0, j, small ? pt.p : nullptr, small ? j + 1 : 0, false));
-      HIPCHK(c, glh::launch_step_end<TV>(SI, np, nrm2, C, j, wv, true, st, s));
+      HIPCHK(c, (glh::launch_step_end<TJ, TV>(SI, np, nrm2, C, j, c->n_nodes, Dinv, wv, Z.p, true, st, s)));
       return GLH_OK;
     }
-    TV *vj = V.p + ldv * j;
-    if (j == 0) HIPCHK(c, glh::launch_seg_scale<TV>(SI, V.p, nrm2, 1, V.p, s, cyc, true));
-    HIPCHK(c, (glh::launch_bj_apply<TJ, TV>(c->n_nodes, Dinv, vj, Z.p, s, rs, cyc, act)));
+    // Z = D^-1 V_j: of the cycle's first vector here, of the others by the
+    // end of the step that normalises them
+    if (j == 0) {
+      HIPCHK(c, glh::launch_seg_scale<TV>(SI, V.p, nrm2, 1, V.p, s, cyc, true));
+      HIPCHK(c, (glh::launch_bj_apply<TJ, TV>(c->n_nodes, Dinv, V.p, Z.p, s, rs, cyc, act)));
+    }
     RCHK(mv(Z.p, wv, cyc, act));
     HIPCHK(c, glh::launch_seg_mdot<TV>(SI, j + 2, V.p, ldv, wv, pt.p, hs, ldh, 0, false, s, cyc, !small));
     HIPCHK(c, glh::launch_seg_sub_lincomb_norm<TV>(SI, j + 1, V.p, ldv, hs, ldh, wv, np, nrm2, 1, 0, s, cyc, nullptr,
                                                    0, j, small ? pt.p : nullptr, small ? j + 2 : 0, false));
-    HIPCHK(c, glh::launch_step_end<TV>(SI, np, nrm2, C, j, wv, false, st, s));
+    HIPCHK(c, (glh::launch_step_end<TJ, TV>(SI, np, nrm2, C, j, c->n_nodes, Dinv, wv, Z.p, false, st, s)));
     return GLH_OK;
   }
   // body block: Arnoldi steps j0 <= j < j1

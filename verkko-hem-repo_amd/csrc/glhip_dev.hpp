@@ -293,12 +293,13 @@ template <typename T>
 hipError_t launch_seg_ctl2_scale(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, T *w,
                                  hipStream_t s);
 // Single instance: the norm from the first pass's chunk partials (resume: the
-// second's), op 1, op 2 and the normalisation in one launch; status (pinned
-// host memory) gets 0 stopped, 1 goes on, 2 second pass needed (the instance
-// then stands still, cyc 0 and ro 1, until that pass and a resume).
-template <typename T>
-hipError_t launch_step_end(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, T *w,
-                           bool resume, int *status, hipStream_t s);
+// second's), op 1, op 2, the normalisation of w and z = D^-1 w in one launch;
+// status (pinned host memory) gets 0 stopped, 1 goes on, 2 second pass needed
+// (the instance then stands still, cyc 0 and ro 1, until that pass and a
+// resume).
+template <typename TJ, typename T>
+hipError_t launch_step_end(const SegInfo &S, const T *partial, T *norm2, const GmresCtl<T> &C, int j, int n_rows,
+                           const TJ *Dinv, T *w, T *z, bool resume, int *status, hipStream_t s);
 // w = sum_{i < min(k, kseg[s])} y[s*ldy + i] V_i
 template <typename T>
 hipError_t launch_seg_lincomb(const SegInfo &S, int k, const T *V, size_t ldv, const T *y, int ldy, T *w,
