@@ -298,7 +298,7 @@ int glh_mlp_predict(glh_mlp *m, int64_t n, const float *X, float *Y);
 /* Uploads geometry, cell->node map, constraint masks, colour sets and the
  * BSR pattern once per refinement cycle (setup_uniform_B-phase.cc:125-198).
  * Also builds the cell->BSR scatter map used by the deterministic
- * colour-ordered assembly. */
+ * colour-ordered assembly and the node->cell lists of the gathers. */
 int glh_upload_mesh(glh_ctx *ctx, const glh_mesh *m);
 
 /* --------------------------------------------------------- solution I/O */
@@ -339,7 +339,9 @@ int glh_get_solution(glh_ctx *ctx, double *U_host);
 int glh_get_update(glh_ctx *ctx, double *dU_host);              /* locally_relevant_newton_solution */
 int glh_get_rhs(glh_ctx *ctx, double *rhs_host);                /* system_rhs (= -R) */
 /* system_matrix values in BSR order [nnzb][18][18] (FP64; an FP32 Jacobian
- * is widened).  For parity dumps of the assembled system. */
+ * is widened).  For parity dumps of the assembled system.  The blocks below
+ * the diagonal are the transposes of those above it where the products read
+ * the upper triangle. */
 int glh_get_jacobian(glh_ctx *ctx, double *val_host);
 /* y = J x with the Jacobian of the last assembly or Newton step, assembled
  * or matrix-free (FP64 vectors of n_dofs on the host).  A Jacobian-vector
@@ -441,7 +443,8 @@ int glh_last_assembly_ms(glh_ctx *ctx, double ms[2]);
  * restart <= 0 (1..126), Arnoldi steps per replayed graph block of a batch
  * (0: 8), grid caps of the active-set launches in block rows / 4 and in
  * chunks (0: 4096 / 1024), Gram-Schmidt tile (4, 8 or 16 basis vectors per
- * multi-dot workgroup and in flight per thread of the update; 0: 8). */
+ * multi-dot workgroup, twice as many loads in flight per thread of the
+ * update; 0: 8). */
 int glh_set_schedule(glh_ctx *ctx, int restart, int q_block, int row_cap, int chunk_cap, int gs_tile);
 /* Second classical Gram-Schmidt pass of GMRES for a column whose squared norm
  * after the projection falls below `ratio` times its squared norm before

@@ -531,10 +531,9 @@ __global__ __launch_bounds__(192, HANG && sizeof(TJ) == 8 ? 3 : 4) void k_assemb
 // sum-factorised, instead of streaming the cell's 729 blocks.  k_mf_setup
 // stores the iterate at the quadrature points per cell (the only state of
 // the operator besides the diagonal blocks; H(q) X(q) is formed from it in
-// the product) and assembles the diagonal blocks for the point-block Jacobi
-// preconditioner with the arithmetic of k_assemble; Dirichlet columns are
-// applied as a zero x there, Dirichlet rows keep only their diagonal
-// (k_mf_gather).
+// the product) and the cells' shares of the diagonal blocks for the
+// point-block Jacobi preconditioner; Dirichlet columns are applied as a zero x
+// in the product, Dirichlet rows keep only their diagonal (k_mf_gather).
 
 // The diagonal blocks are symmetric: a cell's block of a node is its 171
 // entries c <= d, those of the parts (u, u) and (v, v) first (their Hessian

@@ -2439,7 +2439,7 @@ int glh_autotune(glh_ctx *c, int fp32, int trial_newton, double lin_tol, int lin
   // as with 100).  The candidates leave the arithmetic as it is: the launch
   // schedule of a batch (Arnoldi steps per replayed graph block, grid caps),
   // then, with the best schedule, the Gram-Schmidt tile (basis vectors per
-  // multi-dot workgroup and in flight per update thread; every tile sums in
+  // multi-dot workgroup, loads in flight per update thread; every tile sums in
   // the same order, so the iterates are the same bits).
   const bool batch = c->n_seg > 1;
   const int m = c->tuned_restart;

@@ -19,7 +19,7 @@ struct RefTables {
   const double *Sp;   // [NPAIR*9]  sum_q w_q dN_a/dxi_k dN_b/dxi_l, index k*3+l
   const double *Mf;   // [6*NS*NS]  face mass on each unit face
   const int *pa, *pb; // [NPAIR]    pair list (a <= b)
-  const double *At;   // the pairs' tables as MFMA operands (see k_assemble): [row tile][k step][lane]
+  const double *At;   // the pairs' tables as MFMA operands (see k_assemble_q2): [row tile][k step][lane]
 };
 
 struct Material {
@@ -252,8 +252,8 @@ struct SegInfo {
   int n_chunks, n_seg;
   ActiveSet act;  // optional: only the listed instances' chunks are visited
   // Gram-Schmidt tile (4, 8 or 16): basis vectors per multi-dot workgroup,
-  // and basis vectors in flight per thread of the update.  The sums run in
-  // the same order for every tile, so the results do not depend on it.
+  // and half the 16-byte loads in flight per thread of the update.  The sums
+  // run in the same order for every tile, so the results do not depend on it.
   int gs = 8;
   // grid cap of the chunk kernels without an active set (0: one workgroup
   // per chunk): for launches that usually find their flag off (the second
