@@ -663,7 +663,7 @@ def main():
                 # the kernel waits on its LDS passes and barriers (SQ counters
                 # in profiles/matfree_cube_q2_ref5.md)
                 "peak_note": "FP64 dense peak, vector and matrix units alike",
-                "limiter": "LDS passes and barriers between them at 4 waves per SIMD"}
+                "limiter": "FP64 instructions and load latency at 2 waves per SIMD"}
     else:
         roof = spmv_roofline(apply_avg_ms)
     st0 = runs[0]
