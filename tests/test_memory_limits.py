@@ -1,0 +1,71 @@
+"""Calls that run out of device memory, and the calls after them, with the
+library's host code on hip_host.cpp's runtime (no GPU, no kernels)."""
+import pytest
+
+import hip_host
+
+NET = """
+rng = np.random.default_rng(0)
+X = rng.uniform(-1, 1, (70, 6)).astype(np.float32)
+Y = rng.standard_normal((70, 18)).astype(np.float32)
+def zeros(n):
+    return np.zeros((n, 6), np.float32), np.zeros((n, 18), np.float32)
+def trained():
+    net = G.MLP(n_freq=32, sigma=1.0, width=%d, depth=2, n_out=18, seed=1)
+    net.set_data(X, Y)
+    net.train(1, batch=128)
+    assert H.hh_bad() == 0
+    return net
+def refused(f, *a):
+    try:
+        f(*a)
+        return False
+    except G.GLHError as e:
+        assert "out of memory" in str(e), e
+        return True
+"""
+
+
+@pytest.mark.parametrize("width", [64, 320])
+def test_training_after_a_refused_gradient_takes_its_buffers_again(width):
+    # a gradient of 2^16 rows that does not get all of its buffers, for every
+    # place at which the memory can end: some of the training batch's are gone
+    # by then, so training has to take them again and capture its step anew
+    hip_host.run(NET % width + """
+for k in range(64):
+    net = trained()
+    H.hh_limit(H.hh_used() + k * (65536 * 64))
+    out = refused(net.loss_grad, *zeros(65536))
+    H.hh_limit(NO_LIMIT)
+    if not out:
+        break
+    n = H.hh_captures()
+    net.train(1, batch=128)
+    assert H.hh_bad() == 0 and H.hh_captures() == n + 1, (k, H.hh_bad(), H.hh_captures(), n)
+    net.loss_grad(X, Y)
+    net.predict(X)
+    net.train(1, batch=128)
+    assert H.hh_bad() == 0
+    net.close()
+assert k > 3, k
+""")
+
+
+@pytest.mark.parametrize("width", [64, 320])
+def test_refused_data_leaves_none_to_train_on(width):
+    hip_host.run(NET % width + """
+net = trained()
+n = 1 << 20
+for room in (0, n * 6 * 4):  # neither array, or the points alone
+    H.hh_limit(H.hh_used() + room)
+    assert refused(net.set_data, *zeros(n))
+    H.hh_limit(NO_LIMIT)
+    try:
+        net.train(1, batch=128)
+        raise AssertionError("trained on data that is gone")
+    except G.GLHError as e:
+        assert "no training data" in str(e), e
+    net.set_data(X, Y)
+    net.train(1, batch=128)
+    assert H.hh_bad() == 0
+""")

@@ -46,7 +46,11 @@ struct Buf {
     if (count <= n && p) return hipSuccess;
     release();
     hipError_t e = hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T));
-    if (e != hipSuccess) { p = nullptr; return e; }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here: the next launch would find it again
+      p = nullptr;
+      return e;
+    }
     n = count;
     return hipSuccess;
   }
@@ -112,6 +116,15 @@ int fail(glh_mlp *m, int code, const std::string &msg)
     if (rc_) return rc_; \
   } while (0)
 
+// Before buffers that a captured step or the batch's size stand for are
+// taken again: an allocation that fails has given the old one up, and nothing
+// may run on it afterwards.
+void drop_graph(glh_mlp *m)
+{
+  if (m->graph) (void)hipGraphExecDestroy(m->graph);
+  m->graph = nullptr;
+}
+
 int pack_all(glh_mlp *m)
 {
   const auto pack = m->tiled ? glh::mlp::pack_frag : glh::mlp::pack_w;
@@ -152,8 +165,6 @@ int ensure_tiled(glh_mlp *m, int nb)
   MCHK(m, m->lpart.alloc(rows / 32));
   MCHK(m, m->loss.alloc(1));
   m->nb = nb;
-  if (m->graph) (void)hipGraphExecDestroy(m->graph);
-  m->graph = nullptr;
   return GLH_OK;
 }
 
@@ -161,6 +172,8 @@ int ensure_batch(glh_mlp *m, int nb)
 {
   if (nb % 64 || nb < 64) return fail(m, GLH_ERR_ARG, "batch must be a positive multiple of 64");
   if (m->nb == nb) return GLH_OK;
+  drop_graph(m);
+  m->nb = 0;
   if (m->tiled) return ensure_tiled(m, nb);
   m->H.resize(m->depth + 1);
   m->Z.resize(m->depth);
@@ -187,8 +200,6 @@ int ensure_batch(glh_mlp *m, int nb)
   MCHK(m, m->lpart.alloc((size_t)glh::mlp::mse_blocks(nb, OUTP)));
   MCHK(m, m->loss.alloc(1));
   m->nb = nb;
-  if (m->graph) (void)hipGraphExecDestroy(m->graph);
-  m->graph = nullptr;
   return GLH_OK;
 }
 
@@ -467,7 +478,7 @@ int glh_mlp_destroy(glh_mlp *m)
   if (!m) return GLH_OK;
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
-  if (m->graph) (void)hipGraphExecDestroy(m->graph);
+  drop_graph(m);
   Buf<float> *fb[] = {&m->P, &m->G, &m->Mo, &m->Vo, &m->Bf, &m->Xall, &m->Yall, &m->Xb, &m->Yb,
                       &m->Yo, &m->part, &m->cpart, &m->lpart, &m->loss, &m->Xp, &m->Yp};
   for (auto *b : fb) b->release();
@@ -510,14 +521,14 @@ int glh_mlp_set_params(glh_mlp *m, const float *params)
 int glh_mlp_set_data(glh_mlp *m, int64_t n, const float *X, const float *Y)
 {
   if (!m || n < 1 || !X || !Y) return GLH_ERR_ARG;
+  drop_graph(m);
+  m->n_data = 0;
   MCHK(m, m->Xall.alloc((size_t)n * 6));
   MCHK(m, m->Yall.alloc((size_t)n * m->n_out));
   MCHK(m, hipMemcpyAsync(m->Xall.p, X, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, m->stream));
   MCHK(m, hipMemcpyAsync(m->Yall.p, Y, (size_t)n * m->n_out * sizeof(float), hipMemcpyHostToDevice, m->stream));
   MCHK(m, hipStreamSynchronize(m->stream));
   m->n_data = n;
-  if (m->graph) (void)hipGraphExecDestroy(m->graph);
-  m->graph = nullptr;
   return GLH_OK;
 }
 
@@ -528,8 +539,7 @@ int glh_mlp_train(glh_mlp *m, int steps, int batch, double lr, uint64_t seed, in
   RCHK(ensure_batch(m, batch));
   hipStream_t s = m->stream;
   if (!m->graph || m->graph_seed != seed || m->graph_lr != (float)lr) {
-    if (m->graph) (void)hipGraphExecDestroy(m->graph);
-    m->graph = nullptr;
+    drop_graph(m);
     hipGraph_t g = nullptr;
     MCHK(m, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     const int rc = train_step(m, seed, (float)lr);
