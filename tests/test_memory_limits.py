@@ -69,3 +69,38 @@ for room in (0, n * 6 * 4):  # neither array, or the points alone
     net.train(1, batch=128)
     assert H.hh_bad() == 0
 """)
+
+
+def test_a_refused_mesh_leaves_none():
+    # a mesh of other degree and size that does not get all of its buffers,
+    # for every place at which the memory can end
+    hip_host.run("""
+small = G.Mesh(2, (2, 2, 2), (-2, -2, -2), (2, 2, 2), [1, 1, 1, 1, 0, 0])
+large = adaptive_forest(G, (6, 6, 6), (-5, -5, -6), (5, 5, 6), [1, 1, 1, 1, 0, 0], 1, 0, frac=0.3).mesh()
+U = initial_state(small.n_nodes, 20.0, 0.5, 0.05, 1)
+ctx = G.Context(0)
+ctx.set_material_pt(20.0, 0.5)
+for k in range(4096):
+    ctx.upload_mesh(small)
+    ctx.set_solution(U)
+    ctx.assemble()
+    ctx.solve()
+    H.hh_limit(H.hh_used() + k * 2000)
+    out = False
+    try:
+        ctx.upload_mesh(large)
+    except G.GLHError as e:
+        assert "out of memory" in str(e), e
+        out = True
+    H.hh_limit(NO_LIMIT)
+    if not out:
+        break
+    for f in (lambda: ctx.assemble(), lambda: ctx.residual_norm(), lambda: ctx.set_solution(U), lambda: ctx.solve(),
+              lambda: ctx.newton_solve(), lambda: ctx.newton_step(), lambda: ctx.solution()):
+        try:
+            f()
+            raise AssertionError("a call went through without a mesh")
+        except G.GLHError as e:
+            assert "no mesh uploaded" in str(e), e
+assert k > 20, k
+""")

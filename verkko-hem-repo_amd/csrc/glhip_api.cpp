@@ -45,7 +45,11 @@ struct DBuf {
     if (count <= n && p) return hipSuccess;
     release();
     hipError_t e = hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T));
-    if (e != hipSuccess) { p = nullptr; return e; }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here: the next launch would find it again
+      p = nullptr;
+      return e;
+    }
     n = count;
     return hipSuccess;
   }
@@ -72,7 +76,11 @@ struct HBuf {
     if (count <= n && p) return hipSuccess;
     release();
     hipError_t e = hipHostMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocDefault);
-    if (e != hipSuccess) { p = nullptr; return e; }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here: the next launch would find it again
+      p = nullptr;
+      return e;
+    }
     n = count;
     return hipSuccess;
   }
@@ -315,6 +323,7 @@ void lagrange(int deg, double x, double *L, double *dL)
 int build_tables(glh_ctx *c, int deg)
 {
   const int n1 = deg + 1, ns = n1 * n1 * n1, nq = ns, npair = ns * (ns + 1) / 2;
+  c->deg = 0;  // of no degree until all of them are there
   double gx[3], gw[3], L[3][3], dL[3][3];
   gauss01(n1, gx, gw);
   for (int i = 0; i < n1; ++i) lagrange(deg, gx[i], L[i], dL[i]);
@@ -495,7 +504,6 @@ int ensure_sym(glh_ctx *c)
   if (c->sym_state || c->nnzb < SYM_MIN_BLOCKS) return GLH_OK;
   c->sym_state = -1;
   if (c->sym_lo.alloc(c->nnzb) != hipSuccess || c->sym_T.alloc((size_t)c->nnzb * NC) != hipSuccess) {
-    (void)hipGetLastError();
     c->sym_lo.release();
     c->sym_T.release();
     return GLH_OK;
@@ -541,7 +549,6 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
     mf_chunk = (c->n_cells + parts - 1) / parts;
     hipError_t e = c->mf_diag.alloc((size_t)mf_chunk * per);
     while (e == hipErrorOutOfMemory && mf_chunk > 1) {
-      (void)hipGetLastError();
       mf_chunk = (mf_chunk + 1) / 2;
       e = c->mf_diag.alloc((size_t)mf_chunk * per);
     }
@@ -1837,6 +1844,9 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   if (!c || !mm) return GLH_ERR_ARG;
   const glh::Mesh &m = mm->m;
   HIPCHK(c, hipSetDevice(c->device));
+  // until all of it is there: an allocation that fails has given up the
+  // previous mesh's buffer
+  c->have_mesh = c->j_valid = c->d_valid = false;
   if (c->deg != m.deg || !c->tN.p) RCHK(build_tables(c, m.deg));
   hipStream_t s = c->stream;
   drop_graphs(c);  // captured GMRES graphs refer to the previous mesh's buffers
@@ -1971,7 +1981,6 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   HIPCHK(c, hipMemsetAsync(c->dU.p, 0, n * sizeof(double), s));
   HIPCHK(c, hipMemsetAsync(c->rhs.p, 0, n * sizeof(double), s));
   HIPCHK(c, hipStreamSynchronize(s));
-  c->j_valid = c->d_valid = false;
   c->have_mesh = true;
   c->inst_stats.assign((size_t)c->n_seg * 8, 0.0);
   return GLH_OK;
