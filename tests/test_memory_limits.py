@@ -75,7 +75,7 @@ def test_a_refused_mesh_leaves_none():
     # a mesh of other degree and size that does not get all of its buffers,
     # for every place at which the memory can end
     hip_host.run("""
-small = G.Mesh(2, (2, 2, 2), (-2, -2, -2), (2, 2, 2), [1, 1, 1, 1, 0, 0])
+small = G.Mesh(2, (1, 1, 1), (-2, -2, -2), (2, 2, 2), [1, 1, 1, 1, 0, 0])
 large = adaptive_forest(G, (6, 6, 6), (-5, -5, -6), (5, 5, 6), [1, 1, 1, 1, 0, 0], 1, 0, frac=0.3).mesh()
 U = initial_state(small.n_nodes, 20.0, 0.5, 0.05, 1)
 ctx = G.Context(0)
@@ -104,3 +104,64 @@ for k in range(4096):
             assert "no mesh uploaded" in str(e), e
 assert k > 20, k
 """)
+
+
+@pytest.mark.parametrize("mesh", ["box", "hanging"])
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("matrix_free", [False, True])
+def test_what_fits_without_the_scratch_of_the_faster_paths_is_not_refused(mesh, fp32, matrix_free):
+    # The memory that a solve holds at its end, less the upper-triangle
+    # products' map and scratch (4 + 18 * 8 bytes a block) or, matrix-free, the
+    # setup's shares of the diagonal blocks (171 * 8 doubles a Q1 cell): with
+    # that much the same calls go through, twice, and with a block less than
+    # that they are refused for the buffers that they cannot do without.
+    hip_host.run("""
+mesh, fp32, mf = %r, %r, %r
+if mesh == "box":
+    m = G.Mesh(1, (9, 8, 7), (-4, -4, -4), (4, 4, 4), [1, 1, 1, 1, 0, 0])
+else:
+    m = adaptive_forest(G, (6, 6, 6), (-5, -5, -6), (5, 5, 6), [1, 1, 1, 1, 0, 0], 1, 0, frac=0.3).mesh()
+    assert m.constraints()["n_hanging"] > 0
+assert m.nnzb >= 4096, m.nnzb
+U = initial_state(m.n_nodes, 20.0, 0.5, 0.05, 1)
+def calls(ctx):
+    ctx.set_material_pt(20.0, 0.5)
+    ctx.upload_mesh(m)
+    ctx.set_solution(U)
+    for _ in range(2):
+        ctx.assemble(fp32=fp32, matrix_free=mf)
+        ctx.solve(rtol=1e-3, restart=100)  # a basis larger than the scratch: that is there before it
+        ctx.newton_step()
+        ctx.apply_jacobian(U)
+H.hh_limit(NO_LIMIT)
+ctx = G.Context(0)
+n0 = H.hh_used()
+calls(ctx)
+held = H.hh_used() - n0
+ctx.close()
+assert H.hh_used() <= n0
+spare = 171 * 8 * 8 * m.n_cells if mf else 148 * m.nnzb
+ctx = G.Context(0)
+fills = H.hh_launches(b"k_sym_fill")
+least = H.hh_used() + held - spare + (171 * 8 * 8 if mf else 0)  # a setup needs one cell's shares
+H.hh_limit(least)
+calls(ctx)
+whole = H.hh_launches(b"k_spmv_up")
+calls(ctx)
+assert mf or H.hh_launches(b"k_spmv_up") == whole, "upper-triangle products without their scratch"
+if not mf:
+    # the blocks below the diagonal are there for whoever reads them (in FP32
+    # the norms' zeros end the solve before its basis: the scratch stays away)
+    assert mesh == "hanging" or fp32 or H.hh_launches(b"k_sym_fill") > fills
+    n = H.hh_launches(b"k_sym_fill")
+    ctx.jacobian()
+    assert H.hh_launches(b"k_sym_fill") == n
+ctx.close()
+ctx = G.Context(0)
+H.hh_limit(least - 324 * 8)
+try:
+    calls(ctx)
+    raise AssertionError("the limit was not the least")
+except G.GLHError as e:
+    assert "out of memory" in str(e), e
+""" % (mesh, fp32, matrix_free))

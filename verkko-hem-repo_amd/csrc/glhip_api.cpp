@@ -284,10 +284,45 @@ void drop_graphs(glh_ctx *c)
     if (rc_) return rc_; \
   } while (0)
 
+// Device memory that the context holds only to be faster: the upper-triangle
+// products' map and scratch (the whole matrix serves as well, its blocks below
+// the diagonal filled in) and the matrix-free setup's shares (taken again at
+// the next setup).  Returns whether there was any to give back.
+bool give_back(glh_ctx *c)
+{
+  if (!c->mf_diag.p && !c->sym_T.p && !c->sym_lo.p) return false;
+  if (c->sym_state == 1) {
+    hipError_t e = hipSuccess;
+    if (c->j_valid && !c->j_mf && c->j_upper && c->j_fp32)
+      e = glh::launch_sym_fill<float>(c->n_nodes, c->row_ptr.p, c->diag.p, c->sym_lo.p, c->J32.p, c->stream);
+    else if (c->j_valid && !c->j_mf && c->j_upper)
+      e = glh::launch_sym_fill<double>(c->n_nodes, c->row_ptr.p, c->diag.p, c->sym_lo.p, c->J64.p, c->stream);
+    if (e != hipSuccess) return false;
+    c->j_upper = false;
+    c->sym_state = -1;
+  }
+  if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+  drop_graphs(c);  // the recorded products read the scratch
+  c->mf_diag.release();
+  c->sym_T.release();
+  c->sym_lo.release();
+  return true;
+}
+
+// n values of device memory for b, which may be had by giving those back: what
+// fits the card without them does not fail for them
 template <typename T>
-hipError_t upload(DBuf<T> &b, const T *src, size_t n, hipStream_t s)
+hipError_t take(glh_ctx *c, DBuf<T> &b, size_t n)
 {
   hipError_t e = b.alloc(n);
+  if (e == hipErrorOutOfMemory && give_back(c)) e = b.alloc(n);
+  return e;
+}
+
+template <typename T>
+hipError_t upload(glh_ctx *c, DBuf<T> &b, const T *src, size_t n, hipStream_t s)
+{
+  hipError_t e = take(c, b, n);
   if (e != hipSuccess) return e;
   if (n == 0) return hipSuccess;
   return hipMemcpyAsync(b.p, src, n * sizeof(T), hipMemcpyHostToDevice, s);
@@ -375,14 +410,14 @@ int build_tables(glh_ctx *c, int deg)
       }
   }
   hipStream_t s = c->stream;
-  HIPCHK(c, upload(c->tN, N.data(), N.size(), s));
-  HIPCHK(c, upload(c->tdN, dN.data(), dN.size(), s));
-  HIPCHK(c, upload(c->tw, w.data(), w.size(), s));
-  HIPCHK(c, upload(c->tWp, Wp.data(), Wp.size(), s));
-  HIPCHK(c, upload(c->tSp, Sp.data(), Sp.size(), s));
-  HIPCHK(c, upload(c->tMf, Mf.data(), Mf.size(), s));
-  HIPCHK(c, upload(c->tpa, pa.data(), pa.size(), s));
-  HIPCHK(c, upload(c->tpb, pb.data(), pb.size(), s));
+  HIPCHK(c, upload(c, c->tN, N.data(), N.size(), s));
+  HIPCHK(c, upload(c, c->tdN, dN.data(), dN.size(), s));
+  HIPCHK(c, upload(c, c->tw, w.data(), w.size(), s));
+  HIPCHK(c, upload(c, c->tWp, Wp.data(), Wp.size(), s));
+  HIPCHK(c, upload(c, c->tSp, Sp.data(), Sp.size(), s));
+  HIPCHK(c, upload(c, c->tMf, Mf.data(), Mf.size(), s));
+  HIPCHK(c, upload(c, c->tpa, pa.data(), pa.size(), s));
+  HIPCHK(c, upload(c, c->tpb, pb.data(), pb.size(), s));
   // the pair tables as matrix-core operands: row tile t, k step s, lane l hold
   // pair 16 t + l % 16 and k = 4 s + l / 16 (points, derivative pairs, faces)
   // (Q2; the Q1 assembly reads the pair tables themselves)
@@ -399,7 +434,7 @@ int build_tables(glh_ctx *c, int deg)
         else if (k < nq + 15) v = Mf[((size_t)(k - nq - 9) * ns + pa[pr]) * ns + pb[pr]];
         At[((size_t)t * kt + k4) * 64 + l] = v;
       }
-  HIPCHK(c, upload(c->tAt, At.data(), At.size(), s));
+  HIPCHK(c, upload(c, c->tAt, At.data(), At.size(), s));
   HIPCHK(c, hipStreamSynchronize(s));
   c->deg = deg; c->ns = ns; c->nq = nq; c->npair = npair;
   return GLH_OK;
@@ -424,8 +459,8 @@ size_t basis_stride(const glh_ctx *c) { return (ndofs(c) + 3) / 4 * 4; }
 int seg_norm2(glh_ctx *c, const double *v, std::vector<double> &out)
 {
   const size_t n = ndofs(c);
-  HIPCHK(c, c->s_part.alloc((size_t)std::max(1, c->n_chunks)));
-  HIPCHK(c, c->s_norm.alloc(c->n_seg));
+  HIPCHK(c, take(c, c->s_part, (size_t)std::max(1, c->n_chunks)));
+  HIPCHK(c, take(c, c->s_norm, c->n_seg));
   HIPCHK(c, c->pinv.alloc(c->n_seg));
   HIPCHK(c, glh::launch_seg_mdot<double>(c->seg(), 1, v, n, v, c->s_part.p, c->s_norm.p, 1, 0, false, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->pinv.p, c->s_norm.p, c->n_seg * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -469,8 +504,8 @@ int residual_cells(glh_ctx *c, const double *U, double *out, double *part = null
 // -R at U into out and its per-instance ||R_s||^2 on the host
 int residual_norms(glh_ctx *c, const double *U, double *out, std::vector<double> &n2)
 {
-  HIPCHK(c, c->s_part.alloc((size_t)std::max(1, c->n_chunks)));
-  HIPCHK(c, c->s_norm.alloc(c->n_seg));
+  HIPCHK(c, take(c, c->s_part, (size_t)std::max(1, c->n_chunks)));
+  HIPCHK(c, take(c, c->s_norm, c->n_seg));
   HIPCHK(c, c->pinv.alloc(c->n_seg));
   if (c->timing) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   RCHK(residual_cells(c, U, out, c->s_part.p, c->s_norm.p));
@@ -495,20 +530,20 @@ int residual_norms(glh_ctx *c, const double *U, double *out, std::vector<double>
 // 10.7.
 constexpr int SYM_MIN_BLOCKS = 4096;
 
-// the upper-triangle product's map and scratch, once per mesh, before its first
-// assembly (without constraint lines only the blocks it reads are assembled); without the
-// memory for them (or on a pattern that is not symmetric) the products read
-// the whole matrix
+// the upper-triangle product's map and scratch, once per mesh, at its first
+// assembly (without constraint lines only the blocks it reads are assembled);
+// without the memory for them, here or for what is taken later (give_back), or
+// on a pattern that is not symmetric, the products read the whole matrix
 int ensure_sym(glh_ctx *c)
 {
   if (c->sym_state || c->nnzb < SYM_MIN_BLOCKS) return GLH_OK;
+  HIPCHK(c, take(c, c->status, 1));  // (may give back what the scratch held on the last mesh)
   c->sym_state = -1;
   if (c->sym_lo.alloc(c->nnzb) != hipSuccess || c->sym_T.alloc((size_t)c->nnzb * NC) != hipSuccess) {
     c->sym_lo.release();
     c->sym_T.release();
     return GLH_OK;
   }
-  HIPCHK(c, c->status.alloc(1));
   HIPCHK(c, glh::launch_fill<int>(1, 0, c->status.p, c->stream));
   HIPCHK(c, glh::launch_sym_map(c->n_nodes, c->row_ptr.p, c->col.p, c->sym_lo.p, c->status.p, c->stream));
   int bad = 0;
@@ -528,17 +563,17 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
   int mf_chunk = 0;
   if (do_j && mf) {  // matrix-free: H at the quadrature points and the diagonal blocks
     const size_t un = (size_t)c->n_cells * c->nq * NC;
-    if (fp32) HIPCHK(c, c->Uq32.alloc(un));
-    else HIPCHK(c, c->Uq64.alloc(un));
-    HIPCHK(c, c->mf_ycell.alloc((size_t)c->n_cells * c->ns * NC));
+    if (fp32) HIPCHK(c, take(c, c->Uq32, un));
+    else HIPCHK(c, take(c, c->Uq64, un));
+    HIPCHK(c, take(c, c->mf_ycell, (size_t)c->n_cells * c->ns * NC));
     // one block per node, and on a constrained mesh one more per hanging node
     // (its condensed row for the point-block Jacobi, diag_id points there)
-    HIPCHK(c, c->Jd64.alloc(((size_t)c->n_nodes + (c->constrained ? c->n_hang : 0)) * 324));
+    HIPCHK(c, take(c, c->Jd64, ((size_t)c->n_nodes + (c->constrained ? c->n_hang : 0)) * 324));
     if (c->constrained) {
-      HIPCHK(c, c->mfx_LB.alloc(c->mfx_slots * 324));
+      HIPCHK(c, take(c, c->mfx_LB, c->mfx_slots * 324));
       c->mfc.LB = c->mfx_LB.p;
-      HIPCHK(c, c->mf_xf.alloc(ndofs(c)));
-      HIPCHK(c, c->mf_yf.alloc(ndofs(c)));
+      HIPCHK(c, take(c, c->mf_xf, ndofs(c)));
+      HIPCHK(c, take(c, c->mf_yf, ndofs(c)));
     }
     c->mf_sh_on = false;
     // the cells' shares of the diagonal blocks, a chunk of cells at a time:
@@ -547,28 +582,28 @@ int assemble_at(glh_ctx *c, const double *Ustate, bool do_j, bool do_r, bool fp3
     const size_t per = glh::mf_setup_slots(c->deg);
     const int most = std::max(1, (int)(MF_SETUP_VALUES / per)), parts = (c->n_cells + most - 1) / most;
     mf_chunk = (c->n_cells + parts - 1) / parts;
-    hipError_t e = c->mf_diag.alloc((size_t)mf_chunk * per);
+    hipError_t e = take(c, c->mf_diag, (size_t)mf_chunk * per);
     while (e == hipErrorOutOfMemory && mf_chunk > 1) {
       mf_chunk = (mf_chunk + 1) / 2;
       e = c->mf_diag.alloc((size_t)mf_chunk * per);
     }
     HIPCHK(c, e);
   } else if (do_j) {
-    RCHK(ensure_sym(c));
     const size_t nv = (size_t)c->nnzb * 324;
-    if (fp32) { HIPCHK(c, c->J32.alloc(nv)); J = c->J32.p; }
-    else { HIPCHK(c, c->J64.alloc(nv)); J = c->J64.p; }
+    if (fp32) { HIPCHK(c, take(c, c->J32, nv)); J = c->J32.p; }
+    else { HIPCHK(c, take(c, c->J64, nv)); J = c->J64.p; }
   }
   // with hanging nodes the cell loop writes Jf, condensed afterwards
   void *Jcell = J;
   if (c->constrained) {
     if (do_j && !mf) {
       const size_t nv = (size_t)c->nnzb_a * 324;
-      if (fp32) { HIPCHK(c, c->Jf32.alloc(nv)); Jcell = c->Jf32.p; }
-      else { HIPCHK(c, c->Jf64.alloc(nv)); Jcell = c->Jf64.p; }
+      if (fp32) { HIPCHK(c, take(c, c->Jf32, nv)); Jcell = c->Jf32.p; }
+      else { HIPCHK(c, take(c, c->Jf64, nv)); Jcell = c->Jf64.p; }
     }
     if (do_j) HIPCHK(c, glh::launch_fill<double>(ndofs(c), 0.0, c->hdiag.p, c->stream));
   }
+  if (do_j && !mf) RCHK(ensure_sym(c));  // after the matrix, which comes first where the memory is short
   const glh::RefTables T = c->tables();
   const glh::MeshDev M = c->meshdev();
   timed = timed || c->timing;
@@ -631,19 +666,19 @@ int distribute(glh_ctx *c, double *v)
 int ensure_precond(glh_ctx *c)
 {
   if (c->d_valid) return GLH_OK;
-  HIPCHK(c, c->status.alloc(1));
+  HIPCHK(c, take(c, c->status, 1));
   HIPCHK(c, hipMemsetAsync(c->status.p, 0, sizeof(int), c->stream));
   const size_t nv = (size_t)c->n_nodes * 171;  // the inverses' upper triangles
   if (c->j_fp32 && c->j_mf) {  // FP64 inverses of the FP64 diagonal blocks, rounded to FP32
-    HIPCHK(c, c->D64.alloc(nv));
-    HIPCHK(c, c->D32.alloc(nv));
+    HIPCHK(c, take(c, c->D64, nv));
+    HIPCHK(c, take(c, c->D32, nv));
     HIPCHK(c, glh::launch_bj_invert<double>(c->n_nodes, c->diag_id.p, c->Jd64.p, c->D64.p, c->status.p, c->stream));
     HIPCHK(c, (glh::launch_convert<double, float>(nv, c->D64.p, c->D32.p, c->stream)));
   } else if (c->j_fp32) {
-    HIPCHK(c, c->D32.alloc(nv));
+    HIPCHK(c, take(c, c->D32, nv));
     HIPCHK(c, glh::launch_bj_invert<float>(c->n_nodes, c->diag.p, c->J32.p, c->D32.p, c->status.p, c->stream));
   } else {
-    HIPCHK(c, c->D64.alloc(nv));
+    HIPCHK(c, take(c, c->D64, nv));
     if (c->j_mf)
       HIPCHK(c, glh::launch_bj_invert<double>(c->n_nodes, c->diag_id.p, c->Jd64.p, c->D64.p, c->status.p, c->stream));
     else
@@ -914,32 +949,32 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   auto &pt = Work<TV>::part(c);
   auto &yb = Work<TV>::y(c);
   auto &sc = Work<TV>::sc(c);
-  HIPCHK(c, V.alloc(basis_stride(c) * (m + 1)));
-  HIPCHK(c, Z.alloc(n));
-  HIPCHK(c, W.alloc(n));
-  HIPCHK(c, hs.alloc((size_t)S * ldh));
-  HIPCHK(c, hq.alloc((size_t)S * ldh));
-  HIPCHK(c, yb.alloc((size_t)S * ldh));
-  HIPCHK(c, sc.alloc((size_t)S * 2));
-  HIPCHK(c, pt.alloc((size_t)std::max(1, c->n_chunks) * (m + 2)));
-  HIPCHK(c, Work<TV>::npart(c).alloc((size_t)std::max(1, c->n_chunks)));
-  HIPCHK(c, c->gmH.alloc((size_t)S * (m + 1) * m));
-  HIPCHK(c, c->gmcs.alloc((size_t)S * m));
-  HIPCHK(c, c->gmsn.alloc((size_t)S * m));
-  HIPCHK(c, c->gmg.alloc((size_t)S * (m + 1)));
-  HIPCHK(c, c->gmbeta.alloc(S));
-  HIPCHK(c, c->gmtarget.alloc(S));
+  HIPCHK(c, take(c, V, basis_stride(c) * (m + 1)));
+  HIPCHK(c, take(c, Z, n));
+  HIPCHK(c, take(c, W, n));
+  HIPCHK(c, take(c, hs, (size_t)S * ldh));
+  HIPCHK(c, take(c, hq, (size_t)S * ldh));
+  HIPCHK(c, take(c, yb, (size_t)S * ldh));
+  HIPCHK(c, take(c, sc, (size_t)S * 2));
+  HIPCHK(c, take(c, pt, (size_t)std::max(1, c->n_chunks) * (m + 2)));
+  HIPCHK(c, take(c, Work<TV>::npart(c), (size_t)std::max(1, c->n_chunks)));
+  HIPCHK(c, take(c, c->gmH, (size_t)S * (m + 1) * m));
+  HIPCHK(c, take(c, c->gmcs, (size_t)S * m));
+  HIPCHK(c, take(c, c->gmsn, (size_t)S * m));
+  HIPCHK(c, take(c, c->gmg, (size_t)S * (m + 1)));
+  HIPCHK(c, take(c, c->gmbeta, S));
+  HIPCHK(c, take(c, c->gmtarget, S));
   DBuf<int> *ib[] = {&c->gmcyc, &c->gmconv, &c->gmjseg, &c->gmits, &c->gmro, &c->gmfrozen, &c->gmjlast};
-  for (auto *q : ib) HIPCHK(c, q->alloc(S));
+  for (auto *q : ib) HIPCHK(c, take(c, *q, S));
   HIPCHK(c, c->pinv.alloc((size_t)4 * S));
-  HIPCHK(c, c->act_counts.alloc(4));
+  HIPCHK(c, take(c, c->act_counts, 4));
   // every host <-> device copy of the loop below goes through pinned memory
   HIPCHK(c, c->pin_i.alloc(2 * (size_t)S + 4));
   HIPCHK(c, c->pin_st.alloc(128));
   HIPCHK(c, Work<TV>::pin(c).alloc(S));
-  HIPCHK(c, c->act_seg.alloc(S));
-  HIPCHK(c, c->act_rpref.alloc(S + 1));
-  HIPCHK(c, c->act_chunk.alloc(std::max(1, c->n_chunks)));
+  HIPCHK(c, take(c, c->act_seg, S));
+  HIPCHK(c, take(c, c->act_rpref, S + 1));
+  HIPCHK(c, take(c, c->act_chunk, std::max(1, c->n_chunks)));
   glh::GmresCtl<TV> C{S,        m,          ldh,        hs.p,         hq.p,         sc.p,        yb.p,
                       c->gmH.p, c->gmcs.p,  c->gmsn.p,  c->gmg.p,     c->gmbeta.p,  c->gmtarget.p, c->gmcyc.p,
                       c->gmconv.p, c->gmjseg.p, c->gmits.p, c->gmro.p, c->gmfrozen.p, c->gmjlast.p,
@@ -972,7 +1007,8 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   const int nblk = (m + q - 1) / q;
   constexpr int NLEV = 3;
   auto &gc = Work<TV>::graph(c);
-  // every buffer and size the captured launches use
+  // The buffers and sizes the captured launches use and the product they run,
+  // beside what an upload sets (it drops the graphs).
   const std::vector<const void *> key = {J,           Dinv,          b,           x,            V.p,
                                          Z.p,         W.p,           pt.p,        hs.p,         hq.p, Work<TV>::npart(c).p,
                                          yb.p,        sc.p,          c->gmH.p,    c->gmcs.p,    c->gmsn.p,
@@ -980,7 +1016,9 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
                                          c->gmjseg.p, c->gmits.p,    c->gmro.p,   c->gmfrozen.p, c->gmjlast.p,
                                          c->row_seg.p, c->d_node_off.p, c->act_counts.p, c->act_seg.p,
                                          c->act_rpref.p, c->act_chunk.p, c->chunks.p, c->seg_chunk.p,
-                                         c->row_ptr.p, c->col.p, c->Uq64.p, c->Uq32.p, c->Jd64.p,
+                                         c->row_ptr.p, c->col.p, c->diag.p, c->sym_lo.p, c->sym_T.p,
+                                         (const void *)(size_t)(c->sym_state == 1), c->pin_st.p,
+                                         c->Uq64.p, c->Uq32.p, c->Jd64.p,
                                          c->mf_xf.p, c->mf_yf.p, c->mf_sh_on ? c->mf_sh.p : nullptr,
                                          (const void *)(size_t)c->j_mf,
                                          (const void *)(size_t)m, (const void *)(size_t)S,
@@ -1128,10 +1166,10 @@ int solve_impl(glh_ctx *c, const std::vector<double> &rtolv, int maxit, int rest
   } else {
     // FP32 GMRES inside FP64 iterative refinement, per instance:
     //   r = rhs - J32 dU (FP64 arithmetic), solve J32 c = r in FP32, dU += c
-    HIPCHK(c, c->gb32.alloc(n));
-    HIPCHK(c, c->gx32.alloc(n));
-    HIPCHK(c, c->ir_r.alloc(n));
-    HIPCHK(c, c->s_flag.alloc(S));
+    HIPCHK(c, take(c, c->gb32, n));
+    HIPCHK(c, take(c, c->gx32, n));
+    HIPCHK(c, take(c, c->ir_r, n));
+    HIPCHK(c, take(c, c->s_flag, S));
     HIPCHK(c, hipMemsetAsync(c->dU.p, 0, n * sizeof(double), s));
     std::vector<double> bn2, rn2;
     RCHK(seg_norm2(c, c->rhs.p, bn2));
@@ -1206,7 +1244,7 @@ int newton_step_impl(glh_ctx *c, double step, int damped, const std::vector<char
   alpha.assign(S, 0.0);
   trials.assign(S, 0);
   for (int i = 0; i < S; ++i) acc[i] = !active[i];
-  HIPCHK(c, c->s_alpha.alloc(S));
+  HIPCHK(c, take(c, c->s_alpha, S));
   HIPCHK(c, c->pinv.alloc(S));
   const int n_try = damped ? 100 : 1;
   cur.assign(S, 0.0);
@@ -1377,7 +1415,7 @@ int glh_set_materials(glh_ctx *c, int n_inst, const double *coef)
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   drop_graphs(c);  // recorded products read the old materials (and possibly the old buffer)
-  HIPCHK(c, upload(c->mats, ms.data(), ms.size(), c->stream));
+  HIPCHK(c, upload(c, c->mats, ms.data(), ms.size(), c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->mats_host = ms;
   c->mat = ms[0];
@@ -1567,8 +1605,8 @@ int glh_transfer_solution(glh_ctx *c, const glh_forest *fo, const glh_mesh *mo, 
     dt.release();
   };
   const size_t no = (size_t)mo->m.n_nodes * NC, nco = (size_t)mo->m.n_cells * mo->m.ns;
-  hipError_t e = Uo.alloc(no);
-  if (e == hipSuccess) e = cno.alloc(nco);
+  hipError_t e = take(c, Uo, no);
+  if (e == hipSuccess) e = take(c, cno, nco);
   if (e == hipSuccess) e = hipMemcpyAsync(Uo.p, c->U.p, no * sizeof(double), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(cno.p, c->cell_nodes.p, nco * sizeof(int), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1581,8 +1619,8 @@ int glh_transfer_solution(glh_ctx *c, const glh_forest *fo, const glh_mesh *mo, 
     release();
     return rc;
   }
-  e = upload(dcell, cell.data(), cell.size(), s);
-  if (e == hipSuccess) e = upload(dt, t.data(), t.size(), s);
+  e = upload(c, dcell, cell.data(), cell.size(), s);
+  if (e == hipSuccess) e = upload(c, dt, t.data(), t.size(), s);
   if (e == hipSuccess) e = glh::launch_transfer(mn->m.n_nodes, mn->m.deg, dcell.p, dt.p, cno.p, Uo.p, c->U.p, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   release();
@@ -1741,25 +1779,25 @@ int upload_constraints(glh_ctx *c, const glh::Mesh &m, const std::vector<int> &d
     }
     rptr[r + 1] = (int)rsrc.size();
   }
-  HIPCHK(c, upload(c->c_gptr, gptr.data(), gptr.size(), s));
-  HIPCHK(c, upload(c->c_gsrc, gsrc.data(), gsrc.size(), s));
-  HIPCHK(c, upload(c->c_gw, gw.data(), gw.size(), s));
-  HIPCHK(c, upload(c->c_gfl, gfl.data(), gfl.size(), s));
-  HIPCHK(c, upload(c->c_brow, brow.data(), brow.size(), s));
-  HIPCHK(c, upload(c->c_rptr, rptr.data(), rptr.size(), s));
-  HIPCHK(c, upload(c->c_rsrc, rsrc.data(), rsrc.size(), s));
-  HIPCHK(c, upload(c->c_rw, rw.data(), rw.size(), s));
-  HIPCHK(c, upload(c->c_rfl, rfl.data(), rfl.size(), s));
+  HIPCHK(c, upload(c, c->c_gptr, gptr.data(), gptr.size(), s));
+  HIPCHK(c, upload(c, c->c_gsrc, gsrc.data(), gsrc.size(), s));
+  HIPCHK(c, upload(c, c->c_gw, gw.data(), gw.size(), s));
+  HIPCHK(c, upload(c, c->c_gfl, gfl.data(), gfl.size(), s));
+  HIPCHK(c, upload(c, c->c_brow, brow.data(), brow.size(), s));
+  HIPCHK(c, upload(c, c->c_rptr, rptr.data(), rptr.size(), s));
+  HIPCHK(c, upload(c, c->c_rsrc, rsrc.data(), rsrc.size(), s));
+  HIPCHK(c, upload(c, c->c_rw, rw.data(), rw.size(), s));
+  HIPCHK(c, upload(c, c->c_rfl, rfl.data(), rfl.size(), s));
   c->n_hang = (int)hnode.size();
-  HIPCHK(c, upload(c->c_hnode, hnode.data(), hnode.size(), s));
-  HIPCHK(c, upload(c->c_hptr, hptr.data(), hptr.size(), s));
-  HIPCHK(c, upload(c->c_hm, hm.data(), hm.size(), s));
-  HIPCHK(c, upload(c->c_hw, hw.data(), hw.size(), s));
+  HIPCHK(c, upload(c, c->c_hnode, hnode.data(), hnode.size(), s));
+  HIPCHK(c, upload(c, c->c_hptr, hptr.data(), hptr.size(), s));
+  HIPCHK(c, upload(c, c->c_hm, hm.data(), hm.size(), s));
+  HIPCHK(c, upload(c, c->c_hw, hw.data(), hw.size(), s));
   std::vector<int> hidx(nn, -1);
   for (size_t j = 0; j < hnode.size(); ++j) hidx[hnode[j]] = (int)j;
-  HIPCHK(c, upload(c->c_hidx, hidx.data(), hidx.size(), s));
-  HIPCHK(c, c->hdiag.alloc((size_t)nn * NC));
-  HIPCHK(c, c->rfull.alloc((size_t)nn * NC));
+  HIPCHK(c, upload(c, c->c_hidx, hidx.data(), hidx.size(), s));
+  HIPCHK(c, take(c, c->hdiag, (size_t)nn * NC));
+  HIPCHK(c, take(c, c->rfull, (size_t)nn * NC));
   // Matrix-free Jacobian: the condensed diagonal block of a master n holds,
   // besides the (n, n) blocks of its cells, w_A(n) w_B(n) J_K(a, b) for every
   // cell K and local pair (a, b) with A = cn[a], B = cn[b] both reaching n
@@ -1819,15 +1857,15 @@ int upload_constraints(glh_ctx *c, const glh::Mesh &m, const std::vector<int> &d
       tfl.push_back(terms[k].fl);
     }
     if (!terms.empty()) tptr.push_back((int)terms.size());
-    HIPCHK(c, upload(c->mfx_ptr, xptr.data(), xptr.size(), s));
-    HIPCHK(c, upload(c->mfx_pair, xpair.data(), xpair.size(), s));
-    HIPCHK(c, upload(c->mft_node, tnode.data(), tnode.size(), s));
-    HIPCHK(c, upload(c->mft_ptr, tptr.data(), tptr.size(), s));
-    HIPCHK(c, upload(c->mft_slot, tslot.data(), tslot.size(), s));
-    HIPCHK(c, upload(c->mft_A, tA.data(), tA.size(), s));
-    HIPCHK(c, upload(c->mft_B, tB.data(), tB.size(), s));
-    HIPCHK(c, upload(c->mft_w, tw.data(), tw.size(), s));
-    HIPCHK(c, upload(c->mft_fl, tfl.data(), tfl.size(), s));
+    HIPCHK(c, upload(c, c->mfx_ptr, xptr.data(), xptr.size(), s));
+    HIPCHK(c, upload(c, c->mfx_pair, xpair.data(), xpair.size(), s));
+    HIPCHK(c, upload(c, c->mft_node, tnode.data(), tnode.size(), s));
+    HIPCHK(c, upload(c, c->mft_ptr, tptr.data(), tptr.size(), s));
+    HIPCHK(c, upload(c, c->mft_slot, tslot.data(), tslot.size(), s));
+    HIPCHK(c, upload(c, c->mft_A, tA.data(), tA.size(), s));
+    HIPCHK(c, upload(c, c->mft_B, tB.data(), tB.size(), s));
+    HIPCHK(c, upload(c, c->mft_w, tw.data(), tw.size(), s));
+    HIPCHK(c, upload(c, c->mft_fl, tfl.data(), tfl.size(), s));
     c->mfx_slots = xpair.size();
     c->mfc = glh::MfCondDev{c->mfx_ptr.p, c->mfx_pair.p, nullptr, (int)tnode.size(), c->mft_node.p, c->mft_ptr.p,
                             c->mft_slot.p, c->mft_A.p, c->mft_B.p, c->mft_w.p, c->mft_fl.p};
@@ -1880,7 +1918,7 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   std::vector<int> did(m.n_nodes);
   for (int i = 0, j = 0; i < m.n_nodes; ++i)
     did[i] = (c->constrained && m.hang_ptr[i + 1] > m.hang_ptr[i]) ? m.n_nodes + j++ : i;
-  HIPCHK(c, upload(c->diag_id, did.data(), did.size(), s));
+  HIPCHK(c, upload(c, c->diag_id, did.data(), did.size(), s));
   // cell -> block map (cell-loop pattern) with first-writer marks in colour order
   const int ns = m.ns;
   std::vector<int> cblk((size_t)m.n_cells * ns * ns);
@@ -1920,7 +1958,7 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
   c->chunk_len = (int)clen;
   c->max_seg_chunks = 0;
   for (int sg = 0; sg < c->n_seg; ++sg) c->max_seg_chunks = std::max(c->max_seg_chunks, segch[sg + 1] - segch[sg]);
-  HIPCHK(c, upload(c->cell_nodes, m.cell_nodes.data(), m.cell_nodes.size(), s));
+  HIPCHK(c, upload(c, c->cell_nodes, m.cell_nodes.data(), m.cell_nodes.size(), s));
   // node -> (cell * ns + local node) lists in cell order, for the gather of
   // the matrix-free product, and the nodes' range of every MF_RANGE cells
   c->mf_range.clear();
@@ -1938,14 +1976,14 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
     std::vector<int> fill(n2c_ptr.begin(), n2c_ptr.end() - 1);
     for (size_t k = 0; k < m.cell_nodes.size(); ++k) n2c_idx[fill[m.cell_nodes[k]]++] = (int)k;
   }
-  HIPCHK(c, upload(c->n2c_ptr, n2c_ptr.data(), n2c_ptr.size(), s));
-  HIPCHK(c, upload(c->n2c_idx, n2c_idx.data(), n2c_idx.size(), s));
-  HIPCHK(c, upload(c->cell_h, m.cell_h.data(), m.cell_h.size(), s));
-  HIPCHK(c, upload(c->cell_face, cface.data(), cface.size(), s));
-  HIPCHK(c, upload(c->node_mask, m.node_mask.data(), m.node_mask.size(), s));
-  HIPCHK(c, upload(c->row_ptr, m.row_ptr.data(), m.row_ptr.size(), s));
-  HIPCHK(c, upload(c->col, m.col.data(), m.col.size(), s));
-  HIPCHK(c, upload(c->diag, diag.data(), diag.size(), s));
+  HIPCHK(c, upload(c, c->n2c_ptr, n2c_ptr.data(), n2c_ptr.size(), s));
+  HIPCHK(c, upload(c, c->n2c_idx, n2c_idx.data(), n2c_idx.size(), s));
+  HIPCHK(c, upload(c, c->cell_h, m.cell_h.data(), m.cell_h.size(), s));
+  HIPCHK(c, upload(c, c->cell_face, cface.data(), cface.size(), s));
+  HIPCHK(c, upload(c, c->node_mask, m.node_mask.data(), m.node_mask.size(), s));
+  HIPCHK(c, upload(c, c->row_ptr, m.row_ptr.data(), m.row_ptr.size(), s));
+  HIPCHK(c, upload(c, c->col, m.col.data(), m.col.size(), s));
+  HIPCHK(c, upload(c, c->diag, diag.data(), diag.size(), s));
   c->cons = glh::ConstraintDev{};
   if (c->constrained) {
     glh::ConstraintDev &C = c->cons;
@@ -1958,25 +1996,25 @@ int glh_upload_mesh(glh_ctx *c, const glh_mesh *mm)
     C.hnode = c->c_hnode.p; C.hptr = c->c_hptr.p; C.hm = c->c_hm.p; C.hw = c->c_hw.p;
     C.hidx = c->c_hidx.p;
   }
-  HIPCHK(c, upload(c->cell_blk, cblk.data(), cblk.size(), s));
-  HIPCHK(c, upload(c->color_cells, m.color_cells.data(), m.color_cells.size(), s));
-  HIPCHK(c, upload(c->cell_mat, cmat.data(), cmat.size(), s));
-  HIPCHK(c, upload(c->chunks, ch.data(), ch.size(), s));
-  HIPCHK(c, upload(c->seg_chunk, segch.data(), segch.size(), s));
+  HIPCHK(c, upload(c, c->cell_blk, cblk.data(), cblk.size(), s));
+  HIPCHK(c, upload(c, c->color_cells, m.color_cells.data(), m.color_cells.size(), s));
+  HIPCHK(c, upload(c, c->cell_mat, cmat.data(), cmat.size(), s));
+  HIPCHK(c, upload(c, c->chunks, ch.data(), ch.size(), s));
+  HIPCHK(c, upload(c, c->seg_chunk, segch.data(), segch.size(), s));
   std::vector<int> rseg(m.n_nodes);
   for (int sg = 0; sg < c->n_seg; ++sg)
     for (int r = c->node_off[sg]; r < c->node_off[sg + 1]; ++r) rseg[r] = sg;
-  HIPCHK(c, upload(c->row_seg, rseg.data(), rseg.size(), s));
-  HIPCHK(c, upload(c->d_node_off, c->node_off.data(), c->node_off.size(), s));
+  HIPCHK(c, upload(c, c->row_seg, rseg.data(), rseg.size(), s));
+  HIPCHK(c, upload(c, c->d_node_off, c->node_off.data(), c->node_off.size(), s));
   const size_t n = (size_t)m.n_nodes * NC;
-  HIPCHK(c, c->U.alloc(n));
-  HIPCHK(c, c->dU.alloc(n));
-  HIPCHK(c, c->X.alloc(n));
-  HIPCHK(c, c->rhs.alloc(n));
-  HIPCHK(c, c->res.alloc(n));
-  HIPCHK(c, c->Fcell.alloc(m.n_cells));
+  HIPCHK(c, take(c, c->U, n));
+  HIPCHK(c, take(c, c->dU, n));
+  HIPCHK(c, take(c, c->X, n));
+  HIPCHK(c, take(c, c->rhs, n));
+  HIPCHK(c, take(c, c->res, n));
+  HIPCHK(c, take(c, c->Fcell, m.n_cells));
   // the cell slots of the residual (and of the matrix-free product)
-  HIPCHK(c, c->mf_ycell.alloc((size_t)m.n_cells * c->ns * NC));
+  HIPCHK(c, take(c, c->mf_ycell, (size_t)m.n_cells * c->ns * NC));
   HIPCHK(c, hipMemsetAsync(c->U.p, 0, n * sizeof(double), s));
   HIPCHK(c, hipMemsetAsync(c->dU.p, 0, n * sizeof(double), s));
   HIPCHK(c, hipMemsetAsync(c->rhs.p, 0, n * sizeof(double), s));
@@ -2000,7 +2038,7 @@ int glh_set_solution(glh_ctx *c, const double *Uh)
 int glh_store_initial(glh_ctx *c)
 {
   RCHK(check_ready(c, false));
-  HIPCHK(c, c->U0.alloc(ndofs(c)));
+  HIPCHK(c, take(c, c->U0, ndofs(c)));
   HIPCHK(c, hipMemcpyAsync(c->U0.p, c->U.p, ndofs(c) * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return GLH_OK;
@@ -2025,12 +2063,12 @@ int glh_apply_jacobian(glh_ctx *c, const double *x, double *y)
   if (!x || !y) return fail(c, GLH_ERR_ARG, "null vector");
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   const size_t n = ndofs(c);
-  HIPCHK(c, c->gW64.alloc(n));
-  HIPCHK(c, c->gZ64.alloc(n));
+  HIPCHK(c, take(c, c->gW64, n));
+  HIPCHK(c, take(c, c->gZ64, n));
   HIPCHK(c, hipMemcpyAsync(c->gZ64.p, x, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   if (c->j_fp32) {
-    HIPCHK(c, c->gW32.alloc(n));
-    HIPCHK(c, c->gZ32.alloc(n));
+    HIPCHK(c, take(c, c->gW32, n));
+    HIPCHK(c, take(c, c->gZ32, n));
     HIPCHK(c, (glh::launch_convert<double, float>(n, c->gZ64.p, c->gZ32.p, c->stream)));
     RCHK((apply_j<float, float>(c, c->J32.p, c->gZ32.p, c->gW32.p, nullptr, glh::ActiveSet{})));
     HIPCHK(c, (glh::launch_convert<float, double>(n, c->gW32.p, c->gW64.p, c->stream)));
@@ -2049,7 +2087,7 @@ int glh_diagonal_blocks(glh_ctx *c, double *out)
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   const size_t nv = (size_t)c->n_nodes * 324;
   DBuf<double> tmp;
-  HIPCHK(c, tmp.alloc(nv));
+  HIPCHK(c, take(c, tmp, nv));
   if (c->j_mf) HIPCHK(c, glh::launch_gather_blocks<double>(c->n_nodes, c->diag_id.p, c->Jd64.p, tmp.p, c->stream));
   else if (c->j_fp32) HIPCHK(c, glh::launch_gather_blocks<float>(c->n_nodes, c->diag.p, c->J32.p, tmp.p, c->stream));
   else HIPCHK(c, glh::launch_gather_blocks<double>(c->n_nodes, c->diag.p, c->J64.p, tmp.p, c->stream));
@@ -2065,12 +2103,12 @@ int glh_apply_block_jacobi(glh_ctx *c, const double *x, double *y)
   if (!c->j_valid) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   RCHK(ensure_precond(c));
   const size_t n = ndofs(c);
-  HIPCHK(c, c->gW64.alloc(n));
-  HIPCHK(c, c->gZ64.alloc(n));
+  HIPCHK(c, take(c, c->gW64, n));
+  HIPCHK(c, take(c, c->gZ64, n));
   HIPCHK(c, hipMemcpyAsync(c->gZ64.p, x, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   if (c->j_fp32) {  // the FP32 inverses the FP32 inner solve applies, on FP32 vectors
-    HIPCHK(c, c->gW32.alloc(n));
-    HIPCHK(c, c->gZ32.alloc(n));
+    HIPCHK(c, take(c, c->gW32, n));
+    HIPCHK(c, take(c, c->gZ32, n));
     HIPCHK(c, (glh::launch_convert<double, float>(n, c->gZ64.p, c->gZ32.p, c->stream)));
     HIPCHK(c, (glh::launch_bj_apply<float, float>(c->n_nodes, c->D32.p, c->gZ32.p, c->gW32.p, c->stream, nullptr,
                                                   nullptr, glh::ActiveSet{})));
@@ -2231,7 +2269,7 @@ int glh_newton_solve(glh_ctx *c, double rtol, int max_newton, double lin_tol, in
   st.assign((size_t)S * 8, 0.0);
   for (int i = 0; i < S; ++i) { st[8 * i + 2] = r0[i]; st[8 * i + 4] = -1.0; }
   std::vector<char> active(S), stalled(S, 0);
-  HIPCHK(c, c->s_flag.alloc(S));
+  HIPCHK(c, take(c, c->s_flag, S));
   const bool f32 = fp32 != 0;
   // the matrix-free operator when switched on (FP64 or FP32, with or without
   // the continuation shift; a batch, or one instance on a constrained mesh);
@@ -2265,7 +2303,7 @@ int glh_newton_solve(glh_ctx *c, double rtol, int max_newton, double lin_tol, in
     // their rows keep the last Jacobian and get a zero right-hand side
     // (a buffer of its own: solve_impl reuses s_flag for its refinement sweeps)
     for (int i = 0; i < S; ++i) flag[i] = active[i];
-    HIPCHK(c, c->asm_flag.alloc(S));
+    HIPCHK(c, take(c, c->asm_flag, S));
     HIPCHK(c, c->pin_fl.alloc(S));
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the pinned flags of the last step are no longer read
     std::copy(flag.begin(), flag.end(), c->pin_fl.p);
@@ -2280,10 +2318,10 @@ int glh_newton_solve(glh_ctx *c, double rtol, int max_newton, double lin_tol, in
       HIPCHK(c, hipStreamSynchronize(c->stream));
       double *sg = c->pin64.p;  // pinned: the copy below is asynchronous
       for (int i = 0; i < S; ++i) sg[i] = active[i] ? c->ptc_sigma0 * rcur[i] / std::max(r0[i], 1e-300) : 0.0;
-      HIPCHK(c, c->s_norm.alloc(S));
+      HIPCHK(c, take(c, c->s_norm, S));
       HIPCHK(c, hipMemcpyAsync(c->s_norm.p, sg, S * sizeof(double), hipMemcpyHostToDevice, c->stream));
       if (mf) {  // on the diagonal blocks, and as a diagonal term of the product
-        HIPCHK(c, c->mf_sh.alloc(ndofs(c)));
+        HIPCHK(c, take(c, c->mf_sh, ndofs(c)));
         HIPCHK(c, glh::launch_mf_shift(c->n_nodes, c->node_mask.p, c->row_seg.p, c->s_norm.p, c->Jd64.p, c->mf_sh.p,
                                        c->stream));
         c->mf_sh_on = true;
@@ -2565,8 +2603,8 @@ int glh_bench_spmv(glh_ctx *c, int k, double *ms_avg)
   RCHK(check_ready(c));
   if (!c->j_valid || k < 1 || !ms_avg) return fail(c, GLH_ERR_STATE, "no Jacobian assembled");
   if (c->j_fp32) {
-    HIPCHK(c, c->gW32.alloc(ndofs(c)));
-    HIPCHK(c, c->gZ32.alloc(ndofs(c)));
+    HIPCHK(c, take(c, c->gW32, ndofs(c)));
+    HIPCHK(c, take(c, c->gZ32, ndofs(c)));
     HIPCHK(c, (glh::launch_convert<double, float>(ndofs(c), c->U.p, c->gZ32.p, c->stream)));
   }
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -2591,8 +2629,8 @@ int glh_bench_read(glh_ctx *c, size_t nbytes, int k, double *ms_avg)
   constexpr int grid = 1024;
   DBuf<unsigned char> a;
   DBuf<float> out;
-  hipError_t e = a.alloc(nbytes);
-  if (e == hipSuccess) e = out.alloc((size_t)grid * 256);
+  hipError_t e = take(c, a, nbytes);
+  if (e == hipSuccess) e = take(c, out, (size_t)grid * 256);
   if (e == hipSuccess) e = hipMemsetAsync(a.p, 0, nbytes, c->stream);
   if (e == hipSuccess) e = hipEventRecord(c->ev0, c->stream);
   for (int i = 0; i < k && e == hipSuccess; ++i) e = glh::launch_read(nbytes, a.p, out.p, grid, c->stream);
@@ -2612,8 +2650,8 @@ int glh_bench_copy(glh_ctx *c, size_t nbytes, int k, double *ms_avg)
   if (!c || !ms_avg || k < 1 || nbytes % 16 || nbytes == 0) return GLH_ERR_ARG;
   HIPCHK(c, hipSetDevice(c->device));
   DBuf<unsigned char> a, b;
-  hipError_t e = a.alloc(nbytes);
-  if (e == hipSuccess) e = b.alloc(nbytes);
+  hipError_t e = take(c, a, nbytes);
+  if (e == hipSuccess) e = take(c, b, nbytes);
   if (e == hipSuccess) e = hipMemsetAsync(a.p, 0, nbytes, c->stream);
   if (e == hipSuccess) e = hipEventRecord(c->ev0, c->stream);
   for (int i = 0; i < k && e == hipSuccess; ++i) e = glh::launch_copy(nbytes, a.p, b.p, c->stream);
