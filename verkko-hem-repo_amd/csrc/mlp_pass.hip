@@ -122,16 +122,18 @@ struct Weights {
 };
 
 // SiLU(z) = z / (1 + exp(-z)) and sigma(z) = 1 / (1 + exp(-z)): the quotient
-// as a product with the hardware reciprocal and one residual correction, 7
+// as a product with the hardware reciprocal and one residual correction, 8
 // instructions with the sum (sigma 6) where the general division takes 11.
-// The divisor is carried at a quarter, so that its reciprocal is never
-// denormal.  Over all 2^32 values of z SiLU has the division's bits except
-// where 4 z overflows, sigma except where it is denormal (then one unit off
-// in 34043 cases).
+// The reciprocal is that of a quarter of the divisor, so that it is never
+// denormal.  SiLU takes the quarter back from the reciprocal, not from the
+// quotient: the quotient of a quarter overflows from z = FLT_MAX / 4 on, and
+// its residual makes that a NaN.  Over all 2^32 values of z SiLU has the
+// division's bits, sigma except where it is denormal (then one unit off in
+// 34043 cases).
 __device__ inline float silu(float z)
 {
-  const float d = fmaf(expf(-z), 0.25f, 0.25f), y = __builtin_amdgcn_rcpf(d), x = z * y;
-  return 0.25f * __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, x, z), y, x), d, z);
+  const float e = expf(-z), d = 1.f + e, y = 0.25f * __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f)), x = z * y;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, x, z), y, x), d, z);
 }
 __device__ inline float sigma(float z)
 {
@@ -160,7 +162,7 @@ __device__ inline void store_tile(const uint16_t *tile, int nfb, int row0, uint1
 // (131 KB at width 256, from L2) and writes only what the gradient needs; a
 // wavefront holds 64 NB / 4 columns of all 16 MB rows, so the weights go
 // straight to its registers and LDS carries the activations only.  Inference
-// is bound by the SiLU's instructions (24 per value, of which exp 13: 63 of
+// is bound by the SiLU's instructions (25 per value, of which exp 13: 63 of
 // 106 us at 65536 rows, matrix cores 16 us; 237 us as one product a layer);
 // the gradient by those and the 1 GB of Z, H and dZ (267 us against 445 for
 // the same sweeps as products).
