@@ -591,7 +591,8 @@ __device__ inline void square_lines(double *h)
 // ([cell][node][171], raw: no Dirichlet rule).  A thread holds one entry's
 // Hessian at the points and contracts it with w N_a^2, a tensor product, by
 // 1D lines (162 operations instead of 729 multiply-adds in Q2).  Bound by the
-// Hessian entries' instructions and LDS reads.  Per Newton step, setup and
+// Hessian entries' instructions and LDS reads (the vector unit busy 45% of the
+// time, LDS about as much).  Per Newton step, setup and
 // gather: 32^3 Q2 cells 10 x (114 + 39) us, against 8 colours of 280 us that
 // read and rewrote the nodes' blocks; 5586 Q2 cells FP32 2 x (95 + 30) against
 // 8 x 60; 22528 Q1 cells with hanging nodes 2 x (128 + 32) against 11 x 55.
@@ -1076,7 +1077,11 @@ constexpr int mf_waves() { return NCELL == 1 ? 1 : std::is_same<TA, float>::valu
 // and the columns then test it and write their NS values.  Before, a thread
 // per pencil passed every 1D pass through LDS, with nine barriers per cell.
 // XCD x works through the cells [x n8, (x+1) n8) in order, so neighbours
-// share their nodes' x in that XCD's L2.
+// share their nodes' x in that XCD's L2.  Bound by FP64 instructions and load
+// latency at 1.75 waves per SIMD: a Q2 cell takes 40.8 k FP64 instructions by
+// the algorithm and 42.3 k as counted (residual 33.1 k, 34.5 k), which keep
+// the vector unit busy half of the 88 us of 32768 cells; FP32, at 2.5 waves,
+// 88% of 52 us.
 template <int DEG, typename TH, typename TX, bool RES, int NCELL>
 __global__ __launch_bounds__(mf_threads<NCELL>(), (mf_waves<DEG, mf_arith<TH, TX>, NCELL>())) void k_mf_apply(
     MeshDev Mh, Material M0, const TH *__restrict__ Uq, const TX *__restrict__ x, int n_cells, int n8,
@@ -1702,9 +1707,11 @@ inline int mf_grid(int n_cells, int nc) { return 8 * ((mf_range(n_cells) + nc - 
 // Up to this many cells a thread takes one plane of one column (NCELL = 1):
 // its work is a third as long, but it reads and transforms the column once
 // per plane.  Measured, us per launch, NCELL 1 against 7: Q2 FP64 product
-// 7.5 / 12.1 at 8^3 cells, 9.8 / 13.4 at 10^3, 16.2 / 14.8 at 12^3; Q2 FP32
-// 9.6 / 12.0 at 12^3, 12.6 / 14.3 at 14^3; Q1 FP64 6.1 / 6.0 at 8^3 (residual
-// 5.1 / 5.7), 8.4 / 6.4 at 12^3.
+// 7.6 / 12.4 at 8^3 cells, 10.1 / 13.4 at 10^3, 15.2 / 14.5 at 11^3 (residual
+// 11.4 / 12.0), 16.3 / 15.1 at 12^3 (12.8 / 13.6): the line between the last
+// two; Q2 FP32 9.4 / 12.8 at 12^3, 12.8 / 14.4 at 14^3, 15.4 / 15.8 at 15^3;
+// Q1 FP64 5.3 / 6.1 at 5^3 (residual 4.5 / 5.4), 5.9 / 6.1 at 8^3 (5.0 / 5.2),
+// 6.4 / 6.3 at 10^3 (5.6 / 5.6), 8.2 / 6.6 at 12^3 (6.9 / 5.9).
 template <int DEG, typename TA>
 constexpr int mf_small_mesh() { return DEG == 1 ? 512 : std::is_same<TA, float>::value ? 3072 : 1536; }
 

@@ -184,9 +184,10 @@ struct glh_ctx {
   // active set of a batched GMRES cycle (instances still iterating)
   DBuf<int> d_node_off, act_counts, act_seg, act_rpref, act_chunk;
   // one restart cycle as graphs: head (true residual, start of cycle), body
-  // blocks of Arnoldi steps, tail (update of x)
+  // blocks of Arnoldi steps, tail (update of x), a single instance's second
+  // Gram-Schmidt passes
   struct Graph {
-    std::vector<hipGraphExec_t> exec;  // head, tail, blocks...
+    std::vector<hipGraphExec_t> exec;  // head; tail and blocks of each grid size; second passes
     std::vector<const void *> key;
     int q = 1;
   } graph64, graph32;
@@ -805,10 +806,12 @@ constexpr int FOLD_MAX_CHUNKS = 64;
 // coefficients, Givens rotations and stopping test
 // ||b_s - J x_s|| <= rtol[s] ||b_s||.  The Hessenberg updates, rotations and
 // tests run on the device (k_gmres_ctl), and every kernel skips the instances
-// that have stopped, so a restart cycle needs no host round trip: it is
-// enqueued once, captured in a HIP graph and replayed (or launched directly
-// when kernel timing is on).  its_out: lockstep iterations; its_seg:
-// iterations each instance used.
+// that have stopped, so the host needs no values of a step: a batch's cycle is
+// enqueued in blocks of steps, between which the host only asks whether any
+// instance still iterates; a single instance goes step by step, its status
+// read after each and the next one already enqueued.  The pieces are captured
+// in HIP graphs and replayed (or launched directly when kernel timing is on).
+// its_out: lockstep iterations; its_seg: iterations each instance used.
 template <typename TJ, typename TV>
 int enqueue_cycle(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, int m, const glh::GmresCtl<TV> &C,
                   bool timed, int part, int j0 = 0, int j1 = 0, int shift = 0)
@@ -998,7 +1001,9 @@ int gmres(glh_ctx *c, const TJ *J, const TJ *Dinv, const TV *b, TV *x, const std
   // Graphs of one restart cycle, rebuilt whenever their buffers change.  The
   // Arnoldi steps go in blocks of q; the host checks between blocks whether
   // any instance still iterates, so at most q - 1 steps of a cycle run as
-  // skipped launches (none for a single instance, q = 1).  Batches record
+  // skipped launches.  A single instance (q = 1) runs one skipped step where
+  // a cycle stops before its last column, and one at each second pass: the
+  // step enqueued ahead.  Batches record
   // the body and tail at three grid sizes (shift 0, 3, 6) and replay the
   // one that fits the number of rows still iterating, so that a few
   // straggling instances do not pay for the workgroups of the full batch.

@@ -327,8 +327,8 @@ hipError_t launch_build_active(const SegInfo &S, const int *flag, const int *nod
                                int *rpref, int *chunk, hipStream_t s);
 
 // Device state of the batched GMRES: Hessenberg columns, Givens rotations
-// and stopping tests live on the device so a restart cycle needs no host
-// round trip (and can be captured in a HIP graph).
+// and stopping tests live on the device, so that no value of a step goes
+// through the host (and a cycle's pieces can be captured in HIP graphs).
 template <typename T>
 struct GmresCtl {
   int S, m, ldh;

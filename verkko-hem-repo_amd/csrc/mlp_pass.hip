@@ -163,9 +163,10 @@ __device__ inline void store_tile(const uint16_t *tile, int nfb, int row0, uint1
 // wavefront holds 64 NB / 4 columns of all 16 MB rows, so the weights go
 // straight to its registers and LDS carries the activations only.  Inference
 // is bound by the SiLU's instructions (25 per value, of which exp 13: 63 of
-// 106 us at 65536 rows, matrix cores 16 us; 237 us as one product a layer);
-// the gradient by those and the 1 GB of Z, H and dZ (267 us against 445 for
-// the same sweeps as products).
+// 109 us at 65536 rows, the vector unit busy 68% of the time and longer by
+// its exp and reciprocal, matrix cores 17%; 237 us as one product a layer);
+// the gradient by those (vector unit 52%) and the 1.08 GB of Z, H and dZ
+// (264 us, 4.1 TB/s, against 445 for the same sweeps as products).
 template <int MB, int NB, bool GRAD>
 __global__ __launch_bounds__(256, 2) void k_mlp_pass(PassArgs A)
 {
@@ -635,9 +636,14 @@ void launch_pass(const PassArgs &A, int nb, hipStream_t s)
 
 // Small tiles while they leave more workgroups than CUs (32 rows up to 16384:
 // gradient of 14000 rows 75 us against 94 with 64 rows, of 19000 rows 126
-// against 118), the largest once two workgroups of 128 rows fill every CU
-// (45000 rows 224 us with 64 rows, 261 with 128; 65536 rows 277 against 267,
-// half the reads of the weights).  128 rows only at width 256.
+// against 118).  128 rows, at width 256, where the training batches lie: two
+// workgroups a CU are 65536 rows, and half the reads of the weights shorten
+// the gradient from 7/8 of that on.  us with 64 and with 128 rows: gradient
+// of 45000 rows 230 / 233, 49152 238 / 243, 57344 262 / 252, 65536 281 / 273;
+// past 65536 a second round of 128-row tiles is mostly empty (73728 rows
+// 352 / 387, 98304 402 / 420), and inference, which waits for no Z, is a
+// little faster with 64 rows at every size (57344 rows 98 / 104, 65536
+// 100 / 104).
 int pass_rows(int n, int width) { return n >= 57344 && width == 256 ? 128 : n >= 16384 ? 64 : 32; }
 
 hipError_t pass(const PassArgs &A, bool grad, hipStream_t s)
