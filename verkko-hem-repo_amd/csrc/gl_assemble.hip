@@ -1507,6 +1507,7 @@ __global__ void k_mf_gather(int n_nodes, const int *__restrict__ ptr, const int 
 // slabs).  8 waves per workgroup: a chunk of 4096 takes 4 rounds of pairs,
 // one of 1024 one.
 constexpr int GT = 512;
+typedef double pair8 __attribute__((ext_vector_type(2), aligned(8)));  // rhs may be the caller's: aligned to a double
 __global__ __launch_bounds__(GT) void k_res_gather(const long long *__restrict__ ch, const int *__restrict__ ptr,
                                                    const int *__restrict__ idx, const double *__restrict__ ycell,
                                                    const uint32_t *__restrict__ mask,
@@ -1519,7 +1520,7 @@ __global__ __launch_bounds__(GT) void k_res_gather(const long long *__restrict__
   double acc = 0.0;
   for (long long o = beg + 2 * threadIdx.x; o < end; o += 2 * GT) {
     const int node = (int)(o / 18), c = (int)(o - 18LL * node);
-    double2 r = {0.0, 0.0};
+    pair8 r = {0.0, 0.0};
     if (on) {
       double s0 = 0.0, s1 = 0.0;
       slot_pair_sum(ptr, idx, ycell, node, c, s0, s1);
@@ -1527,7 +1528,7 @@ __global__ __launch_bounds__(GT) void k_res_gather(const long long *__restrict__
       r.x = ((mk >> c) & 1u) ? 0.0 : -s0;
       r.y = ((mk >> (c + 1)) & 1u) ? 0.0 : -s1;
     }
-    *reinterpret_cast<double2 *>(rhs + o) = r;
+    *reinterpret_cast<pair8 *>(rhs + o) = r;
     acc += r.x * r.x;
     acc += r.y * r.y;
   }

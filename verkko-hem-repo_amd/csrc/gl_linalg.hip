@@ -822,7 +822,7 @@ __global__ void k_set_scalar(T *p, T v)
 // at least, and an FP32 chunk may end with a pair.
 template <typename T> struct Quad;
 template <> struct Quad<double> {
-  typedef double type __attribute__((ext_vector_type(2)));
+  typedef double type __attribute__((ext_vector_type(2), aligned(8)));  // (glh_residual_into's R may be no better aligned)
   static constexpr int N = 2;
 };
 template <> struct Quad<float> {
