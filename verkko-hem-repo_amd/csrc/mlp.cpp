@@ -88,7 +88,7 @@ struct glh_mlp {
   std::vector<Buf<bf16>> H;
   std::vector<Buf<float>> Z;
   Buf<bf16> dY, dZa, dZb;
-  std::vector<Buf<bf16>> dZ;  // tiled: every layer's, kept for the weight gradients
+  Buf<bf16> dZo;              // tiled: the output layer's dZ (a hidden layer's lies in its Z)
   Buf<float> Xp, Yp;          // inference: points of a pass, outputs
   Buf<int> step;
   hipGraphExec_t graph = nullptr;
@@ -149,17 +149,16 @@ int ensure_tiled(glh_mlp *m, int nb)
   const size_t rows = ((size_t)nb + 127) / 128 * 128;
   m->H.resize(m->depth + 1);
   m->Z.resize(m->depth);
-  m->dZ.resize(m->depth + 1);
   MCHK(m, m->Xb.alloc((size_t)nb * 6));
   MCHK(m, m->Yb.alloc((size_t)nb * m->n_out));
   size_t ptot = 0, ctot = 0;
   for (int l = 0; l <= m->depth; ++l) {
     MCHK(m, m->H[l].alloc(rows * m->K[l]));
-    MCHK(m, m->dZ[l].alloc(rows * m->Np[l]));
     if (l < m->depth) MCHK(m, m->Z[l].alloc(rows * m->width));
     ptot += (size_t)m->K[l] * m->Np[l];
     ctot += (size_t)m->Np[l];
   }
+  MCHK(m, m->dZo.alloc(rows * m->Np[m->depth]));
   MCHK(m, m->part.alloc(ptot * DW_SPLITS));
   MCHK(m, m->cpart.alloc(ctot * DW_SPLITS));
   MCHK(m, m->lpart.alloc(rows / 32));
@@ -338,10 +337,10 @@ int tiled_step(glh_mlp *m, int n_real, const float *X, const float *T, bool adam
   int unit = 0;
   for (int l = 0; l <= D; ++l) {
     A.H[l] = m->H[l].p;
-    A.dZ[l] = m->dZ[l].p;
+    A.dZ[l] = l < D ? reinterpret_cast<bf16 *>(m->Z[l].p) : m->dZo.p;
     if (l < D) A.Z[l] = m->Z[l].p;
     Wg.H[l] = m->H[l].p;
-    Wg.dZ[l] = m->dZ[l].p;
+    Wg.dZ[l] = A.dZ[l];
     const int nA = m->K[l] / 16, nB = l < D ? m->width / 16 : (m->n_out + 31) / 32 * 2;
     Wg.nA[l] = U.nA[l] = nA;
     Wg.nB[l] = U.nB[l] = nB;
@@ -486,7 +485,7 @@ int glh_mlp_destroy(glh_mlp *m)
   for (auto &b : m->WbT) b.release();
   for (auto &b : m->H) b.release();
   for (auto &b : m->Z) b.release();
-  for (auto &b : m->dZ) b.release();
+  m->dZo.release();
   m->dY.release();
   m->dZa.release();
   m->dZb.release();

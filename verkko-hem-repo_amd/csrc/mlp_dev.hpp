@@ -84,7 +84,7 @@ struct PassArgs {
   const bf16 *WT[MLP_MAX_LAYERS], *Wb[MLP_MAX_LAYERS];
   float *Y = nullptr;  // inference: n_real x n_out
   // gradient: what the weight gradients and the backward sweep read, in rows
-  // padded to pass_rows
+  // padded to pass_rows; a hidden layer's dZ lies in its Z
   bf16 *H[MLP_MAX_LAYERS], *dZ[MLP_MAX_LAYERS];
   float *Z[MLP_MAX_LAYERS];
   float *lpart = nullptr;  // sums of squares, one per pass_rows

@@ -12,7 +12,8 @@
 //   Wb[l]: fragments [k block][n step] of W's transpose (input gradients);
 //   H[l], dZ[l]: fragments [32 samples][feature block], k the samples (the
 //     operands of the weight gradients);
-//   Z[l]: the FP32 accumulator blocks [16 samples][16 features], 64 lanes x 4.
+//   Z[l]: the FP32 accumulator blocks [16 samples][16 features], 64 lanes x 4;
+//     a hidden layer's dZ takes its place (dz_block).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -141,8 +142,15 @@ __device__ inline float sigma(float z)
   return 0.25f * __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, y, 1.f), y, y), d, 1.f);
 }
 
-// the tile's nfb feature blocks to memory as fragments of 32 samples
-template <int MB>
+// Fragment blocks before the 32 samples sb of a hidden layer's dZ, nfb blocks
+// each.  They lie in the layer's Z, twice as large, of which a tile has read
+// its rows when it writes them: in the first half of its 32 samples' part for
+// even sb, the second for odd, so that they meet every memory channel.
+__device__ inline size_t dz_block(int sb, int nfb) { return (size_t)(2 * sb + (sb & 1)) * nfb; }
+
+// the tile's nfb feature blocks to memory as fragments of 32 samples (INZ: a
+// hidden layer's dZ, at dz_block)
+template <int MB, bool INZ = false>
 __device__ inline void store_tile(const uint16_t *tile, int nfb, int row0, uint16_t *__restrict__ dst, int w, int lane)
 {
   const int g = lane >> 4;
@@ -150,9 +158,10 @@ __device__ inline void store_tile(const uint16_t *tile, int nfb, int row0, uint1
     const int sb = q / nfb, fb = q - sb * nfb;
     const uint4 v =
         *reinterpret_cast<const uint4 *>(tile + tile_at<MB>(fb * 16 + (lane & 15), 2 * sb + (g >> 1)) + 8 * (g & 1));
+    const size_t block = INZ ? dz_block(row0 / 32 + sb, nfb) : (size_t)(row0 / 32 + sb) * nfb;
     // past the caches, which keep Z for the backward sweep
     __builtin_nontemporal_store(__builtin_bit_cast(f32x4, v),
-                                reinterpret_cast<f32x4 *>(dst + ((size_t)(row0 / 32 + sb) * nfb + fb) * 512 + lane * 8));
+                                reinterpret_cast<f32x4 *>(dst + (block + fb) * 512 + lane * 8));
   }
 }
 
@@ -370,7 +379,7 @@ __global__ __launch_bounds__(256, 2) void k_mlp_pass(PassArgs A)
       }
     }
     put();
-    store_tile<MB>(tile, W / 16, row0, reinterpret_cast<uint16_t *>(A.dZ[l - 1]), w, lane);
+    store_tile<MB, true>(tile, W / 16, row0, reinterpret_cast<uint16_t *>(A.dZ[l - 1]), w, lane);
   }
 }
 
@@ -409,12 +418,13 @@ __global__ __launch_bounds__(256, TB == 4 ? 2 : 4) void k_mlp_wgrad(WgradArgs A)
   // the wavefront's TB fragments of a step: A's blocks (w = 0, 1) or B's
   const bool isB = w >= 2;
   const int f0 = (isB ? b0 : a0) + (w & 1) * TB, nf = isB ? nB : nA;
+  const bool inz = isB && l + 1 < A.n_layers;
   const uint16_t *src = (isB ? dZ : H) + (size_t)f0 * 512 + lane * 8;
   uint4 x[R][TB];
   const auto load = [&](int u, int k) {
 #pragma unroll
     for (int i = 0; i < TB; ++i)
-      if (f0 + i < nf && k < k1) x[u][i] = *reinterpret_cast<const uint4 *>(src + ((size_t)k * nf + i) * 512);
+      if (f0 + i < nf && k < k1) x[u][i] = *reinterpret_cast<const uint4 *>(src + ((inz ? dz_block(k, nf) : (size_t)k * nf) + i) * 512);
   };
   const auto stage = [&](int u, int b) {
 #pragma unroll
