@@ -55,24 +55,25 @@ def spmv_bytes(n_nodes, nnzb, val_bytes, vec_bytes):
     return upper * (324 * val_bytes + 4) + (n_nodes + 1) * 4 + 2 * n_nodes * 18 * vec_bytes
 
 
-# flops per quadrature point of H(q) X(q) formed as the derivative of the
-# residual density at the stored iterate: 6 dot products of 9 values (108),
-# the spin-space products u u^T, v v^T, u v^T and their derivatives along X
-# (378), their sums and differences (72), their products with the iterate and
-# X for the 18 components (864), the final combination (216); and the
-# gradient terms gamma with the quadrature weight (234)
-MF_POINT_FLOPS = 108 + 378 + 72 + 864 + 216 + 234
+# flops (a fused multiply-add counts two) of k_mf_apply's arithmetic, term by
+# term.  Per quadrature point, H(q) X(q) as the derivative of N(A) (u; v): the
+# Gram matrices u u^T, v v^T, u v^T of the iterate (105) and their derivatives
+# along X (201), N and dN from them (88 each), N (a; b) + dN (u; v) (432).
+MF_POINT_FLOPS = 105 + 201 + 2 * 88 + 432
+# Per cell and component, by degree: to the z lines' coefficients and back
+# (Q2: 36 each), per plane of points the z and y lines of values and gradients,
+# the x lines, divergence and fluxes, and their tests (Q1 226, Q2 627), then
+# the tests of H(q) X(q) (Q1 40, Q2 114).
+MF_COLUMN_FLOPS = {1: 2 * (226 + 40), 2: 36 + 3 * (627 + 114) + 36}
+# the same in FP64 instructions (an add, a product or a fused multiply-add),
+# per cell: the counters read 42.3 k for Q2, idle lanes included
+MF_CELL_INSTS = {1: 18 * 356 + 8 * 521, 2: 18 * 1485 + 27 * 521}
 
 
 def mf_flops(deg, n_cells):
-    """Algorithmic FP64 flops of one sum-factorised matrix-free product J x
-    (k_mf_apply): per cell and component the three 1D passes for x and its
-    gradients at the quadrature points (2 + 3 + 4 outputs per point, N1
-    multiply-adds each) and the three 1D test passes (4 + 3 + 2 outputs per
-    point), and per point MF_POINT_FLOPS; Robin faces left out."""
-    n1 = deg + 1
-    ns = n1 ** 3
-    return n_cells * (2 * 18 * 18 * n1 * ns + ns * MF_POINT_FLOPS)
+    """FP64 flops of one matrix-free product J x (k_mf_apply) over the cells:
+    18 columns and the quadrature points of each; Robin faces left out."""
+    return n_cells * (18 * MF_COLUMN_FLOPS[deg] + (deg + 1) ** 3 * MF_POINT_FLOPS)
 
 
 def mf_bytes(deg, n_cells, n_dofs):
@@ -647,7 +648,8 @@ def main():
     if mf:
         # algorithmically bound by the FP64 arithmetic: with H(q) X(q) formed
         # from the stored iterate (0.13 GB at the 32^3 Q2 cube) the flops at
-        # the FP64 peak take longer than the bytes at the HBM peak.  MI355X runs
+        # the FP64 peak (28 us there) take longer than the bytes at the HBM
+        # peak (26 us), and their instructions longer (34 us).  MI355X runs
         # FP64 at 78.6 TFLOP/s on the vector and the matrix units alike.
         flops, nbytes = mf_flops(deg, mesh.n_cells), mf_bytes(deg, mesh.n_cells, n_dofs)
         tfs = flops / (apply_avg_ms * 1e-3) / 1e12
@@ -658,10 +660,12 @@ def main():
                 "frac": tfs / FP64_PEAK_TFS,
                 "traffic": tjson.get("k_mf_apply", {}).get("bytes_per_product"), "algorithmic_bytes": nbytes,
                 "algorithmic_flops": flops, "hbm_gb_s": gbs, "frac_hbm_peak": gbs / HBM_PEAK_GBS,
+                "fp64_insts": mesh.n_cells * MF_CELL_INSTS[deg],
+                "frac_issue": mesh.n_cells * MF_CELL_INSTS[deg] * 2 / (apply_avg_ms * 1e-3) / 1e12 / FP64_PEAK_TFS,
                 "stream_read_gb_s": stream_gbs,
                 # FP64 on the vector unit (the same peak as the matrix unit);
-                # the kernel waits on its LDS passes and barriers (SQ counters
-                # in profiles/matfree_cube_q2_ref5.md)
+                # frac_issue: its instructions at the rate of one fused
+                # multiply-add each (counters: profiles/case_kernel_counters.md)
                 "peak_note": "FP64 dense peak, vector and matrix units alike",
                 "limiter": "FP64 instructions and load latency at 2 waves per SIMD"}
     else:
